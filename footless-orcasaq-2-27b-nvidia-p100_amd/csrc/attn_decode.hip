@@ -883,10 +883,11 @@ attn_gate_vec_kernel(f16* __restrict__ z, const f16* __restrict__ g, int n_heads
     const int d = (int)(c - row * per_row) * 8;
     f16x8* zp = (f16x8*)(z + row * z_pitch + d);
     const f16x8 gv = *(const f16x8*)(g + row * g_pitch + g_off + d);
-    f16x8 zv = *zp;
+    const f16x8 zv = *zp;
+    float f[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) zv[e] = f16_sat((float)zv[e] * sigmoid_f((float)gv[e]));
-    *zp = zv;
+    for (int e = 0; e < 8; ++e) f[e] = (float)zv[e] * sigmoid_f((float)gv[e]);
+    *zp = f16_sat8(f);
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }

@@ -162,9 +162,9 @@ __device__ __forceinline__ float cv_get(const typename ConvVec<CPL>::type& v, in
     else return (float)v;
 }
 template <int CPL>
-__device__ __forceinline__ void cv_set(typename ConvVec<CPL>::type& v, int i, f16 h) {
-    if constexpr (CPL == 8) v[i] = h;
-    else v = h;
+__device__ __forceinline__ typename ConvVec<CPL>::type cv_sat(const float (&v)[CPL]) {
+    if constexpr (CPL == 8) return f16_sat8(v);
+    else return f16_sat(v[0]);
 }
 
 // N consecutive fp16 values at p as floats: N / 8 16-byte loads when VEC
@@ -254,8 +254,7 @@ conv_window_kernel(const f16* __restrict__ x, const f16* __restrict__ w, const f
 #pragma unroll
     for (int i = 0; i < NTOK; ++i) {
         if (i >= nt) continue;   // uniform; keeps the trip count constant (full unroll)
-        vec out;
-        float xf[CPL];
+        float xf[CPL], yf[CPL];
 #pragma unroll
         for (int c = 0; c < CPL; ++c) {
             xf[c] = cv_get<CPL>(xr[i], c);
@@ -263,9 +262,9 @@ conv_window_kernel(const f16* __restrict__ x, const f16* __restrict__ w, const f
 #pragma unroll
             for (int j = 0; j < H; ++j) acc = fmaf(taps[c * W + j], win[j][c], acc);
             acc = fmaf(taps[c * W + H], xf[c], acc);
-            cv_set<CPL>(out, c, f16_sat(silu_f(acc)));
+            yf[c] = silu_f(acc);
         }
-        *(vec*)(y + (size_t)(t0 + i) * row_stride + d) = out;
+        *(vec*)(y + (size_t)(t0 + i) * row_stride + d) = cv_sat<CPL>(yf);
         if constexpr (H > 0) {
 #pragma unroll
             for (int c = 0; c < CPL; ++c) {
@@ -986,10 +985,10 @@ rmsnorm_gated_rows_kernel(const f16* __restrict__ o, const f16* __restrict__ z,
         ss += lane_xor(ss, 8);                                         // r0 + r2, r1 + r3
         ss += lane_xor(ss, 4);                                         // (r0 + r2) + (r1 + r3)
         const float inv = 1.f / sqrtf(ss / (float)GR_K + eps);
-        f16x8v out;
+        float yf[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) out[i] = f16_sat(x[i] * inv * wv[i] * silu_f((float)zv[p][i]));
-        if (ok[p]) *(f16x8v*)(y + base[p]) = out;
+        for (int i = 0; i < 8; ++i) yf[i] = x[i] * inv * wv[i] * silu_f((float)zv[p][i]);
+        if (ok[p]) *(f16x8v*)(y + base[p]) = f16_sat8(yf);
     }
 }
 
@@ -1035,10 +1034,10 @@ l2norm_rows_kernel(const f16* __restrict__ x, f16* __restrict__ y, int rows, int
     ss += lane_xor(ss, 8);                                         // r0 + r2, r1 + r3
     ss += lane_xor(ss, 4);                                         // (r0 + r2) + (r1 + r3)
     const float den = sqrtf(ss + eps);
-    f16x8v out;
+    float yf[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) out[i] = f16_sat((xf[i] / den) * scale);
-    if (ok) *(f16x8v*)(y + base) = out;
+    for (int i = 0; i < 8; ++i) yf[i] = (xf[i] / den) * scale;
+    if (ok) *(f16x8v*)(y + base) = f16_sat8(yf);
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
