@@ -86,6 +86,9 @@ SIGNATURES = {
                                     _F, _I, _I, _P, _SZ, _P]),
     "fl_gdn_prefill_chunked_logits": (_I, [_P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I,
                                            _I, _I, _I, _I, _I, _F, _I, _I, _P, _SZ, _P]),
+    "fl_gdn_prefill_layer_work_bytes": (_SZ, [_I, _I, _I, _I, _I]),
+    "fl_gdn_prefill_layer": (_I, [_P, _I, _P, _P, _P, _I, _P, _P, _I, _P, _P, _P, _P, _P, _P, _I,
+                                  _I, _I, _I, _I, _F, _F, _F, _P, _SZ, _P]),
 }
 
 

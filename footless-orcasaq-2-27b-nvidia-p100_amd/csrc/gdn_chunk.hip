@@ -58,6 +58,7 @@
 #include "fl_common.hpp"
 
 #include <mutex>
+#include <type_traits>
 
 #pragma clang fp contract(off)
 
@@ -176,32 +177,39 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// T's block (bi, bj), bi > bj, from the blocks of T already in sA (kept
+// T's block (bi, bj), bi = bj + LV, from the blocks of T already in sA (kept
 // transposed above the diagonal, the diagonal blocks D with their zeros):
 // S = sum_k A_{bi,k} T_{k,bj} (k-step s takes k = 16 k + 4 s + g), then
 // T_{bi,bj} = -D_bi S with S's result slots as the B operand as they stand
 // (k-step s pairs lane group g with S's row 4 g + s, so D is read at column
-// 4 g + s)
-__device__ __forceinline__ void t_block(float (*sA)[CK_C + 4], int bi, int bj, int lane) {
-    const int g = lane >> 4, i = lane & 15;
-    f32x4 sm = (f32x4)(0.f);
-    for (int kb = bj; kb < bi; ++kb) {
+// 4 g + s); returns -T_{bi,bj}'s values of this lane
+// Every operand is read before the first product (in turn with them each pair
+// waited out an LDS round trip).
+template <int LV>
+__device__ __forceinline__ f32x4 t_block(float (*sA)[CK_C + 4], int bj, int lane) {
+    const int g = lane >> 4, i = lane & 15, bi = bj + LV;
+    float a[LV][4], t[LV][4], d[4];
+#pragma unroll
+    for (int m = 0; m < LV; ++m)
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            const int kk = 4 * s + g;
-            const float a = sA[16 * bi + i][16 * kb + kk];
-            // T_{kb,bj}[kk][i]: transposed at sA[16 bj + i][16 kb + kk] (D's
-            // zeros above its diagonal are stored)
-            sm = mfma4(a, sA[16 * bj + i][16 * kb + kk], sm);
+            const int kk = 16 * (bj + m) + 4 * s + g;
+            a[m][s] = sA[16 * bi + i][kk];
+            // T_{kb,bj}[kk][i]: transposed at sA[16 bj + i][kk] (D's zeros above
+            // its diagonal are stored)
+            t[m][s] = sA[16 * bj + i][kk];
         }
-    }
-    f32x4 t = (f32x4)(0.f);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        const int kk = 4 * g + s;
-        t = mfma4(sA[16 * bi + kk][16 * bi + i], sm[s], t);   // D_bi[i][kk], transposed
-    }
-    *(f32x4*)&sA[16 * bj + i][16 * bi + 4 * g] = -t;
+    for (int s = 0; s < 4; ++s) d[s] = sA[16 * bi + 4 * g + s][16 * bi + i];   // D_bi[i][kk], transposed
+    f32x4 sm = (f32x4)(0.f), r = (f32x4)(0.f);
+#pragma unroll
+    for (int m = 0; m < LV; ++m)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) sm = mfma4(a[m][s], t[m][s], sm);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) r = mfma4(d[s], sm[s], r);
+    *(f32x4*)&sA[16 * bj + i][16 * bi + 4 * g] = -r;
+    return r;
 }
 
 
@@ -230,58 +238,46 @@ struct PrepGates {
     int stride;            // n_vheads, or ab_stride
 };
 
-// One workgroup of 4 waves a (chunk, v head), a grid of chunks x v heads: it
-// loads its k head's K and Q rows of the chunk, forms K K^T and Q K^T (wave w
-// the 32 x 32 block (w / 2, w % 2)), then its v head's A, T and M o QK^T from
-// them with that head's gates, into the head's block of the workspace.
-template <bool LOGITS>
-__global__ void __launch_bounds__(256)
-chunk_prep_kernel(const f16* __restrict__ q, const f16* __restrict__ k, const PrepGates gates,
-                  int T, int n_vheads, int qk_stride, int group, char* __restrict__ work) {
-    __shared__ __attribute__((aligned(16))) char smem[2 * CK_C * PK_P * 2];
-    __shared__ float sG[CK_C], sB[CK_C], sRed[8];
-    f16(*sK)[PK_P] = (f16(*)[PK_P])smem;
-    f16(*sQ)[PK_P] = (f16(*)[PK_P])(smem + CK_C * PK_P * 2);
-    float(*sA)[PA_P] = (float(*)[PA_P])smem;                     // after the products
-    float(*sM)[PA_P] = (float(*)[PA_P])(smem + CK_C * PA_P * 4);
+// v of lane I of this lane's row of 16 (DPP row broadcast)
+template <int I>
+__device__ __forceinline__ float row_bcast(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + I, 0xF, 0xF, true));
+}
 
-    const int c = blockIdx.x, hv_blk = blockIdx.y, hk = hv_blk / group;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+// Rows I .. 15 of column j of D = (I + A)^-1 for each 16-lane row's own 16 x 16
+// A: na is row (lane % 16) of -A, x[i] = [i == j] + sum_{m < i} -A[i][m] x[m],
+// even and odd m in two chains.
+template <int I>
+__device__ __forceinline__ void solve_rows(const float (&na)[16], float (&x)[16], int j) {
+    if constexpr (I < 16) {
+        float a0 = I == j ? 1.f : 0.f, a1 = 0.f;
+#pragma unroll
+        for (int m = 0; m < I; ++m) {
+            if (m & 1)
+                a1 = fmaf(row_bcast<I>(na[m]), x[m], a1);
+            else
+                a0 = fmaf(row_bcast<I>(na[m]), x[m], a0);
+        }
+        x[I] = a0 + a1;
+        solve_rows<I + 1>(na, x, j);
+    }
+}
+
+// A v head's part of a chunk's prep, on a team of 4 waves (w = 0..3, tid = 64 w
+// + lane): K K^T and Q K^T from the staged rows (wave w the 32 x 32 block (w /
+// 2, w % 2)), then A, T and M o QK^T with the head's gates (this lane's token's
+// dec and bet; n tokens in the chunk), into the head's block of the workspace.
+// sA / sM may lie over sK / sQ. The parts that take less than the four waves
+// start at wave `rot`: teams of one workgroup pass different ones, or they
+// would all fall to the same SIMD (a wave's place is its number modulo 4). mid() runs between the products and the first
+// barrier, its vector instructions under the products' MFMAs.
+template <class Mid>
+__device__ __forceinline__ void prep_head(f16 (*sK)[PK_P], f16 (*sQ)[PK_P], float (*sA)[PA_P],
+                                          float (*sM)[PA_P], float* sG, float* sB, float* sRed,
+                                          int tid, int n, float dec, float bet, char* blk,
+                                          int rot, Mid mid) {
+    const int lane = tid & 63, w = tid >> 6, wr = (w - rot) & 3;
     const int ql = lane & 31, hh = lane >> 5;
-    const int t0 = c * CK_C;
-    const int n = min(CK_C, T - t0);
-    const int hv0 = hv_blk;
-
-    // Every global load issued up front and unconditionally, rows clamped to
-    // the chunk's last token, past-the-end rows zeroed by a select: K and Q
-    // (4 rows x 16 B a thread), the first v head's beta and decay.
-    f16x8 kv8[4], qv8[4];
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        const int idx = tid + 256 * m, i = idx >> 4, c8 = (idx & 15) * 8;
-        const size_t off = (size_t)(t0 + min(i, n - 1)) * qk_stride + (size_t)hk * CK_K + c8;
-        kv8[m] = *(const f16x8*)(k + off);
-        qv8[m] = *(const f16x8*)(q + off);
-    }
-    const size_t gt = (size_t)(t0 + min(lane, n - 1)) * gates.stride + hv0;
-    float dec, bet;
-    if constexpr (LOGITS) {
-        const float av = gates.beta[gt], bv = gates.decay[gt];
-        const float dtb = gates.dt_bias[hv0], A = gates.A_log[hv0];
-        dec = gdn_decay(av + dtb, A);
-        bet = gdn_beta(bv);
-    } else {
-        dec = gates.decay[gt];
-        bet = gates.beta[gt];
-    }
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        const int idx = tid + 256 * m, i = idx >> 4, c8 = (idx & 15) * 8;
-        *(f16x8*)&sK[i][c8] = i < n ? kv8[m] : (f16x8)(0);
-        *(f16x8*)&sQ[i][c8] = i < n ? qv8[m] : (f16x8)(0);
-    }
-    __syncthreads();
-
     // K K^T and Q K^T: wave w the 32 x 32 block (bi, bj), kept in registers
     const int bi = w >> 1, bj = w & 1;
     f32x16 kk = (f32x16)(0.f), qk = (f32x16)(0.f);
@@ -294,83 +290,93 @@ chunk_prep_kernel(const f16* __restrict__ q, const f16* __restrict__ k, const Pr
         qk = __builtin_amdgcn_mfma_f32_32x32x16_f16(aq, bk, qk, 0, 0, 0);
     }
 
+    // this head's gates (decay 1 and beta 0 past the end: g stays at the last
+    // token's), the in-chunk prefix sums of log decay on one wave
+    if (wr == 0) {
+        const float gs = wave_prefix_sum(lane < n ? safe_log(dec) : 0.f);
+        sG[lane] = gs;
+        sB[lane] = lane < n ? bet : 0.f;
+    }
+    mid();
     {
-        const int hv = hv0;
-        char* blk = work + ((size_t)c * n_vheads + hv) * CK_BLK;
-        // this head's gates (decay 1 and beta 0 past the end: g stays at the
-        // last token's), the in-chunk prefix sums of log decay on wave 0
-        if (w == 0) {
-            const float gs = wave_prefix_sum(lane < n ? safe_log(dec) : 0.f);
-            sG[lane] = gs;
-            sB[lane] = lane < n ? bet : 0.f;
-        }
-        __syncthreads();   // the gates in; every K / Q read (or T / M o QK^T
-                           // read of the previous head) done
+        __syncthreads();   // the gates in; every K / Q read done
 
-        // A = strictly lower beta_i e^{g_i - g_j} k_i.k_j and M o QK^T. The
-        // 32 x 32 block above the diagonal (wave 1) is left alone: nothing
-        // reads M there, and T's blocks below the diagonal are written there
-        // (transposed) before anything reads it
+        // A = strictly lower beta_i e^{g_i - g_j} k_i.k_j and M o QK^T, rows i =
+        // 32 bi + 8 q + 4 hh + e of column j. The 32 x 32 block above the
+        // diagonal (wave 1) is left alone: nothing reads M there, and T's
+        // blocks below the diagonal are written there (transposed) before
+        // anything reads it. mt, mq: the running maxima of |T| and |M o QK^T|
+        // over their lower triangles (their operands' scales), kept as the
+        // values are formed. The rows' gates are read four at a time ahead of
+        // the stores: read one by one between them (the compiler has to
+        // assume that they alias) this part took 4.4 k clocks instead of 2 k
+        // with 12 waves on the LDS.
+        float mt = 0.f, mq = 0.f;
         if (bi >= bj) {
+            const int j = 32 * bj + ql;
+            const float gj = sG[j];
+            f32x4 gi[4], be[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                gi[q] = *(const f32x4*)&sG[32 * bi + 8 * q + 4 * hh];
+                be[q] = *(const f32x4*)&sB[32 * bi + 8 * q + 4 * hh];
+            }
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int i = 32 * bi + 8 * (r >> 2) + 4 * hh + (r & 3);
-                const int j = 32 * bj + ql;
                 // e^{g_i - g_j}, taken for every pair (above the diagonal it may
                 // be inf, and is not selected)
-                const float ratio = fast_exp2((sG[i] - sG[j]) * FL_LOG2E);
-                sA[i][j] = j < i ? sB[i] * ratio * kk[r] : 0.f;
-                sM[i][j] = j <= i ? ratio * qk[r] : 0.f;
+                const float ratio = fast_exp2((gi[r >> 2][r & 3] - gj) * FL_LOG2E);
+                const float m = j <= i ? ratio * qk[r] : 0.f;
+                sA[i][j] = j < i ? be[r >> 2][r & 3] * ratio * kk[r] : 0.f;
+                sM[i][j] = m;
+                mq = fmaxf(mq, fabsf(m));
             }
         }
         __syncthreads();
 
         // T = (I + A)^-1 by blocks of 16, in fp32: T_ii = D_i = (I + A_ii)^-1
-        // by forward substitution (wave i, lane j solving column j), then, a
-        // block diagonal at a time, T_ij = -D_i sum_{k = j .. i-1} A_ik T_kj on
-        // fp32 MFMA. T is kept transposed in sA's upper triangle
-        // (T_ij[a][b] at sA[16 j + b][16 i + a]), clear of A below the diagonal.
-        if (lane < 16) {
-            const int o = 16 * w, j = lane;
-            float xd[16];
+        // by forward substitution, then, a block diagonal at a time, T_ij = -D_i
+        // sum_{k = j .. i-1} A_ik T_kj on fp32 MFMA. T is kept transposed in
+        // sA's upper triangle (T_ij[a][b] at sA[16 j + b][16 i + a]), clear of A
+        // below the diagonal. The substitution is one wave's: lane 16 i + j holds
+        // row j of -A_ii and solves column j, row r's elements reaching the 16
+        // lanes of their block by DPP row broadcasts. (A wave a block, the
+        // elements read from LDS where they are used, kept the LDS busy for
+        // 8 k clocks with three teams at it.)
+        if (wr == 0) {
+            const int o = lane & 48, j = lane & 15;
+            float na[16];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                float a0 = i == j ? 1.f : 0.f, a1 = 0.f;
+            for (int m = 0; m < 16; m += 4) {
+                const f32x4 v = *(const f32x4*)&sA[lane][o + m];
 #pragma unroll
-                for (int m = 0; m < i; ++m) {
-                    if (m & 1)
-                        a1 = fmaf(-sA[o + i][o + m], xd[m], a1);
-                    else
-                        a0 = fmaf(-sA[o + i][o + m], xd[m], a0);
-                }
-                xd[i] = a0 + a1;
+                for (int e = 0; e < 4; ++e) na[m + e] = -v[e];
             }
-            // every element, the zeros above D_w's diagonal included: they land
-            // on A_ww, which the remaining steps do not read
+            float xd[16];
+            solve_rows<0>(na, xd, j);
 #pragma unroll
-            for (int i = 0; i < 16; ++i) sA[o + j][o + i] = xd[i];
+            for (int i = 0; i < 16; ++i) mt = fmaxf(mt, fabsf(xd[i]));
+            // every element, the zeros above D's diagonal included: they land on
+            // A_ii, which the remaining steps do not read
+#pragma unroll
+            for (int i = 0; i < 16; i += 4)
+                *(f32x4*)&sA[lane][o + i] = (f32x4){xd[i], xd[i + 1], xd[i + 2], xd[i + 3]};
         }
         __syncthreads();
+        auto level = [&](auto lv) {
+            constexpr int LV = decltype(lv)::value;
+            if (wr < 4 - LV) {
+                const f32x4 t = t_block<LV>(sA, wr, lane);
 #pragma unroll
-        for (int lv = 1; lv < 4; ++lv) {
-            if (w < 4 - lv) t_block(sA, w + lv, w, lane);
-            __syncthreads();
-        }
-
-        // the scales: block maxima of |T| and |M o QK^T| over their lower
-        // triangles, a row of each a pass (the lanes along it: no bank
-        // conflicts). sA[r][c] holds T[c][r] where c >= r (A's values below)
-        float mt = 0.f, mq = 0.f;
-#pragma unroll
-        for (int m = 0; m < CK_C * CK_C / 256; ++m) {
-            const int idx = tid + 256 * m, r = idx >> 6, c = idx & 63;
-            float tv = sA[r][c];
-            keep(tv);
-            mt = fmaxf(mt, c >= r ? fabsf(tv) : 0.f);
-            float qv = sM[r][c];
-            keep(qv);
-            mq = fmaxf(mq, c <= r ? fabsf(qv) : 0.f);
-        }
+                for (int r = 0; r < 4; ++r) mt = fmaxf(mt, fabsf(t[r]));
+            }
+        };
+        level(std::integral_constant<int, 1>());
+        __syncthreads();
+        level(std::integral_constant<int, 2>());
+        __syncthreads();
+        level(std::integral_constant<int, 3>());
         mt = wave_max(mt);
         mq = wave_max(mq);
         if (lane == 0) {
@@ -434,6 +440,279 @@ chunk_prep_kernel(const f16* __restrict__ q, const f16* __restrict__ k, const Pr
                     tid == 0 ? expf(gC) : tid == 1 ? t_inv : tid == 2 ? q_inv : 0.f;
         }
     }
+}
+
+// One workgroup of 4 waves a (chunk, v head), a grid of chunks x v heads: it
+// loads its k head's K and Q rows of the chunk, then prep_head.
+template <bool LOGITS>
+__global__ void __launch_bounds__(256)
+chunk_prep_kernel(const f16* __restrict__ q, const f16* __restrict__ k, const PrepGates gates,
+                  int T, int n_vheads, int qk_stride, int group, char* __restrict__ work) {
+    __shared__ __attribute__((aligned(16))) char smem[2 * CK_C * PK_P * 2];
+    __shared__ __attribute__((aligned(16))) float sG[CK_C], sB[CK_C];
+    __shared__ float sRed[8];
+    f16(*sK)[PK_P] = (f16(*)[PK_P])smem;
+    f16(*sQ)[PK_P] = (f16(*)[PK_P])(smem + CK_C * PK_P * 2);
+    float(*sA)[PA_P] = (float(*)[PA_P])smem;                     // after the products
+    float(*sM)[PA_P] = (float(*)[PA_P])(smem + CK_C * PA_P * 4);
+
+    const int c = blockIdx.x, hv0 = blockIdx.y, hk = hv0 / group;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int t0 = c * CK_C;
+    const int n = min(CK_C, T - t0);
+
+    // Every global load issued up front and unconditionally, rows clamped to
+    // the chunk's last token, past-the-end rows zeroed by a select: K and Q
+    // (4 rows x 16 B a thread), the first v head's beta and decay.
+    f16x8 kv8[4], qv8[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        const int idx = tid + 256 * m, i = idx >> 4, c8 = (idx & 15) * 8;
+        const size_t off = (size_t)(t0 + min(i, n - 1)) * qk_stride + (size_t)hk * CK_K + c8;
+        kv8[m] = *(const f16x8*)(k + off);
+        qv8[m] = *(const f16x8*)(q + off);
+    }
+    const size_t gt = (size_t)(t0 + min(lane, n - 1)) * gates.stride + hv0;
+    float dec, bet;
+    if constexpr (LOGITS) {
+        const float av = gates.beta[gt], bv = gates.decay[gt];
+        const float dtb = gates.dt_bias[hv0], A = gates.A_log[hv0];
+        dec = gdn_decay(av + dtb, A);
+        bet = gdn_beta(bv);
+    } else {
+        dec = gates.decay[gt];
+        bet = gates.beta[gt];
+    }
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        const int idx = tid + 256 * m, i = idx >> 4, c8 = (idx & 15) * 8;
+        *(f16x8*)&sK[i][c8] = i < n ? kv8[m] : (f16x8)(0);
+        *(f16x8*)&sQ[i][c8] = i < n ? qv8[m] : (f16x8)(0);
+    }
+    __syncthreads();
+    prep_head(sK, sQ, sA, sM, sG, sB, sRed, tid, n, dec, bet,
+              work + ((size_t)c * n_vheads + hv0) * CK_BLK, 0, [] {});
+}
+
+// ---------------------------------------------------------------------------
+// gdn_front_kernel: everything of a GDN prefill layer ahead of the state pass,
+// a workgroup of 12 waves a (chunk, k head): the causal conv (width 4) of the
+// k head's q and k channels and of its FG v heads' channels over the chunk's
+// 64 tokens, the L2 norm of the q and k rows, and then a team of 4 waves a v
+// head the prep (prep_head) on the rows still in LDS. Separately (conv, norm
+// and prep kernels, the q / k rows through HBM between them and read by every
+// v head) the three took 18 + 5.7 + 15 us of a 1024-token layer's 89; here
+// 16 chunks x 16 k heads are one workgroup a CU and 23 us (kernel traces).
+// Bound by the conv's vector instructions (of 43 k clocks ~18 k, most of them
+// the silu), then the chain from A to T's operands (~13 k) that one workgroup
+// a CU leaves exposed. 139 KiB of LDS.
+//
+// Conv: a 16-lane group takes one head's 128 channels (8 a lane) of 4
+// consecutive tokens, all 7 rows requested at once; the chunk's 5 heads x 16
+// token blocks are 20 wave tasks: waves 0-3 q, 4-7 k, 8-11 the first v head,
+// then waves 0-7 the other two under the products' MFMAs, 5 tasks a SIMD. Same
+// taps order, silu and roundings as conv_window_kernel; the norm's sums in the
+// order of l2norm_rows_kernel.
+// ---------------------------------------------------------------------------
+constexpr int FG = 3;                        // v heads a k head
+constexpr int FR_THREADS = 256 * FG;
+constexpr int FR_TB = 4;                     // tokens a conv task
+constexpr int FR_TILE = CK_C * PK_P * 2;     // staged K or Q rows; A or M o QK^T of a team
+constexpr int FR_LDS = 2 * FR_TILE + FG * 2 * FR_TILE + FG * (2 * CK_C + 8) * 4;
+static_assert(FR_LDS <= 160 * 1024, "the front kernel's LDS fits 160 KiB");
+
+// v of the lane 4 or 8 further round its 16-lane row (DPP row rotations)
+template <int D>
+__device__ __forceinline__ float row_ror(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x120 + D, 0xF, 0xF, true));
+}
+
+// One 16-lane group's conv rows in flight: E[j] = row (tb - 3 + j) of its 8
+// channels, the taps [channel][tap].
+struct FrontRows {
+    f16x8 e[FR_TB + 3];
+    f16x8 w[4];
+};
+
+// Task of the group: head `ch0` (its first channel + 8 times this lane's place)
+// and the call's tokens tb .. tb + 3. Rows are clamped to [0, T): those before
+// the call are replaced by the stored frames (zeros at pos0 == 0), those after
+// it are not used.
+__device__ __forceinline__ FrontRows front_load(const f16* __restrict__ x,
+                                                const f16* __restrict__ conv_w,
+                                                const f16* __restrict__ st_in, int ch, int tb,
+                                                int T, int pos0, int x_stride) {
+    FrontRows r;
+#pragma unroll
+    for (int j = 0; j < FR_TB + 3; ++j)
+        r.e[j] = *(const f16x8*)(x + (size_t)min(max(tb - 3 + j, 0), T - 1) * x_stride + ch);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) r.w[m] = *(const f16x8*)(conv_w + (size_t)ch * 4 + 8 * m);
+    if (tb == 0) {
+        f16x8 h[3];   // [channel][frame]
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+            h[m] = pos0 > 0 ? *(const f16x8*)(st_in + (size_t)ch * 3 + 8 * m) : (f16x8)(f16)0.f;
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int c = 0; c < 8; ++c) r.e[j][c] = h[(3 * c + j) >> 3][(3 * c + j) & 7];
+    }
+    return r;
+}
+
+// acc + a[A] * b[B] of two packed fp16 pairs, fp32 (v_fma_mix reads the halves
+// as they stand: no conversions)
+template <int A, int B>
+__device__ __forceinline__ float fma_half(uint32_t a, uint32_t b, float acc) {
+    float r;
+    if constexpr (A == 0 && B == 0)
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,1,0]" : "=v"(r) : "v"(a), "v"(b), "v"(acc));
+    else if constexpr (A == 1 && B == 0)
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,1,0]"
+            : "=v"(r) : "v"(a), "v"(b), "v"(acc));
+    else if constexpr (A == 0)
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,1,0] op_sel_hi:[1,1,0]"
+            : "=v"(r) : "v"(a), "v"(b), "v"(acc));
+    else
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,1,0] op_sel_hi:[1,1,0]"
+            : "=v"(r) : "v"(a), "v"(b), "v"(acc));
+    return r;
+}
+
+// The conv of channels c and c + 1 (one word of a row) at token row i of the task
+__device__ __forceinline__ void conv_pair(const FrontRows& r, int i, int c, float& y0, float& y1) {
+    const u32x4 w = __builtin_bit_cast(u32x4, r.w[c >> 1]);   // channel c: words 0, 1; c + 1: 2, 3
+    uint32_t e[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) e[j] = __builtin_bit_cast(u32x4, r.e[i + j])[c >> 1];
+    y0 = fma_half<0, 0>(w[0], e[0], 0.f);
+    y1 = fma_half<0, 1>(w[2], e[0], 0.f);
+    y0 = fma_half<1, 0>(w[0], e[1], y0);
+    y1 = fma_half<1, 1>(w[2], e[1], y1);
+    y0 = fma_half<0, 0>(w[1], e[2], y0);
+    y1 = fma_half<0, 1>(w[3], e[2], y1);
+    y0 = fma_half<1, 0>(w[1], e[3], y0);
+    y1 = fma_half<1, 1>(w[3], e[3], y1);
+}
+
+// The task's outputs into cx (global, the conv'd and, NORM, normed rows) and,
+// NORM, into the staged rows `stage` at this lane's place (row tb - t0, zeros
+// past the call); the lane of the call's last token stores the new frames.
+template <bool NORM>
+__device__ __forceinline__ void front_conv(const FrontRows& r, f16* __restrict__ cx,
+                                           f16* __restrict__ st_out, f16 (*stage)[PK_P], int ch,
+                                           int c8, int t0, int tb, int T, int x_stride,
+                                           float l2eps) {
+    const int nt = T - tb;   // tokens of the task inside the call (may be <= 0)
+#pragma unroll
+    for (int i = 0; i < FR_TB; ++i) {
+        float yf[8];
+#pragma unroll
+        for (int c = 0; c < 8; c += 2) conv_pair(r, i, c, yf[c], yf[c + 1]);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) yf[c] = silu_f(yf[c]);
+        f16x8 out = f16_sat8(yf);
+        if constexpr (NORM) {
+            float xf[8], sq[8];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                xf[c] = (float)out[c];
+                sq[c] = xf[c] * xf[c];
+            }
+#pragma unroll
+            for (int c = 0; c < 8; ++c) sq[c] += dpp_xor2(sq[c]);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) sq[c] += dpp_xor1(sq[c]);
+            const float ss4 = ((sq[0] + sq[4]) + (sq[2] + sq[6])) + ((sq[1] + sq[5]) + (sq[3] + sq[7]));
+            // quads q and q + 2, then the two pairs: rotations by 8 and 4
+            float ss = ss4 + row_ror<8>(ss4);
+            ss += row_ror<4>(ss);
+            const float den = sqrtf(ss + l2eps);
+            float rd = __builtin_amdgcn_rcpf(den);
+            rd = fmaf(fmaf(-den, rd, 1.f), rd, rd);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {   // xf / den, rounded once (as div_big; den is normal)
+                const float q = xf[c] * rd;
+                yf[c] = fmaf(fmaf(-den, q, xf[c]), rd, q);
+            }
+            out = f16_sat8(yf);
+            if (i >= nt) out = (f16x8)(f16)0.f;
+            *(f16x8*)&stage[tb - t0 + i][c8] = out;
+        }
+        // (an opaque use: only the store is conditional, not the row's arithmetic)
+        asm volatile("" : "+v"(out));
+        if (i < nt) *(f16x8*)(cx + (size_t)(tb + i) * x_stride + ch) = out;
+    }
+    if (nt >= 1 && nt <= FR_TB) {   // the call's last token is here: the last three frames
+        f16x8 f[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            f[j] = r.e[1 + j];
+#pragma unroll
+            for (int i = 1; i < FR_TB; ++i)
+                if (i == nt - 1) f[j] = r.e[i + 1 + j];
+            f[j] = __builtin_elementwise_maximum(   // f16_sat of an fp16: inf to the largest
+                __builtin_elementwise_minimum(f[j], (f16x8)(f16)65504.f), (f16x8)(f16)-65504.f);
+        }
+        f16x8 h[3];   // [channel][frame]
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int c = 0; c < 8; ++c) h[(3 * c + j) >> 3][(3 * c + j) & 7] = f[j][c];
+#pragma unroll
+        for (int m = 0; m < 3; ++m) *(f16x8*)(st_out + (size_t)ch * 3 + 8 * m) = h[m];
+    }
+}
+
+__global__ void __launch_bounds__(FR_THREADS)
+gdn_front_kernel(const f16* __restrict__ x, const f16* __restrict__ conv_w,
+                 const f16* __restrict__ st_in, f16* __restrict__ st_out, f16* __restrict__ cx,
+                 const PrepGates gates, int T, int pos0, int n_kheads, int x_stride, float l2eps,
+                 char* __restrict__ work) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    f16(*sK)[PK_P] = (f16(*)[PK_P])smem;
+    f16(*sQ)[PK_P] = (f16(*)[PK_P])(smem + FR_TILE);
+    const int c = blockIdx.x, hk = blockIdx.y;
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // 0 .. 11
+    const int team = wv >> 2;                                          // v head hk FG + team
+    const int t0 = c * CK_C;
+    const int n = min(CK_C, T - t0);
+    const int c8 = 8 * (lane & 15);
+    const int kdim = n_kheads * CK_K;
+    // wave task wt: head wt / 4 (q, k, then the v heads), token blocks 4 (wt % 4) + lane / 16
+    auto first_ch = [&](int wt) {
+        const int head = wt >> 2;
+        return (head == 0 ? hk * CK_K
+                : head == 1 ? kdim + hk * CK_K
+                            : 2 * kdim + (hk * FG + head - 2) * CK_V) + c8;
+    };
+    const int tb = t0 + FR_TB * (4 * (wv & 3) + (lane >> 4));   // the same for both tasks of a wave
+    const int ch1 = first_ch(wv), ch2 = first_ch(wv + 4 * FG);
+    const FrontRows r1 = front_load(x, conv_w, st_in, ch1, tb, T, pos0, x_stride);
+    const int hv = hk * FG + team;
+    const size_t gt = (size_t)(t0 + min(lane, n - 1)) * gates.stride + hv;
+    const float av = gates.beta[gt], bv = gates.decay[gt];
+    const float dtb = gates.dt_bias[hv], A = gates.A_log[hv];
+    if (wv < 8)
+        front_conv<true>(r1, cx, st_out, wv < 4 ? sQ : sK, ch1, c8, t0, tb, T, x_stride, l2eps);
+    else
+        front_conv<false>(r1, cx, st_out, nullptr, ch1, c8, t0, tb, T, x_stride, l2eps);
+    // the second task's rows, on their way under the barrier and the products
+    FrontRows r2;
+    if (wv < 8) r2 = front_load(x, conv_w, st_in, ch2, tb, T, pos0, x_stride);
+    const float dec = gdn_decay(av + dtb, A), bet = gdn_beta(bv);
+    __syncthreads();   // the chunk's normed q and k rows staged
+    char* own = smem + 2 * FR_TILE + team * 2 * FR_TILE;
+    float* sml = (float*)(smem + 2 * FR_TILE + FG * 2 * FR_TILE) + team * (2 * CK_C + 8);
+    prep_head(sK, sQ, (float(*)[PA_P])own, (float(*)[PA_P])(own + FR_TILE), sml, sml + CK_C,
+              sml + 2 * CK_C, threadIdx.x & 255, n, dec, bet,
+              work + ((size_t)c * (n_kheads * FG) + hv) * CK_BLK, team, [&] {
+                  if (wv < 8)
+                      front_conv<false>(r2, cx, st_out, nullptr, ch2, c8, t0, tb, T, x_stride,
+                                        l2eps);
+              });
 }
 
 // ---------------------------------------------------------------------------
@@ -931,13 +1210,13 @@ chunk_state_kernel(const f16* __restrict__ q, const f16* __restrict__ k,
                        w - 2, g, i, l, n_chunks, 2 * qk_stride, 2 * v_stride, y_stride, out_scale);
 }
 
-// The state pass's dynamic LDS is above the 64 KiB default: raised once per
-// device (a mutex: callers may come from several threads).
+// The front kernel's and the state pass's dynamic LDS is above the 64 KiB
+// default: raised once per device (a mutex: callers may come from several threads).
 std::mutex g_cs_mu;
 constexpr int CS_MAX_DEVICES = 64;
 bool g_cs_done[CS_MAX_DEVICES];
 
-int raise_state_lds_limit() {
+int raise_lds_limit() {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= CS_MAX_DEVICES) {
         fl::set_error("gdn_chunk_state: no current device below index %d", CS_MAX_DEVICES);
@@ -946,8 +1225,11 @@ int raise_state_lds_limit() {
     std::lock_guard<std::mutex> lock(g_cs_mu);
     if (g_cs_done[dev]) return FL_OK;
     if (hipFuncSetAttribute((const void*)chunk_state_kernel,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, CS_LDS) != hipSuccess) {
-        fl::set_error("gdn_chunk_state: cannot raise the dynamic LDS limit to %d bytes", CS_LDS);
+                            hipFuncAttributeMaxDynamicSharedMemorySize, CS_LDS) != hipSuccess ||
+        hipFuncSetAttribute((const void*)gdn_front_kernel,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, FR_LDS) != hipSuccess) {
+        fl::set_error("gdn_chunk: cannot raise the dynamic LDS limit to %d bytes",
+                      CS_LDS > FR_LDS ? CS_LDS : FR_LDS);
         return FL_ELAUNCH;
     }
     g_cs_done[dev] = true;
@@ -967,6 +1249,18 @@ size_t fl_gdn_chunked_work_bytes(int T, int n_vheads, int K, int V, int chunk) {
 }  // extern "C"
 
 namespace {
+
+int launch_state(const void* q, const void* k, const void* v, float* S, void* y, int T,
+                 int n_vheads, int qk_stride, int v_stride, int y_stride, float out_scale,
+                 int group, const void* work, fl_stream_t stream) {
+    const int rc = raise_lds_limit();
+    if (rc) return rc;
+    hipLaunchKernelGGL(chunk_state_kernel, dim3(n_vheads * (CK_V / CS_ROWS)), dim3(256),
+                       CS_LDS, (hipStream_t)stream, (const f16*)q, (const f16*)k, (const f16*)v, S,
+                       (f16*)y, T, n_vheads, qk_stride, v_stride, y_stride, out_scale, group,
+                       (const char*)work);
+    return fl::check_launch("gdn_chunk_state");
+}
 
 int prefill_chunked(const void* q, const void* k, const void* v, const PrepGates& gates,
                     bool logits, float* S, void* y, int T, int n_kheads, int n_vheads, int K,
@@ -1001,13 +1295,8 @@ int prefill_chunked(const void* q, const void* k, const void* v, const PrepGates
                            qk_stride, group, (char*)work);
     int rc = fl::check_launch("gdn_chunk_prep");
     if (rc) return rc;
-    rc = raise_state_lds_limit();
-    if (rc) return rc;
-    hipLaunchKernelGGL(chunk_state_kernel, dim3(n_vheads * (CK_V / CS_ROWS)), dim3(256),
-                       CS_LDS, (hipStream_t)stream, (const f16*)q, (const f16*)k, (const f16*)v, S,
-                       (f16*)y, T, n_vheads, qk_stride, v_stride, y_stride, out_scale, group,
-                       (const char*)work);
-    return fl::check_launch("gdn_chunk_state");
+    return launch_state(q, k, v, S, y, T, n_vheads, qk_stride, v_stride, y_stride, out_scale, group,
+                        work, stream);
 }
 
 }  // namespace
@@ -1033,6 +1322,73 @@ int fl_gdn_prefill_chunked_logits(const void* q, const void* k, const void* v, c
     return prefill_chunked(q, k, v, PrepGates{a, b, A_log, dt_bias, ab_stride}, true, S, y, T,
                            n_kheads, n_vheads, K, V, qk_stride, v_stride, y_stride, out_scale,
                            group, chunk, work, work_bytes, stream);
+}
+
+size_t fl_gdn_prefill_layer_work_bytes(int T, int x_stride, int n_vheads, int K, int V) {
+    const size_t chunks = fl_gdn_chunked_work_bytes(T, n_vheads, K, V, CK_C);
+    if (chunks == 0 || x_stride < 1) return 0;
+    // the chunks' blocks, the conv'd (normed) rows, the unnormed outputs
+    return chunks + ((size_t)T * x_stride * 2 + 15) / 16 * 16 + (size_t)T * n_vheads * V * 2;
+}
+
+int fl_gdn_prefill_layer(const void* x, int x_stride, const void* conv_w, const void* st_in,
+                         void* st_out, int pos0, const float* a, const float* b, int ab_stride,
+                         const float* A_log, const float* dt_bias, float* S, const void* z,
+                         const float* norm_w, void* y, int T, int n_kheads, int n_vheads, int K,
+                         int V, float out_scale, float l2eps, float norm_eps, void* work,
+                         size_t work_bytes, fl_stream_t stream) {
+    FL_REQUIRE(x && conv_w && st_in && st_out && a && b && A_log && dt_bias && S && z && norm_w &&
+                   y && work,
+               "null pointer");
+    FL_REQUIRE(K == CK_K && V == CK_V, "K == V == 128");
+    FL_REQUIRE(T >= 1 && pos0 >= 0, "T >= 1, pos0 >= 0");
+    FL_REQUIRE(n_kheads >= 1 && n_vheads >= 1 && n_vheads % n_kheads == 0, "n_vheads % n_kheads");
+    const int dim = 2 * n_kheads * K + n_vheads * V;
+    FL_REQUIRE(x_stride >= dim && x_stride % 8 == 0, "x_stride covers q|k|v, a multiple of 8");
+    FL_REQUIRE(ab_stride >= n_vheads, "ab_stride >= n_vheads");
+    FL_REQUIRE(st_in != st_out, "st_in and st_out must be distinct buffers");
+    FL_REQUIRE(((uintptr_t)S & 15u) == 0 && ((uintptr_t)work & 15u) == 0, "16-byte aligned S, work");
+    const size_t need = fl_gdn_prefill_layer_work_bytes(T, x_stride, n_vheads, K, V);
+    if (work_bytes < need) {
+        fl::set_error("work: %zu bytes, fl_gdn_prefill_layer_work_bytes asks %zu", work_bytes, need);
+        return FL_ESCRATCH;
+    }
+    char* blocks = (char*)work;
+    f16* cx = (f16*)(blocks + fl_gdn_chunked_work_bytes(T, n_vheads, K, V, CK_C));
+    f16* yr = (f16*)((char*)cx + ((size_t)T * x_stride * 2 + 15) / 16 * 16);
+    const f16* q = cx;
+    const f16* k = cx + n_kheads * K;
+    const f16* v = cx + 2 * n_kheads * K;
+    const PrepGates gates = {a, b, A_log, dt_bias, ab_stride};
+    const int group = n_vheads / n_kheads;
+    auto al16 = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
+    int rc;
+    // the one-launch front takes the model's three v heads a k head with 16-byte
+    // rows; anything else the conv and norm kernels, then the chunked scan's
+    // own prep
+    if (group == FG && al16(x) && al16(conv_w) && al16(st_in) && al16(st_out)) {
+        rc = raise_lds_limit();
+        if (rc) return rc;
+        const int n_chunks = (T + CK_C - 1) / CK_C;
+        hipLaunchKernelGGL(gdn_front_kernel, dim3(n_chunks, n_kheads), dim3(FR_THREADS), FR_LDS,
+                           (hipStream_t)stream, (const f16*)x, (const f16*)conv_w,
+                           (const f16*)st_in, (f16*)st_out, cx, gates, T, pos0, n_kheads, x_stride,
+                           l2eps, blocks);
+        rc = fl::check_launch("gdn_front");
+        if (rc) return rc;
+        rc = launch_state(q, k, v, S, yr, T, n_vheads, x_stride, x_stride, n_vheads * V, out_scale,
+                          group, blocks, stream);
+    } else {
+        rc = fl_conv1d_causal(x, conv_w, st_in, cx, st_out, dim, T, pos0, x_stride, 4, stream);
+        if (rc) return rc;
+        rc = fl_l2norm_scaled_strided(cx, cx, 2 * n_kheads, K, x_stride, l2eps, 1.f, T, stream);
+        if (rc) return rc;
+        rc = prefill_chunked(q, k, v, gates, true, S, yr, T, n_kheads, n_vheads, K, V, x_stride,
+                             x_stride, n_vheads * V, out_scale, group, CK_C, blocks,
+                             fl_gdn_chunked_work_bytes(T, n_vheads, K, V, CK_C), stream);
+    }
+    if (rc) return rc;
+    return fl_rmsnorm_gated(yr, z, norm_w, y, V, n_vheads, V, T, norm_eps, stream);
 }
 
 }  // extern "C"

@@ -724,3 +724,32 @@ def gdn_prefill_chunked_logits(q, k, v, a, b, A_log, dt_bias, S, y=None, *, T: i
               V, qk_stride, v_stride, y.shape[-1], float(out_scale), group, chunk,
               _ptr(work, torch.uint8, "work", need), work.numel(), _stream())
     return y
+
+
+def gdn_prefill_layer(x, conv_w, st_in, st_out, a, b, A_log, dt_bias, S, z, norm_w, y=None, *,
+                      T: int, pos0: int, ab_stride: int = GDN_V_HEADS,
+                      n_kheads: int = GDN_K_HEADS, n_vheads: int = GDN_V_HEADS, K: int = GDN_K,
+                      V: int = GDN_V, x_stride: int = QKV_ROWS, out_scale: float = Q_SCALE,
+                      l2eps: float = L2_EPS, norm_eps: float = GDN_NORM_EPS, work=None):
+    """A GDN layer over a prompt's rows (runtime.py:3035-3111): conv1d_causal,
+    l2norm_scaled of q and k, gdn_prefill_chunked_logits and rmsnorm_gated in one
+    call. x [T, x_stride] fp16 the raw q|k|v rows, z [T, n_vheads, V] fp16; S
+    and st_out are written. Returns y [T, n_vheads, V] fp16."""
+    _contig(S, "S")
+    if y is None:
+        y = torch.empty((T, n_vheads, V), dtype=F16, device=x.device)
+    dim = 2 * n_kheads * K + n_vheads * V
+    need = int(_lib.lib().fl_gdn_prefill_layer_work_bytes(T, x_stride, n_vheads, K, V))
+    if work is None:
+        work = torch.empty(need, dtype=torch.uint8, device=x.device)
+    _lib.call("fl_gdn_prefill_layer", _ptr(x, F16, "x", (T - 1) * x_stride + dim), x_stride,
+              _ptr(conv_w, F16, "conv_w", dim * 4), _ptr(st_in, F16, "st_in", dim * 3),
+              _ptr(st_out, F16, "st_out", dim * 3), pos0,
+              _ptr(a, F32, "a", (T - 1) * ab_stride + n_vheads),
+              _ptr(b, F32, "b", (T - 1) * ab_stride + n_vheads), ab_stride,
+              _ptr(A_log, F32, "A_log", n_vheads), _ptr(dt_bias, F32, "dt_bias", n_vheads),
+              _ptr(S, F32, "S", n_vheads * V * K), _ptr(z, F16, "z", T * n_vheads * V),
+              _ptr(norm_w, F32, "norm_w", V), _ptr(y, F16, "y", T * n_vheads * V), T, n_kheads,
+              n_vheads, K, V, float(out_scale), float(l2eps), float(norm_eps),
+              _ptr(work, torch.uint8, "work", need), work.numel(), _stream())
+    return y

@@ -471,6 +471,24 @@ int fl_gdn_prefill_chunked_logits(const void* q, const void* k, const void* v, c
                                   int y_stride, float out_scale, int group, int chunk, void* work,
                                   size_t work_bytes, fl_stream_t stream);
 
+/* A GDN layer over a prompt's T tokens, from its projected rows to its normed
+ * output: conv1d_causal (width 4), l2norm_scaled of the q and k rows, the gates
+ * and the chunked scan (fl_gdn_prefill_chunked_logits), rmsnorm_gated -- the
+ * sequence runtime.py:3035-3111 launches, the same values as the separate
+ * calls; the conv, the norm and the scan's prep are one launch where a k head
+ * has three v heads. x [T][x_stride] f16 the raw q|k|v rows; conv_w [dim][4],
+ * st_in / st_out [dim][3] f16 as fl_conv1d_causal's (distinct); a, b
+ * [T][ab_stride] f32; S as fl_gdn_prefill_chunked; z, y [T][n_vheads][V] f16,
+ * norm_w [V] f32. work: fl_gdn_prefill_layer_work_bytes(...) bytes, 16-byte
+ * aligned. K == V == 128, x_stride a multiple of 8. */
+size_t fl_gdn_prefill_layer_work_bytes(int T, int x_stride, int n_vheads, int K, int V);
+int fl_gdn_prefill_layer(const void* x, int x_stride, const void* conv_w, const void* st_in,
+                         void* st_out, int pos0, const float* a, const float* b, int ab_stride,
+                         const float* A_log, const float* dt_bias, float* S, const void* z,
+                         const float* norm_w, void* y, int T, int n_kheads, int n_vheads, int K,
+                         int V, float out_scale, float l2eps, float norm_eps, void* work,
+                         size_t work_bytes, fl_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

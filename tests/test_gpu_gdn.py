@@ -696,3 +696,41 @@ def test_verify_normed_equals_verify_then_norm(fl, dev, rng, B, T):
     for i in range(B):
         assert torch.equal(Sf[i], Su[i]), f"seq {i}: state differs"
         assert torch.equal(ckf[i], cku[i]), f"seq {i}: checkpoints differ"
+
+
+# token counts around the conv's 4-token tasks, the 3 frames of history and the
+# 64-token chunk; x_off 1 shifts the rows off 16-byte alignment (the separate
+# kernels inside the call)
+@pytest.mark.parametrize("T,pos0,x_off", [(1, 0, 0), (2, 7, 0), (3, 0, 0), (5, 9, 0), (63, 0, 0),
+                                          (64, 5, 0), (65, 0, 0), (130, 64, 0), (1000, 0, 0),
+                                          (70, 3, 1)])
+def test_prefill_layer_equals_separate_calls(fl, dev, rng, T, pos0, x_off):
+    """A GDN layer's prefill in one call against conv1d_causal,
+    l2norm_scaled_strided, gdn_prefill_chunked_logits and rmsnorm_gated: the
+    normed rows, the state and the conv frames bit for bit."""
+    x = (rng.standard_normal(T * ROW + x_off) * 1.5).astype(np.float16)
+    xd = to_dev(x, dev)[x_off:].view(T, ROW)
+    w = to_dev((rng.standard_normal((ROW, 4)) * 0.5).astype(np.float16), dev)
+    st = to_dev(rng.standard_normal((ROW, 3)).astype(np.float16), dev)
+    ad = to_dev(rng.standard_normal((T, NV)).astype(np.float32), dev)
+    bd = to_dev(rng.standard_normal((T, NV)).astype(np.float32), dev)
+    A_log = to_dev((rng.standard_normal(NV) * 0.3).astype(np.float32), dev)
+    dt = to_dev((rng.standard_normal(NV) * 0.3).astype(np.float32), dev)
+    z = to_dev(rng.standard_normal((T, NV, 128)).astype(np.float16), dev)
+    nw = to_dev((1 + rng.standard_normal(128) * 0.2).astype(np.float32), dev)
+    S1 = to_dev((rng.standard_normal((NV, 128, 128)) * 0.05).astype(np.float32), dev)
+    S2 = S1.clone()
+    so1, so2 = torch.full_like(st, 9.0), torch.full_like(st, 9.0)
+    y1 = fl.ops.gdn_prefill_layer(xd, w, st, so1, ad, bd, A_log, dt, S1, z, nw, T=T, pos0=pos0)
+    c = torch.empty((T, ROW), dtype=torch.float16, device=dev)
+    ln = torch.empty_like(c)
+    fl.ops.conv1d_causal(xd, w, st, c, so2, T=T, pos0=pos0)
+    fl.ops.l2norm_scaled_strided(c, ln, rows=32, token_stride=ROW, T=T)
+    yr = fl.ops.gdn_prefill_chunked_logits(ln[:, :2048], ln[:, 2048:4096], c[:, 4096:], ad, bd,
+                                           A_log, dt, S2, T=T)
+    y2 = fl.ops.rmsnorm_gated(yr.view(T, NV, 128), z, nw, T=T)
+    torch.cuda.synchronize()
+    assert torch.isfinite(y1.float()).all()
+    assert torch.equal(so1, so2), "conv frames differ"
+    assert torch.equal(S1, S2), "state differs"
+    assert torch.equal(y1, y2), "normed rows differ"
