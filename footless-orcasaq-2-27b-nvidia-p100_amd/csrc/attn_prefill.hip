@@ -493,13 +493,18 @@ attn_prefill_kernel(const f16* __restrict__ q, int q_pitch, const void* __restri
 // One HBM -> LDS copy of 16 bytes a lane to LDS dst + IMM (+ 16 lane). m0 is
 // set inside the asm from a wave-uniform base and an immediate, so the
 // compiler keeps no per-copy LDS addresses in SGPRs (it would otherwise hoist
-// all of them out of the tile loop); the asm declares m0 as its output.
+// all of them out of the tile loop); the asm declares m0 as its output, and that
+// the s_add overwrites SCC: without that the compiler put a copy between the two
+// halves of a 64-bit address add (s_add_u32 .. s_addc_u32) and the carry was
+// lost, so a V cache whose rows cross a 4 GiB boundary of the address space was
+// read 4 GiB below it (a memory fault, or another allocation's bytes).
 template <int IMM>
 __device__ __forceinline__ void copy16_at(const char* sbase, uint32_t voff, uint32_t dst) {
     uint32_t m0v;
     asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                  : "={m0}"(m0v)
-                 : "v"(voff), "s"(sbase), "s"(dst), "i"(IMM));
+                 : "v"(voff), "s"(sbase), "s"(dst), "i"(IMM)
+                 : "scc");
 }
 
 // ---------------------------------------------------------------------------

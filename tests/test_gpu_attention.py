@@ -395,6 +395,31 @@ def test_prefill_kv_split_vs_oracle(fl, dev, orc, rng, T, pos0, split):
     assert ok, f"T={T} pos0={pos0} split={split}: max|err| {err}"
 
 
+# the long-prompt kernel whole (4096 tokens) and with its KV split (683 at 16000)
+@pytest.mark.parametrize("T,pos0", [(4096, 0), (683, 16000)])
+@pytest.mark.parametrize("which", ["k", "v"])
+def test_prefill_cache_across_4gib_boundary(fl, dev, T, pos0, which):
+    """A K or V cache whose rows cross a 4 GiB boundary of the address space: the
+    row addresses of the tile copies carry into their upper half there. The
+    same bits as over a copy of it elsewhere."""
+    L = pos0 + T
+    n = L * 4 * 256 * 2
+    g = torch.Generator(device=dev).manual_seed(L)
+    q = (torch.randn((T, 24, 256), generator=g, device=dev) / 16).half()
+    cache = {c: torch.randn((L, 4, 256), generator=g, device=dev).half() for c in "kv"}
+    room = torch.empty((1 << 32) + 2 * n, dtype=torch.uint8, device=dev)
+    base = room.data_ptr()
+    at = (base + n + (1 << 32) - 1 >> 32 << 32) - n // 2 // 4096 * 4096
+    assert base <= at and at + n <= base + room.numel() and at >> 32 != (at + n - 1) >> 32
+    across = room[at - base:at - base + n].view(torch.float16).view(L, 4, 256)
+    across.copy_(cache[which])
+    want = fl.ops.attention_prefill(q, cache["k"], cache["v"], pos0=pos0, scale=1.0)
+    got = fl.ops.attention_prefill(q, *(across if c == which else cache[c] for c in "kv"),
+                                   pos0=pos0, scale=1.0)
+    torch.cuda.synchronize()
+    assert torch.isfinite(want.float()).all() and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("T,pos0,split", [(683, 16000, 5), (700, 15700, 16)])
 def test_prefill_r64_kv_split_vs_fp32(fl, dev, T, pos0, split):
     """The 64-rows-a-wave kernel's KV split (>= 64 workgroups of 256 rows and

@@ -266,11 +266,6 @@ def test_prefill_q8_staged_equals_direct(fl, dev, orc, rng):
     assert ok, f"staged vs direct: max|err| {err}"
 
 
-@pytest.mark.skip(reason="T=1024 at pos0=98000 over an int8 cache: a timing sweep that ran this "
-                         "call with four builds of the library loaded in one process ended in a "
-                         "GPU memory fault; no out-of-bounds access was found in the int8 split "
-                         "kernel, the staging copy, the 64-rows-a-wave split kernel or the merge, "
-                         "so the call stays off the GPU until a cause is shown")
 def test_prefill_q8_chunk_deep_in_prompt(fl, dev, orc):
     """The reference's prefill shape over its shipped int8 cache: a 1024-token
     chunk (MAX_CHUNK, runtime.py:196) at pos0 = 98000, sampled rows against the
