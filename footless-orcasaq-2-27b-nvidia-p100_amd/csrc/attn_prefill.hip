@@ -39,7 +39,9 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <functional>
 #include <mutex>
+#include <queue>
 #include <vector>
 
 namespace {
@@ -57,6 +59,11 @@ constexpr int V_OFF = 2 * TILE_B;
 // than this (log2 units): P = 2^(s - m) stays <= 256, exact in fp16 range,
 // and the O / l rescale is skipped on almost every tile.
 constexpr float RESCALE_LOG2 = 8.f;
+
+// f16_sat for this file's NaN-free arithmetic (-fno-honor-nans): one median
+__device__ __forceinline__ f16 z_sat(float v) {
+    return (f16)__builtin_amdgcn_fmed3f(v, -65504.f, 65504.f);
+}
 
 // the chunk swizzle of tile row r: chunk c is stored at c ^ sw(r)
 __device__ __forceinline__ int sw(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
@@ -485,8 +492,8 @@ attn_prefill_kernel(const f16* __restrict__ q, int q_pitch, const void* __restri
 #pragma unroll
             for (int r4 = 0; r4 < 4; ++r4)
                 *(f16x4*)(zrow + 32 * mb + 8 * r4) =
-                    (f16x4){f16_sat(o[mb][4 * r4] * inv), f16_sat(o[mb][4 * r4 + 1] * inv),
-                            f16_sat(o[mb][4 * r4 + 2] * inv), f16_sat(o[mb][4 * r4 + 3] * inv)};
+                    (f16x4){z_sat(o[mb][4 * r4] * inv), z_sat(o[mb][4 * r4 + 1] * inv),
+                            z_sat(o[mb][4 * r4 + 2] * inv), z_sat(o[mb][4 * r4 + 3] * inv)};
     }
 }
 
@@ -644,28 +651,74 @@ __device__ __forceinline__ void r64_vfrags(s16x4 (&vb)[8], const char* vt,
         vb[i] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vt + b[i] + imm));
 }
 
-// SPLIT: blockIdx.z is the KV split (tile grid only, bins == 0): the
-// workgroup walks tiles [n s / S, n (s + 1) / S) of its causal range (n
-// tiles) and leaves the partials in `sp`, as attn_prefill_kernel<Q8, true>.
-template <bool SPLIT>
+// A call's work over one kv head as a list of pieces (STREAM): the row tiles'
+// causal walks laid end to end and cut into `bins` runs of equal cost, one a
+// workgroup, wherever the cuts fall. Bin b runs from tile start[b].tile, KV tile
+// start[b].j, up to start[b + 1]. Every piece leaves a partial, a row tile's in
+// slots slot0[tile] .. slot0[tile + 1] - 1 of its kv head in KV order (an uncut
+// tile's in its one slot: a second epilogue for it costs more registers than
+// the kernel has); `first[b]` is bin b's first piece's slot. v[]: start (2 (bins
+// + 1)), first (bins), slot0 (row tiles + 1).
+struct StreamAt {
+    const uint16_t* v;
+    int bins;
+    __device__ __forceinline__ int at(int i) const {   // (uniform)
+        return __builtin_amdgcn_readfirstlane((int)v[i]);
+    }
+    __device__ __forceinline__ int tile(int b) const { return at(2 * b); }
+    __device__ __forceinline__ int j(int b) const { return at(2 * b + 1); }
+    __device__ __forceinline__ int first(int b) const { return at(2 * (bins + 1) + b); }
+    __device__ __forceinline__ int slot0(int t) const { return at(3 * bins + 2 + t); }
+};
+// The partials of all kv heads: O unnormalised [slot][256 rows][256], then the
+// running max (natural-log units) and sum [slot][256 rows]; kv head h's slots
+// start at h * n.
+struct StreamOut {
+    float* pacc;
+    float* pm;
+    float* pd;
+    int n;   // slots a kv head (R64_PIECES), splits (R64_SPLIT)
+};
+
+// R64_ROWS: whole row tiles, bins > 0 the persistent plan's lists or bins == 0 a
+// grid of row tiles x kv heads, to z. R64_SPLIT: that grid with the uniform KV
+// split blockIdx.z of so.n, partials to `so` in the decode layout (PfSplit's).
+// R64_PIECES: `plan` is a piece list (bins workgroups a kv head), partials to
+// `so` a slot a piece.
+enum { R64_ROWS, R64_SPLIT, R64_PIECES };
+template <int MODE>
 __global__ void __launch_bounds__(PF_THREADS)
 attn_prefill_r64_kernel(const f16* __restrict__ q, int q_pitch, const f16* __restrict__ kc,
                         const f16* __restrict__ vc, f16* __restrict__ z, int z_pitch,
                         int n_q_heads, int n_kv, int pos0, int T, float sl2, int n_row_tiles,
-                        int bins, const R64Plan plan, PfSplit sp) {
+                        int bins, const R64Plan plan, StreamOut so) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
+    constexpr bool STREAM = MODE == R64_PIECES, SPLIT = MODE == R64_SPLIT;
 
     // This workgroup's row tiles: one, of a grid of row tiles x kv heads
     // (bins == 0), or the list of its bin, of a grid of one workgroup a CU.
     int h, tile = 0, item0 = 0, n_items = 1;
+    int j_first = 0, j_last = 0, slot = 0;   // STREAM: the first piece's start, the last one's end
+    const StreamAt sa = {plan.v, bins};
     if (bins == 0) {
         xcd_tile(n_row_tiles, n_kv, tile, h);
     } else {
         const int id = blockIdx.x, xcd = id & 7, per = 8 / n_kv;
         h = xcd / per;
         const int bin = (id >> 3) * per + xcd % per;
-        item0 = plan.v[bin];
-        n_items = plan.v[bin + 1] - item0;
+        if constexpr (STREAM) {
+            if (bin >= bins) return;   // a short call: fewer bins than CUs
+            item0 = sa.tile(bin);
+            j_first = sa.j(bin);
+            j_last = sa.j(bin + 1);
+            // the tiles entered: the one the next bin starts in counts if this
+            // bin has a share of it
+            n_items = sa.tile(bin + 1) - item0 + (j_last > 0 ? 1 : 0);
+            slot = sa.first(bin);
+        } else {
+            item0 = plan.v[bin];
+            n_items = plan.v[bin + 1] - item0;
+        }
     }
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -695,7 +748,10 @@ attn_prefill_r64_kernel(const f16* __restrict__ q, int q_pitch, const f16* __res
                                 16 * ((tr_d >> 3) ^ (hh + 2 * s2)) + 2 * (tr_d & 7);
 
     for (int it = 0; it < n_items; ++it) {
-        if (bins != 0) tile = __builtin_amdgcn_readfirstlane(plan.v[bins + 1 + item0 + it]);
+        if (STREAM)
+            tile = item0 + it;
+        else if (bins != 0)
+            tile = __builtin_amdgcn_readfirstlane(plan.v[bins + 1 + item0 + it]);
         if (it > 0) tile_done();   // every wave is done with the previous row tile's stages
         const int R0 = tile * R64_BQ;
         // this lane's two query rows (columns of the two MFMA blocks)
@@ -715,30 +771,35 @@ attn_prefill_r64_kernel(const f16* __restrict__ q, int q_pitch, const f16* __res
         const int wqmin = __builtin_amdgcn_readfirstlane(pos0 + wfirst / G);
         const int blast = min(R0 + R64_BQ - 1, RT - 1);
         const int kv_end = __builtin_amdgcn_readfirstlane(pos0 + blast / G + 1);
-        // this item's tiles [j_lo, j_lo + n_tiles): all, or split s's share
+        // this item's tiles [j_lo, j_lo + n_tiles): all of them, split s's share, or
+        // the bin's
         const int n_all = (kv_end + R64_BK - 1) / R64_BK;
         const int s_idx = SPLIT ? (int)blockIdx.z : 0;
-        const int j_lo = SPLIT ? __builtin_amdgcn_readfirstlane(n_all * s_idx / sp.n) : 0;
+        const int j_lo = SPLIT            ? __builtin_amdgcn_readfirstlane(n_all * s_idx / so.n)
+                         : STREAM && it == 0 ? j_first
+                                             : 0;
         const int n_tiles =
-            SPLIT ? __builtin_amdgcn_readfirstlane(n_all * (s_idx + 1) / sp.n) - j_lo : n_all;
+            __builtin_amdgcn_readfirstlane(SPLIT ? n_all * (s_idx + 1) / so.n
+                                           : STREAM && it == n_items - 1 && j_last > 0 ? j_last
+                                                                                       : n_all) -
+            j_lo;
         if constexpr (SPLIT) {
             if (n_tiles == 0) {   // an empty split: the empty partial (uniform exit)
 #pragma unroll
                 for (int nb = 0; nb < 2; ++nb) {
                     if (!rvalid[nb]) continue;
-                    const size_t part = ((size_t)t[nb] * n_q_heads + h * G + g[nb]) * sp.n + s_idx;
-                    float* acc = sp.pacc + part * PF_HD + 4 * hh;
+                    const size_t part = ((size_t)t[nb] * n_q_heads + h * G + g[nb]) * so.n + s_idx;
+                    float* acc = so.pacc + part * PF_HD + 4 * hh;
 #pragma unroll
                     for (int i = 0; i < 32; ++i) *(f32x4*)(acc + 8 * i) = (f32x4)(0.f);
                     if (hh == 0) {
-                        sp.pm[part] = -1e30f;
-                        sp.pd[part] = 0.f;
+                        so.pm[part] = -1e30f;
+                        so.pd[part] = 0.f;
                     }
                 }
                 continue;
             }
         }
-
 
 #pragma unroll
         for (int d = 0; d < R64_DIST; ++d)
@@ -752,7 +813,10 @@ attn_prefill_r64_kernel(const f16* __restrict__ q, int q_pitch, const f16* __res
             const f16* qrow = q + ((size_t)t[nb] * n_q_heads + h * G + g[nb]) * q_pitch + 128 * hh;
 #pragma unroll
             for (int ks = 0; ks < 16; ++ks)
-                qreg[nb][ks] = rvalid[nb] ? *(const f16x8*)(qrow + 8 * ks) : (f16x8)(0);
+                // (STREAM: unconditional, a lane past the rows reads token 0's row and
+                // its column is never stored: 3 % at T = 777 from 3001; the other
+                // modes' tile loop is scheduled 2 - 3 % worse without the select)
+                qreg[nb][ks] = STREAM || rvalid[nb] ? *(const f16x8*)(qrow + 8 * ks) : (f16x8)(0);
         }
         WAIT_VMCNT(0);   // Q and the first tiles: the wait left to the compiler lands in the loop
 
@@ -825,13 +889,16 @@ attn_prefill_r64_kernel(const f16* __restrict__ q, int q_pitch, const f16* __res
 
         acc_settle(o[0]);
         acc_settle(o[1]);
-        if constexpr (SPLIT) {
+        if constexpr (STREAM || SPLIT) {
             // dims 32 mb + 8 r4 + 4 hh + 0..3 of O, unnormalised; m in natural-log units
+            const int sl = STREAM ? (it == 0 ? slot : sa.slot0(tile)) + h * so.n : 0;
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb) {
                 if (!rvalid[nb]) continue;
-                const size_t part = ((size_t)t[nb] * n_q_heads + h * G + g[nb]) * sp.n + s_idx;
-                float* acc = sp.pacc + part * PF_HD + 4 * hh;
+                const size_t part =
+                    STREAM ? (size_t)sl * R64_BQ + 64 * w + 32 * nb + ql
+                           : ((size_t)t[nb] * n_q_heads + h * G + g[nb]) * so.n + s_idx;
+                float* acc = so.pacc + part * PF_HD + 4 * hh;
 #pragma unroll
                 for (int mb = 0; mb < 8; ++mb)
 #pragma unroll
@@ -840,8 +907,8 @@ attn_prefill_r64_kernel(const f16* __restrict__ q, int q_pitch, const f16* __res
                             (f32x4){o[nb][mb][4 * r4], o[nb][mb][4 * r4 + 1], o[nb][mb][4 * r4 + 2],
                                     o[nb][mb][4 * r4 + 3]};
                 if (hh == 0) {
-                    sp.pm[part] = l_run[nb] > 0.f ? m_run[nb] * FL_LN2 : -1e30f;
-                    sp.pd[part] = l_run[nb];
+                    so.pm[part] = l_run[nb] > 0.f ? m_run[nb] * FL_LN2 : -1e30f;
+                    so.pd[part] = l_run[nb];
                 }
             }
             continue;
@@ -856,10 +923,73 @@ attn_prefill_r64_kernel(const f16* __restrict__ q, int q_pitch, const f16* __res
 #pragma unroll
                 for (int r4 = 0; r4 < 4; ++r4)
                     *(f16x4*)(zrow + 32 * mb + 8 * r4) = (f16x4){
-                        f16_sat(o[nb][mb][4 * r4] * inv), f16_sat(o[nb][mb][4 * r4 + 1] * inv),
-                        f16_sat(o[nb][mb][4 * r4 + 2] * inv), f16_sat(o[nb][mb][4 * r4 + 3] * inv)};
+                        z_sat(o[nb][mb][4 * r4] * inv), z_sat(o[nb][mb][4 * r4 + 1] * inv),
+                        z_sat(o[nb][mb][4 * r4 + 2] * inv), z_sat(o[nb][mb][4 * r4 + 3] * inv)};
         }
     }
+}
+
+// The merge of a piece list's partials, with the output gate (attn_gate) when
+// `gate` (the call's q | gate rows, the gate 256 halves into a head's row) is
+// given: one wavefront a (token, q head), lane l holding dims 4 l .. 4 l + 3,
+// its row tile's pieces in batches of eight against one running max
+// (attn_merge_rows_kernel's arithmetic).
+constexpr int SM_PAIRS = 4;   // (token, head) pairs a workgroup
+constexpr int SM_BATCH = 8;
+__global__ void __launch_bounds__(64 * SM_PAIRS)
+attn_prefill_stream_merge_kernel(const StreamOut so, f16* __restrict__ z, int z_pitch,
+                                 const f16* __restrict__ gate, int g_pitch, int n_q_heads, int G,
+                                 int bins, int n_pairs, const R64Plan plan) {
+    const int lane = threadIdx.x & 63;
+    const int rh = __builtin_amdgcn_readfirstlane(blockIdx.x * SM_PAIRS + (threadIdx.x >> 6));
+    if (rh >= n_pairs) return;   // wave-uniform
+    const int t = rh / n_q_heads, head = rh - t * n_q_heads, h = head / G;
+    const int row = t * G + head - h * G;   // among its kv head's rows
+    const int tile = row / R64_BQ;
+    const StreamAt sa = {plan.v, bins};
+    const int s0 = sa.slot0(tile), ns = sa.slot0(tile + 1) - s0;
+    f16x4 gv = {};
+    if (gate != nullptr) gv = *(const f16x4*)(gate + (size_t)rh * g_pitch + PF_HD + 4 * lane);
+    const size_t p0 = (size_t)(h * so.n + s0) * R64_BQ + (row - tile * R64_BQ);
+    const f32x4* acc = (const f32x4*)(so.pacc + p0 * PF_HD) + lane;
+    f32x4 num = (f32x4)(0.f);
+    float den = 0.f, M = -1e30f;
+    for (int s = 0; s < ns; s += SM_BATCH) {
+        float mv[SM_BATCH], dv[SM_BATCH];
+        f32x4 av[SM_BATCH];
+#pragma unroll
+        for (int u = 0; u < SM_BATCH; ++u) {
+            if (s + u >= ns) break;   // uniform: no load past the row's pieces
+            const size_t si = (size_t)(s + u) * R64_BQ;
+            mv[u] = so.pm[p0 + si];
+            dv[u] = so.pd[p0 + si];
+            av[u] = acc[si * (PF_HD / 4)];
+        }
+        float bm = M;
+#pragma unroll
+        for (int u = 0; u < SM_BATCH; ++u)
+            if (s + u < ns) bm = fmaxf(bm, mv[u]);
+        const float corr = fast_exp2((M - bm) * FL_LOG2E);
+        num *= corr;
+        den *= corr;
+        M = bm;
+#pragma unroll
+        for (int u = 0; u < SM_BATCH; ++u) {
+            if (s + u >= ns) break;
+            const float e = fast_exp2((mv[u] - M) * FL_LOG2E);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) num[d] = fmaf(e, av[u][d], num[d]);
+            den = fmaf(e, dv[u], den);
+        }
+    }
+    const float inv = 1.f / den;
+    f16x4 out;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        out[d] = f16_sat(num[d] * inv);
+        if (gate != nullptr) out[d] = f16_sat((float)out[d] * sigmoid_f((float)gv[d]));
+    }
+    *(f16x4*)(z + (size_t)rh * z_pitch + 4 * lane) = out;
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
@@ -893,8 +1023,9 @@ int prefill_device_setup(int& n_cu) {
             fl::set_error("attn_prefill: cannot raise the dynamic LDS limit to %d bytes", LDS_B);
             return FL_ELAUNCH;
         }
-    const void* fns64[] = {(const void*)attn_prefill_r64_kernel<false>,
-                           (const void*)attn_prefill_r64_kernel<true>};
+    const void* fns64[] = {(const void*)attn_prefill_r64_kernel<R64_ROWS>,
+                           (const void*)attn_prefill_r64_kernel<R64_SPLIT>,
+                           (const void*)attn_prefill_r64_kernel<R64_PIECES>};
     for (const void* f : fns64)
         if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, R64_LDS) !=
             hipSuccess) {
@@ -1053,6 +1184,128 @@ int r64_plan(int T, int pos0, int G, int n_kv, int n_cu, R64Plan& plan) {
     return used;
 }
 
+// A piece list (STREAM) for T rows from pos0: the row tiles cut into at most
+// n_cu / n_kv runs a kv head of equal cost: a piece costs the KV tiles it walks +
+// R64_PIECE_COST (Q, pipeline fill, its 256 KiB partial). Short calls use fewer
+// runs than CUs rather than pieces shorter than R64_PIECE_MIN tiles. `cost` is
+// the longest run plus the merge's share, in KV tiles (~2 us each). Returns the entries of `plan` used, 0 where
+// the list does not apply (kv heads that do not divide the 8 XCDs, too many row
+// tiles or cache rows for its 16-bit entries).
+constexpr int R64_PIECE_COST = 8;
+constexpr int R64_PIECE_MIN = 6;
+constexpr int R64_MERGE_COST = 2;         // the merge's launch, in KV tiles
+constexpr int R64_SLOTS_PER_TILE = 40;    // partials the merge reads in a KV tile's time
+
+struct StreamPlan {
+    R64Plan plan;
+    int bins, slots, cost;
+};
+
+int r64_stream_plan(int T, int pos0, int G, int n_kv, int n_cu, StreamPlan& sp) {
+    if (T < 1 || pos0 < 0 || G < 1 || n_kv < 1 || 8 % n_kv != 0 || n_cu < 8 || n_cu % 8 != 0)
+        return 0;
+    const long long RT = (long long)T * G;
+    const long long N = (RT + R64_BQ - 1) / R64_BQ;
+    const int max_bins = n_cu / n_kv;
+    if (N + 1 + 3 * max_bins + 2 > R64_PLAN_MAX) return 0;
+    if (((long long)pos0 + T + R64_BK - 1) / R64_BK > 65535) return 0;
+    std::vector<int> nt(N);
+    long long walk = 0;
+    for (int t = 0; t < N; ++t) {
+        const int kv_end = pos0 + (int)(std::min<long long>((long long)t * R64_BQ + R64_BQ - 1, RT - 1) / G) + 1;
+        nt[t] = (kv_end + R64_BK - 1) / R64_BK;
+        walk += nt[t];
+    }
+    struct Start {
+        int tile, j;
+    };
+    std::vector<Start> start;
+    std::vector<int> pieces(N);
+    // The cut at run ends `end(b)` (in cost from the start) for at most `most`
+    // runs; returns the longest run's cost, 0 if they do not suffice (the last
+    // run never takes more than its end when `strict`).
+    auto cut = [&](int most, bool strict, auto end) -> long long {
+        start.clear();
+        std::fill(pieces.begin(), pieces.end(), 0);
+        long long used = 0, from = 0, longest = 0, stop = 0;
+        for (int t = 0; t < N; ++t) {
+            int left = nt[t], j = 0;
+            while (left > 0) {
+                const bool last = (int)start.size() == most;
+                // no room for a piece worth cutting: the next run
+                if (stop - used < R64_PIECE_COST + std::min(left, R64_PIECE_MIN) && (!last || strict)) {
+                    if (last) return 0;
+                    from = used;
+                    stop = end((int)start.size(), from);
+                    start.push_back({t, j});
+                    continue;
+                }
+                int take = left;
+                if (left + R64_PIECE_COST > stop - used && (!last || strict)) {
+                    take = (int)(stop - used - R64_PIECE_COST);
+                    // (no crumb left for the next run)
+                    if (left - take < R64_PIECE_MIN) take = std::max(1, left - R64_PIECE_MIN);
+                }
+                ++pieces[t];
+                j += take;
+                left -= take;
+                used += take + R64_PIECE_COST;
+                longest = std::max(longest, used - from);
+                if (left > 0) stop = used;   // the rest is the next run's
+            }
+        }
+        return longest;
+    };
+    // Runs of one capacity, the smallest that max_bins of them suffice for ...
+    const int min_run = R64_PIECE_COST + 2 * R64_PIECE_MIN;
+    auto fixed = [&](long long C) {
+        return cut(max_bins, true, [&](int, long long from) { return from + C; });
+    };
+    long long lo = min_run, hi = lo;
+    while (fixed(hi) == 0) hi *= 2;
+    while (lo < hi) {
+        const long long mid = lo + (hi - lo) / 2;
+        if (fixed(mid) > 0) hi = mid;
+        else lo = mid + 1;
+    }
+    long long longest = lo;
+    // ... or run b ending at (b + 1) / max_bins of the whole, where that is as
+    // short to 2 %: the fixed capacity's rounding adds up over the runs, and those
+    // that walk the same cache rows for different row tiles (every eighth one of a
+    // 1024-token chunk's) drift apart and out of each other's L2 lines.
+    const long long total = walk + (long long)R64_PIECE_COST * (N + max_bins - 1);
+    const long long even = cut(max_bins, false, [&](int b, long long from) {
+        return std::max(from + min_run, total * (b + 1) / max_bins);
+    });
+    if (even <= lo + lo / 50) longest = even;
+    else fixed(lo);
+    const int bins = (int)start.size();
+    std::vector<int> slot0(N + 1);
+    for (int t = 0; t < N; ++t) slot0[t + 1] = slot0[t] + pieces[t];
+    uint16_t* v = sp.plan.v;
+    int seen = 0, last_tile = -1;   // runs opened inside the current tile after its start
+    for (int b = 0; b < bins; ++b) {
+        const int t = start[b].tile;
+        seen = t == last_tile ? seen : 0;
+        last_tile = t;
+        if (start[b].j > 0) ++seen;
+        v[2 * b] = (uint16_t)t;
+        v[2 * b + 1] = (uint16_t)start[b].j;
+        v[2 * (bins + 1) + b] = (uint16_t)(slot0[t] + (start[b].j > 0 ? seen : 0));
+    }
+    v[2 * bins] = (uint16_t)N;
+    v[2 * bins + 1] = 0;
+    for (int t = 0; t <= N; ++t) v[3 * bins + 2 + t] = (uint16_t)slot0[t];
+    sp.bins = bins;
+    sp.slots = slot0[N];
+    sp.cost = (int)longest + R64_MERGE_COST + sp.slots * n_kv / R64_SLOTS_PER_TILE;
+    return 3 * bins + 2 + (int)N + 1;
+}
+
+size_t stream_work_bytes(const StreamPlan& sp, int n_kv) {
+    return (size_t)sp.slots * n_kv * R64_BQ * ((size_t)PF_HD * 4 + 8);
+}
+
 // The 64-rows-a-wave kernel takes a call once there are enough 256-row
 // workgroups to fill the chip twice over.
 bool use_r64(int T, int n_q_heads, int n_kv_heads) {
@@ -1115,6 +1368,138 @@ int split_policy(int T, int pos0, int n_q_heads, int n_kv_heads, bool q8 = false
     return best_split(wgs, (pos0 + T + PF_BK - 1) / PF_BK, PF_SPLIT_OVH);
 }
 
+// A launch of `wgs` workgroups, one a CU at a time, heaviest first, their
+// weights falling evenly from `heavy` to `light`: when the last one ends.
+int grid_makespan(int wgs, int cus, int heavy, int light) {
+    std::priority_queue<int, std::vector<int>, std::greater<int>> free_at;
+    for (int i = 0; i < cus; ++i) free_at.push(0);
+    int last = 0;
+    for (int i = 0; i < wgs; ++i) {
+        const int e = free_at.top() + heavy - (int)((long long)(heavy - light) * i / wgs);
+        free_at.pop();
+        free_at.push(e);
+        last = std::max(last, e);
+    }
+    return last;
+}
+
+// Whether a call that leaves its split to the library takes the piece list goes
+// by the costs of the two in KV tiles: the list against the persistent plan
+// (balanced to its heaviest row tile), the 128-row grid or its KV split (a
+// 64-row tile of 128 rows takes 1.1 times what a 32-row tile of 256 does, a
+// workgroup of the unsplit grid 9 more, its successor's start included), or
+// the 64-rows-a-wave kernel's uniform split. That one stays where it runs and the
+// K and V rows pass R64_LLC_ROWS a kv head's share of the last-level cache: its
+// row tiles walk each split's rows together, a list's runs walk as many places
+// as there are runs to a row tile, and past the cache that costs more than the
+// even runs save. Same box, gated, list against what ran without it: T = 1024
+// from 0 56 / 56 us, 1024 79 / 102, 3072 135 / 151, 8000 251 / 278, 30000 767 /
+// 795, 98000 2458 / 2366; T = 777 at 3072 104 / 134, 683 at 8000 185 / 235, 512 at
+// 98000 1284 / 1437, 2048 at 8000 487 / 603, 3000 at 30000 2328 / 3324, 16 at
+// 98000 132 / 236, 4096 from 0 286 / 273.
+constexpr long long R64_LLC_ROWS = 65536;   // x 4 kv heads x 1 KiB: 256 MiB
+constexpr int PF_UNIT_TENTHS = 11;
+constexpr int PF_UNIT_Q8_TENTHS = 15;   // the int8 128-row kernel
+constexpr int PF_WG_COST = 9;
+constexpr int Q8_STAGE_COST = 45;       // the staging launch, and its rows x kv heads a tenth
+constexpr int Q8_STAGE_ROWS = 640;
+
+// What a call costs without the list, in tenths of a KV tile of the
+// 64-rows-a-wave kernel, over an fp16 cache or (q8) the int8 128-row kernel.
+long long plain_cost(int T, int pos0, int n_q_heads, int n_kv_heads, int n_cu, bool q8) {
+    const int G = n_q_heads / n_kv_heads, rows = T * G;
+    const int heaviest64 = (pos0 + T + PF_BK - 1) / PF_BK;
+    const int unit = q8 ? PF_UNIT_Q8_TENTHS : PF_UNIT_TENTHS;
+    if (!q8 && use_r64(T, n_q_heads, n_kv_heads)) {
+        const int N = (rows + R64_BQ - 1) / R64_BQ;
+        long long total = 0;
+        int wmax = 0;
+        for (int t = 0; t < N; ++t) {
+            const int kv_end = pos0 + std::min(t * R64_BQ + R64_BQ - 1, rows - 1) / G + 1;
+            wmax = (kv_end + R64_BK - 1) / R64_BK + R64_ITEM_COST;
+            total += wmax;
+        }
+        const int bins = std::max(1, n_cu / n_kv_heads);
+        return 10 * std::max<long long>((total + bins - 1) / bins, wmax);
+    }
+    const int S = split_policy(T, pos0, n_q_heads, n_kv_heads, q8);
+    const int wgs = n_kv_heads * ((rows + PF_BQ - 1) / PF_BQ);
+    if (S == 1)
+        return (long long)unit * grid_makespan(wgs, n_cu, heaviest64 + PF_WG_COST,
+                                               pos0 / PF_BK + 1 + PF_WG_COST);
+    const long long merge =
+        10 * (R64_MERGE_COST + (long long)T * n_q_heads * S / R64_BQ / R64_SLOTS_PER_TILE);
+    if (!q8 && use_r64_split(T, pos0, n_q_heads, n_kv_heads)) {
+        const int wgs64 = n_kv_heads * ((rows + R64_BQ - 1) / R64_BQ);
+        const long long rounds = ((long long)wgs64 * S + n_cu - 1) / n_cu;
+        return 10 * rounds * ((2 * heaviest64 + S - 1) / S + R64_SPLIT_OVH) + merge;
+    }
+    const long long rounds = ((long long)wgs * S + n_cu - 1) / n_cu;
+    return unit * rounds * ((heaviest64 + S - 1) / S + R64_ITEM_COST) + merge;
+}
+
+// How a call that leaves its split to the library runs: over an fp16 cache by the
+// piece list or without it; over an int8 cache with the rows first copied to
+// fp16 (the staging copy, ~6 KiB a cache row at the copy rate) and the fp16
+// path on the copy, where that costs less than the int8 kernel, whose waves
+// dequantise each tile again for every 128 rows with their MFMAs idle. Same box,
+// gated, staged against the int8 kernel: T = 1024 from 0 59 / 71 us, 3072 133 /
+// 202, 30000 784 / 1139; T = 512 at 1024 54 / 64, 256 at 8000 90 / 106, 16 at
+// 30000 86 / 107; a short call over few rows stays (T = 16 at 3072: 33 staged, 26;
+// 64 at 1024: 32, 29), which Q8_STAGE_COST is set for.
+struct AutoChoice {
+    bool stage, stream;
+    StreamPlan sp;
+};
+
+void choose(int T, int pos0, int n_q_heads, int n_kv_heads, int n_cu, bool q8, AutoChoice& c) {
+    const int G = n_q_heads / n_kv_heads;
+    long long cost = plain_cost(T, pos0, n_q_heads, n_kv_heads, n_cu, false);
+    const bool together = split_policy(T, pos0, n_q_heads, n_kv_heads) > 1 &&
+                          use_r64_split(T, pos0, n_q_heads, n_kv_heads) &&
+                          (pos0 + (long long)T) * n_kv_heads > R64_LLC_ROWS * 4;
+    c.stage = false;
+    c.stream = !together && r64_stream_plan(T, pos0, G, n_kv_heads, n_cu, c.sp) > 0 &&
+               10 * (long long)c.sp.cost < cost;
+    if (!q8) return;
+    if (c.stream) cost = 10 * (long long)c.sp.cost;
+    cost += Q8_STAGE_COST + (pos0 + (long long)T) * n_kv_heads / Q8_STAGE_ROWS;
+    c.stage = cost < plain_cost(T, pos0, n_q_heads, n_kv_heads, n_cu, true);
+    c.stream = c.stream && c.stage;
+}
+
+// That choice, kept for the last few shapes (a prompt's chunk asks the same of
+// every layer); copied out under the lock.
+struct AutoEntry {
+    int T, pos0, nq, nkv, n_cu;
+    bool q8;
+    AutoChoice c;
+};
+constexpr int AUTO_CACHE = 8;
+std::mutex g_auto_mu;
+AutoEntry g_auto_cache[AUTO_CACHE];
+int g_auto_fill, g_auto_next;
+
+void auto_choice(int T, int pos0, int n_q_heads, int n_kv_heads, int n_cu, bool q8,
+                 AutoChoice& c) {
+    {
+        std::lock_guard<std::mutex> lock(g_auto_mu);
+        for (int i = 0; i < g_auto_fill; ++i) {
+            const AutoEntry& e = g_auto_cache[i];
+            if (e.T == T && e.pos0 == pos0 && e.nq == n_q_heads && e.nkv == n_kv_heads &&
+                e.n_cu == n_cu && e.q8 == q8) {
+                c = e.c;
+                return;
+            }
+        }
+    }
+    choose(T, pos0, n_q_heads, n_kv_heads, n_cu, q8, c);
+    std::lock_guard<std::mutex> lock(g_auto_mu);
+    g_auto_cache[g_auto_next] = {T, pos0, n_q_heads, n_kv_heads, n_cu, q8, c};
+    g_auto_next = (g_auto_next + 1) % AUTO_CACHE;
+    g_auto_fill = std::min(g_auto_fill + 1, AUTO_CACHE);
+}
+
 // The int8 cache's rows [0, rows) as fp16(byte * scale), the values the int8
 // kernel builds in LDS, into a staging copy [rows][n_kv][256] of K then V:
 // thread i converts 16-byte chunk i of a K row and of a V row (16 values of
@@ -1150,6 +1535,18 @@ size_t split_work_bytes(int T, int n_q_heads, int head_dim, int split) {
     return (size_t)T * n_q_heads * split * ((size_t)head_dim * 4 + 8);
 }
 
+// the fp16 copy of an int8 cache's rows [0, pos0 + T), K then V
+size_t q8_copy_bytes(int T, int pos0, int n_kv_heads) {
+    return 2 * (size_t)(pos0 + T) * n_kv_heads * PF_HD * sizeof(f16);
+}
+
+// the work of an fp16 call that leaves its split to the library
+size_t auto_f16_bytes(int T, int pos0, int n_q_heads, int n_kv_heads, const AutoChoice& c) {
+    if (c.stream) return stream_work_bytes(c.sp, n_kv_heads);
+    const int S = split_policy(T, pos0, n_q_heads, n_kv_heads);
+    return S > 1 ? split_work_bytes(T, n_q_heads, PF_HD, S) : 0;
+}
+
 // gated: z *= sigmoid(gate) after the attention (attn_gate), the gate being
 // the second half of each head's q row (q | gate rows, q_pitch >= 2 head_dim):
 // applied by the merge when the KV is split, else by fl_attn_gate after it.
@@ -1157,13 +1554,13 @@ template <bool Q8>
 int prefill(const void* q, int q_pitch, const void* k_new, const void* v_new, void* kcache,
             void* vcache, int layer, int n_q_heads, int n_kv_heads, int head_dim, int pos0,
             int max_pos, float scale, int T, void* z, int z_pitch, int split, void* work,
-            size_t work_bytes, fl_stream_t stream, bool gated = false) {
+            size_t work_bytes, fl_stream_t stream_, bool gated = false) {
     FL_REQUIRE(q && kcache && vcache && z, "null pointer");
     FL_REQUIRE(!gated || q_pitch >= 2 * head_dim, "gated: q_pitch >= 2 head_dim (q | gate rows)");
     const void* gate = gated ? q : nullptr;
     auto gate_after = [&](int rc_) {
         if (rc_ || !gated) return rc_;
-        return fl_attn_gate(z, q, n_q_heads, head_dim, z_pitch, q_pitch, head_dim, T, stream);
+        return fl_attn_gate(z, q, n_q_heads, head_dim, z_pitch, q_pitch, head_dim, T, stream_);
     };
     FL_REQUIRE(head_dim == PF_HD, "head_dim must be 256");
     FL_REQUIRE(n_kv_heads > 0 && n_q_heads > 0 && n_q_heads % n_kv_heads == 0,
@@ -1175,8 +1572,25 @@ int prefill(const void* q, int q_pitch, const void* k_new, const void* v_new, vo
     FL_REQUIRE((k_new == nullptr) == (v_new == nullptr), "k_new and v_new together");
     FL_REQUIRE(aligned16(q) && aligned16(kcache) && aligned16(vcache) && ((uintptr_t)z & 7u) == 0,
                "aligned buffers");
-    FL_REQUIRE(split >= 1 && split <= 1024, "1 <= split <= 1024");
-    if (split > 1) {
+    FL_REQUIRE(split >= 0 && split <= 1024, "0 <= split <= 1024");
+    int n_cu = 0;
+    int rc = prefill_device_setup(n_cu);
+    if (rc) return rc;
+    // the library's own choice (split 0, or the count it gives out): a piece list
+    // where that is cheaper and its partials fit in `work`
+    const int policy = split_policy(T, pos0, n_q_heads, n_kv_heads, Q8);
+    AutoChoice c;
+    c.stage = c.stream = false;
+    if (split == 0 || (split > 1 && split == policy))
+        auto_choice(T, pos0, n_q_heads, n_kv_heads, n_cu, Q8, c);
+    const StreamPlan& sp_plan = c.sp;
+    const size_t copy = c.stage ? q8_copy_bytes(T, pos0, n_kv_heads) : 0;
+    const bool staged_auto = c.stage && work != nullptr && aligned16(work) &&
+                             work_bytes >= copy + auto_f16_bytes(T, pos0, n_q_heads, n_kv_heads, c);
+    const bool stream = !Q8 && c.stream && work != nullptr && aligned16(work) &&
+                        work_bytes >= stream_work_bytes(sp_plan, n_kv_heads);
+    if (split == 0) split = policy;
+    if (split > 1 && !stream && !staged_auto) {
         FL_REQUIRE(work != nullptr && aligned16(work), "16-byte aligned work for a split");
         if (work_bytes < split_work_bytes(T, n_q_heads, head_dim, split)) {
             fl::set_error("work: %zu bytes, fl_attention_prefill_work_bytes asks %zu", work_bytes,
@@ -1185,15 +1599,12 @@ int prefill(const void* q, int q_pitch, const void* k_new, const void* v_new, vo
         }
     }
     if (k_new != nullptr) {
-        const int rc = Q8 ? fl_kv_store_q8(k_new, v_new, kcache, vcache, layer, pos0, T,
-                                           n_kv_heads, head_dim, max_pos, stream)
-                          : fl_kv_store(k_new, v_new, kcache, vcache, layer, pos0, T, n_kv_heads,
-                                        head_dim, max_pos, stream);
+        rc = Q8 ? fl_kv_store_q8(k_new, v_new, kcache, vcache, layer, pos0, T,
+                                 n_kv_heads, head_dim, max_pos, stream_)
+                : fl_kv_store(k_new, v_new, kcache, vcache, layer, pos0, T, n_kv_heads, head_dim,
+                              max_pos, stream_);
         if (rc) return rc;
     }
-    int n_cu = 0;
-    int rc = prefill_device_setup(n_cu);
-    if (rc) return rc;
     const void* kc;
     const void* vc;
     const f16* ksc = nullptr;
@@ -1212,55 +1623,79 @@ int prefill(const void* q, int q_pitch, const void* k_new, const void* v_new, vo
     const int rows = T * (n_q_heads / n_kv_heads);
     const int r64_tiles = (rows + R64_BQ - 1) / R64_BQ;
     // over an int8 cache with room in `work` for the fp16 staging copy: stage,
-    // then the fp16 path below on the copy
+    // then the fp16 path on the copy
     const size_t stage = Q8 && split == 1 ? q8_stage_bytes(T, pos0, n_q_heads, n_kv_heads, head_dim)
                                           : 0;
-    const bool staged = stage > 0 && work != nullptr && aligned16(work) && work_bytes >= stage;
+    const bool staged =
+        staged_auto || (stage > 0 && work != nullptr && aligned16(work) && work_bytes >= stage);
     if (staged) {
         const size_t cache_rows = (size_t)(pos0 + T) * n_kv_heads;
         const int n_chunks = (int)(cache_rows * (PF_HD / 16));
         f16* ko = (f16*)work;
         f16* vo = ko + cache_rows * PF_HD;
         hipLaunchKernelGGL(q8_stage_kernel, dim3((n_chunks + 255) / 256), dim3(256), 0,
-                           (hipStream_t)stream, (const uint4*)kc, (const uint4*)vc, ksc, vsc,
+                           (hipStream_t)stream_, (const uint4*)kc, (const uint4*)vc, ksc, vsc,
                            (f16x8*)ko, (f16x8*)vo, n_chunks);
         rc = fl::check_launch("attn_prefill q8 staging");
         if (rc) return rc;
-        kc = ko;
-        vc = vo;
+        if constexpr (Q8) {
+            const size_t used = q8_copy_bytes(T, pos0, n_kv_heads);
+            return prefill<false>(q, q_pitch, nullptr, nullptr, ko, vo, 0, n_q_heads, n_kv_heads,
+                                  head_dim, pos0, pos0 + T, scale, T, z, z_pitch,
+                                  staged_auto ? 0 : 1, (char*)work + used, work_bytes - used,
+                                  stream_, gated);
+        }
     }
-    if ((!Q8 || staged) && split == 1 && use_r64(T, n_q_heads, n_kv_heads)) {
+    if (stream) {
+        const size_t rows256 = (size_t)sp_plan.slots * n_kv_heads * R64_BQ;
+        StreamOut so = {(float*)work, nullptr, nullptr, sp_plan.slots};
+        so.pm = so.pacc + rows256 * PF_HD;
+        so.pd = so.pm + rows256;
+        hipLaunchKernelGGL(attn_prefill_r64_kernel<R64_PIECES>, dim3(n_cu), dim3(PF_THREADS), R64_LDS,
+                           (hipStream_t)stream_, (const f16*)q, q_pitch, (const f16*)kc,
+                           (const f16*)vc, (f16*)z, z_pitch, n_q_heads, n_kv_heads, pos0, T,
+                           scale * FL_LOG2E, r64_tiles, sp_plan.bins, sp_plan.plan, so);
+        rc = fl::check_launch("attn_prefill_r64 (pieces)");
+        if (rc) return rc;
+        const int n_pairs = T * n_q_heads;
+        hipLaunchKernelGGL(attn_prefill_stream_merge_kernel,
+                           dim3((n_pairs + SM_PAIRS - 1) / SM_PAIRS), dim3(64 * SM_PAIRS), 0,
+                           (hipStream_t)stream_, so, (f16*)z, z_pitch, (const f16*)gate, q_pitch,
+                           n_q_heads, n_q_heads / n_kv_heads, sp_plan.bins, n_pairs, sp_plan.plan);
+        return fl::check_launch("attn_prefill merge (pieces)");
+    }
+    if (!Q8 && split == 1 && use_r64(T, n_q_heads, n_kv_heads)) {
         R64Plan plan;
         const int G = n_q_heads / n_kv_heads;
         const int bins = r64_plan(T, pos0, G, n_kv_heads, n_cu, plan) > 0 ? n_cu / n_kv_heads : 0;
         const dim3 grid = bins > 0 ? dim3(n_cu) : dim3(r64_tiles, n_kv_heads);
-        hipLaunchKernelGGL(attn_prefill_r64_kernel<false>, grid, dim3(PF_THREADS), R64_LDS,
-                           (hipStream_t)stream, (const f16*)q, q_pitch, (const f16*)kc,
+        hipLaunchKernelGGL(attn_prefill_r64_kernel<R64_ROWS>, grid, dim3(PF_THREADS), R64_LDS,
+                           (hipStream_t)stream_, (const f16*)q, q_pitch, (const f16*)kc,
                            (const f16*)vc, (f16*)z, z_pitch, n_q_heads, n_kv_heads, pos0, T,
                            scale * FL_LOG2E, r64_tiles, bins, plan,
-                           PfSplit{nullptr, nullptr, nullptr, 1});
+                           StreamOut{nullptr, nullptr, nullptr, 0});
         return gate_after(fl::check_launch("attn_prefill_r64"));
     }
     if (!Q8 && split > 1 && use_r64_split(T, pos0, n_q_heads, n_kv_heads)) {
         const size_t parts = (size_t)T * n_q_heads * split;
-        PfSplit sp = {(float*)work, nullptr, nullptr, split};
-        sp.pm = sp.pacc + parts * PF_HD;
-        sp.pd = sp.pm + parts;
+        StreamOut so = {(float*)work, nullptr, nullptr, split};
+        so.pm = so.pacc + parts * PF_HD;
+        so.pd = so.pm + parts;
         R64Plan plan;
         plan.v[0] = 0;
-        hipLaunchKernelGGL(attn_prefill_r64_kernel<true>, dim3(r64_tiles, n_kv_heads, split),
-                           dim3(PF_THREADS), R64_LDS, (hipStream_t)stream, (const f16*)q, q_pitch,
+        hipLaunchKernelGGL(attn_prefill_r64_kernel<R64_SPLIT>, dim3(r64_tiles, n_kv_heads, split),
+                           dim3(PF_THREADS), R64_LDS, (hipStream_t)stream_, (const f16*)q, q_pitch,
                            (const f16*)kc, (const f16*)vc, (f16*)z, z_pitch, n_q_heads,
-                           n_kv_heads, pos0, T, scale * FL_LOG2E, r64_tiles, 0, plan, sp);
+                           n_kv_heads, pos0, T, scale * FL_LOG2E, r64_tiles, 0, plan, so);
         rc = fl::check_launch("attn_prefill_r64 (kv split)");
         if (rc) return rc;
-        return fl_attention_merge(sp.pacc, sp.pm, sp.pd, z, n_q_heads, head_dim, z_pitch, T,
-                                  split, gate, q_pitch, head_dim, stream);
+        return fl_attention_merge(so.pacc, so.pm, so.pd, z, n_q_heads, head_dim, z_pitch, T,
+                                  split, gate, q_pitch, head_dim, stream_);
     }
     const int n_row_tiles = (rows + PF_BQ - 1) / PF_BQ;
     if (split == 1) {
         hipLaunchKernelGGL((attn_prefill_kernel<Q8, false>), dim3(n_row_tiles, n_kv_heads),
-                           dim3(PF_THREADS), LDS_B, (hipStream_t)stream, (const f16*)q, q_pitch,
+                           dim3(PF_THREADS), LDS_B, (hipStream_t)stream_, (const f16*)q, q_pitch,
                            kc, vc, ksc, vsc, (f16*)z, z_pitch, n_q_heads, n_kv_heads, pos0, T,
                            scale * FL_LOG2E, n_row_tiles, PfSplit{nullptr, nullptr, nullptr, 1});
         return gate_after(fl::check_launch("attn_prefill"));
@@ -1270,13 +1705,13 @@ int prefill(const void* q, int q_pitch, const void* k_new, const void* v_new, vo
     sp.pm = sp.pacc + parts * PF_HD;
     sp.pd = sp.pm + parts;
     hipLaunchKernelGGL((attn_prefill_kernel<Q8, true>), dim3(n_row_tiles, n_kv_heads, split),
-                       dim3(PF_THREADS), LDS_B, (hipStream_t)stream, (const f16*)q, q_pitch, kc,
+                       dim3(PF_THREADS), LDS_B, (hipStream_t)stream_, (const f16*)q, q_pitch, kc,
                        vc, ksc, vsc, (f16*)z, z_pitch, n_q_heads, n_kv_heads, pos0, T,
                        scale * FL_LOG2E, n_row_tiles, sp);
     rc = fl::check_launch("attn_prefill (kv split)");
     if (rc) return rc;
     return fl_attention_merge(sp.pacc, sp.pm, sp.pd, z, n_q_heads, head_dim, z_pitch, T, split,
-                              gate, q_pitch, head_dim, stream);
+                              gate, q_pitch, head_dim, stream_);
 }
 
 }  // namespace
@@ -1312,6 +1747,19 @@ extern "C" int fl_attention_prefill_plan(int T, int pos0, int n_q_heads, int n_k
     return used;
 }
 
+extern "C" int fl_attention_prefill_pieces(int T, int pos0, int n_q_heads, int n_kv_heads, int n_cu,
+                                           unsigned short* out, int cap, int* bins, int* slots) {
+    if (n_kv_heads < 1 || n_q_heads < 1 || n_q_heads % n_kv_heads != 0) return 0;
+    StreamPlan sp;
+    const int used = r64_stream_plan(T, pos0, n_q_heads / n_kv_heads, n_kv_heads, n_cu, sp);
+    if (used == 0) return 0;
+    if (bins != nullptr) *bins = sp.bins;
+    if (slots != nullptr) *slots = sp.slots;
+    if (out != nullptr)
+        for (int i = 0; i < used && i < cap; ++i) out[i] = sp.plan.v[i];
+    return used;
+}
+
 extern "C" int fl_attention_prefill_split_count(int T, int pos0, int n_q_heads, int n_kv_heads) {
     return split_policy(T, pos0, n_q_heads, n_kv_heads);
 }
@@ -1326,6 +1774,24 @@ extern "C" size_t fl_attention_prefill_q8_stage_bytes(int T, int pos0, int n_q_h
     return q8_stage_bytes(T, pos0, n_q_heads, n_kv_heads, head_dim);
 }
 
+extern "C" size_t fl_attention_prefill_auto_work_bytes(int T, int pos0, int n_q_heads,
+                                                       int n_kv_heads, int head_dim, int q8) {
+    if (T < 1 || pos0 < 0 || n_kv_heads < 1 || n_q_heads < 1 || n_q_heads % n_kv_heads != 0 ||
+        head_dim != PF_HD)
+        return 0;
+    int n_cu = PF_CUS;
+    if (prefill_device_setup(n_cu) != FL_OK) n_cu = PF_CUS;   // no device: an MI355X's count
+    AutoChoice c;
+    auto_choice(T, pos0, n_q_heads, n_kv_heads, n_cu, q8 != 0, c);
+    if (!q8) return auto_f16_bytes(T, pos0, n_q_heads, n_kv_heads, c);
+    if (c.stage)
+        return q8_copy_bytes(T, pos0, n_kv_heads) +
+               auto_f16_bytes(T, pos0, n_q_heads, n_kv_heads, c);
+    const int S = split_policy(T, pos0, n_q_heads, n_kv_heads, q8 != 0);
+    if (S > 1) return split_work_bytes(T, n_q_heads, head_dim, S);
+    return q8 ? q8_stage_bytes(T, pos0, n_q_heads, n_kv_heads, head_dim) : 0;
+}
+
 extern "C" size_t fl_attention_prefill_work_bytes(int T, int n_q_heads, int head_dim, int split) {
     if (T < 1 || n_q_heads < 1 || head_dim < 1 || split < 1) return 0;
     return split > 1 ? split_work_bytes(T, n_q_heads, head_dim, split) : 0;
@@ -1337,7 +1803,6 @@ extern "C" int fl_attention_prefill_kv(const void* q, int q_pitch, const void* k
                                        int max_pos, float scale, int T, int split, void* z,
                                        int z_pitch, void* work, size_t work_bytes,
                                        fl_stream_t stream) {
-    if (split == 0) split = split_policy(T, pos0, n_q_heads, n_kv_heads);
     return prefill<false>(q, q_pitch, k_new, v_new, kcache, vcache, layer, n_q_heads, n_kv_heads,
                           head_dim, pos0, max_pos, scale, T, z, z_pitch, split, work, work_bytes,
                           stream);
@@ -1349,7 +1814,6 @@ extern "C" int fl_attention_prefill_gated(const void* q, int q_pitch, const void
                                           int head_dim, int pos0, int max_pos, float scale, int T,
                                           int split, void* z, int z_pitch, void* work,
                                           size_t work_bytes, fl_stream_t stream) {
-    if (split == 0) split = split_policy(T, pos0, n_q_heads, n_kv_heads, q8 != 0);
     if (q8)
         return prefill<true>(q, q_pitch, k_new, v_new, kcache, vcache, layer, n_q_heads,
                              n_kv_heads, head_dim, pos0, max_pos, scale, T, z, z_pitch, split, work,
@@ -1365,7 +1829,6 @@ extern "C" int fl_attention_prefill_kv_q8(const void* q, int q_pitch, const void
                                           int pos0, int max_pos, float scale, int T, int split,
                                           void* z, int z_pitch, void* work, size_t work_bytes,
                                           fl_stream_t stream) {
-    if (split == 0) split = split_policy(T, pos0, n_q_heads, n_kv_heads, true);
     return prefill<true>(q, q_pitch, k_new, v_new, kcache, vcache, layer, n_q_heads, n_kv_heads,
                          head_dim, pos0, max_pos, scale, T, z, z_pitch, split, work, work_bytes,
                          stream);

@@ -235,8 +235,8 @@ def attention_prefill(q, kcache, vcache, *, pos0: int, T: int | None = None, z=N
     _attn_fh runtime.py:2943-2959), with kv_store (kernels.cu:465-484) of
     k_new / v_new [T, n_kv, head_dim] fused in front when given. q [T,
     n_q_heads, q_pitch] fp16 (q first in a head's row). split: the KV split
-    (None: prefill_split_count's choice; a split > 1 leaves partials in `work`,
-    a uint8 tensor, allocated here unless given). gated: attn_gate applied too
+    (None: the library's choice; a split > 1 leaves partials in `work`, a
+    uint8 tensor, allocated here unless given). gated: attn_gate applied too
     (kernels.cu:1585-1600, runtime.py:2860-2862), the gate the second half of
     each head's q row -- in the merge when the KV is split. Returns z [T,
     n_q_heads, head_dim] fp16."""
@@ -259,17 +259,15 @@ def attention_prefill(q, kcache, vcache, *, pos0: int, T: int | None = None, z=N
     elif split == 1:
         _lib.call("fl_attention_prefill", *args, *zargs, _stream())
     else:
-        _lib.call("fl_attention_prefill_kv", *args, split, *zargs,
-                  _ptr(work, torch.uint8, "work", work.numel()), work.numel(), _stream())
+        _lib.call("fl_attention_prefill_kv", *args, split, *zargs, *_prefill_work(work), _stream())
     return z
 
 
 def _prefill_gated(args, q8: int, split: int, zargs, work):
     """fl_attention_prefill_gated over the (q .. T) arguments of the ungated
     entry points (layer is args[6]; the cache flag goes after it)."""
-    wp = _ptr(work, torch.uint8, "work", work.numel()) if work is not None else None
-    _lib.call("fl_attention_prefill_gated", *args[:7], q8, *args[7:], split, *zargs, wp,
-              work.numel() if work is not None else 0, _stream())
+    _lib.call("fl_attention_prefill_gated", *args[:7], q8, *args[7:], split, *zargs,
+              *_prefill_work(work), _stream())
 
 
 def prefill_split_count(T: int, pos0: int, n_q_heads: int = N_HEADS,
@@ -290,13 +288,23 @@ def prefill_split_count_q8(T: int, pos0: int, n_q_heads: int = N_HEADS,
 
 
 def _prefill_split(T, pos0, n_q_heads, n_kv_heads, head_dim, split, work, device, q8=False):
+    """(split, work) of a prefill call: a split left to the library goes down as 0,
+    with the work its choice needs where none is given."""
     if split is None:
-        split = (prefill_split_count_q8 if q8 else prefill_split_count)(T, pos0, n_q_heads,
-                                                                          n_kv_heads)
-    if split > 1 and work is None:
+        split = 0
+        if work is None:
+            need = int(_lib.lib().fl_attention_prefill_auto_work_bytes(
+                T, pos0, n_q_heads, n_kv_heads, head_dim, int(q8)))
+            work = torch.empty(need, dtype=torch.uint8, device=device) if need else None
+    elif split > 1 and work is None:
         need = int(_lib.lib().fl_attention_prefill_work_bytes(T, n_q_heads, head_dim, split))
         work = torch.empty(need, dtype=torch.uint8, device=device)
     return split, work
+
+
+def _prefill_work(work):
+    return (None, 0) if work is None else (_ptr(work, torch.uint8, "work", work.numel()),
+                                           work.numel())
 
 
 # ---------------------------------------------------------------------------
@@ -468,21 +476,18 @@ def attention_prefill_q8(q, kcache, vcache, *, pos0: int, max_pos: int, T: int |
             HEAD_DIM, pos0, max_pos, float(scale), T)
     zargs = (_ptr(z, F16, "z", T * n_q_heads * z.shape[-1]), z.shape[-1])
     stage = 0
-    if split == 1:
+    if split <= 1:
         stage = int(_lib.lib().fl_attention_prefill_q8_stage_bytes(T, pos0, n_q_heads, n_kv_heads,
                                                                    HEAD_DIM))
-    if split == 1 and stage > 0 and (work is None or work.numel() < stage):
+    if stage > 0 and (work is None or work.numel() < stage):
         work = torch.empty(stage, dtype=torch.uint8, device=q.device)
     if gated:
         _prefill_gated(args, 1, split, zargs, work)
-    elif split == 1 and stage > 0:
-        _lib.call("fl_attention_prefill_kv_q8", *args, 1, *zargs,
-                  _ptr(work, torch.uint8, "work", stage), work.numel(), _stream())
-    elif split == 1:
+    elif split == 1 and stage == 0:
         _lib.call("fl_attention_prefill_q8", *args, *zargs, _stream())
     else:
-        _lib.call("fl_attention_prefill_kv_q8", *args, split, *zargs,
-                  _ptr(work, torch.uint8, "work", work.numel()), work.numel(), _stream())
+        _lib.call("fl_attention_prefill_kv_q8", *args, split, *zargs, *_prefill_work(work),
+                  _stream())
     return z
 
 

@@ -278,7 +278,8 @@ size_t fl_attn_decode_noalloc_max_bytes(void);
  * (runtime.py:196): the 64-rows-a-wave kernel splits from 64 workgroups of
  * 256 rows and 16384 cache rows (fp16 caches), the 128-row kernel otherwise
  * and over int8 caches.
- * split 0: fl_attention_prefill_split_count's choice; split 1:
+ * split 0: the library's choice (fl_attention_prefill_auto_work_bytes below, or
+ * fl_attention_prefill_split_count's with less work); split 1:
  * fl_attention_prefill (no work needed). */
 int fl_attention_prefill_split_count(int T, int pos0, int n_q_heads, int n_kv_heads);
 /* The same choice for an int8 cache (_fh_split's role for
@@ -286,6 +287,21 @@ int fl_attention_prefill_split_count(int T, int pos0, int n_q_heads, int n_kv_he
  * kernel's split, what fl_attention_prefill_kv_q8 takes for split 0. */
 int fl_attention_prefill_split_count_q8(int T, int pos0, int n_q_heads, int n_kv_heads);
 size_t fl_attention_prefill_work_bytes(int T, int n_q_heads, int head_dim, int split);
+/* The `work` bytes of a call that leaves its split to the library (split 0):
+ * beside a uniform split, the row tiles' causal walks cut into equal runs, one
+ * a CU, whose cut tiles leave partials that one merge combines (gate included).
+ * A split 0 call, or one with the count that fl_attention_prefill_split_count
+ * gives, takes that where it is cheaper and `work` holds these bytes, else the
+ * uniform split (or none). q8: over an int8 cache. 0: no work needed. */
+size_t fl_attention_prefill_auto_work_bytes(int T, int pos0, int n_q_heads, int n_kv_heads,
+                                            int head_dim, int q8);
+/* That cut for n_cu CUs, for tests and tuning (as fl_attention_prefill_plan):
+ * out[0 .. 2 bins + 1] = (row tile of 256 rows, first tile of 32 cache rows) of
+ * each run's start and of the end, then each run's first partial slot [bins],
+ * then each row tile's first slot [row tiles + 1]. Returns the entries (at most
+ * `cap` written), 0 where a call has no such cut. */
+int fl_attention_prefill_pieces(int T, int pos0, int n_q_heads, int n_kv_heads, int n_cu,
+                                unsigned short* out, int cap, int* bins, int* slots);
 int fl_attention_prefill_kv(const void* q, int q_pitch, const void* k_new, const void* v_new,
                             void* kcache, void* vcache, int layer, int n_q_heads, int n_kv_heads,
                             int head_dim, int pos0, int max_pos, float scale, int T, int split,
@@ -295,7 +311,9 @@ int fl_attention_prefill_kv(const void* q, int q_pitch, const void* k_new, const
  * With split 1 and `work` of at least fl_attention_prefill_q8_stage_bytes
  * bytes (nonzero for long prompts), the rows [0, pos0 + T) are first
  * converted to fp16 (byte * scale, the values the int8 kernel forms) into
- * `work`, and the long-prompt fp16 kernel runs on that copy. */
+ * `work`, and the long-prompt fp16 kernel runs on that copy. So they are for a
+ * split 0 call with fl_attention_prefill_auto_work_bytes of work where the copy
+ * and the fp16 path cost less than the int8 kernel. */
 size_t fl_attention_prefill_q8_stage_bytes(int T, int pos0, int n_q_heads, int n_kv_heads,
                                            int head_dim);
 int fl_attention_prefill_kv_q8(const void* q, int q_pitch, const void* k_new, const void* v_new,

@@ -229,6 +229,55 @@ def test_prefill_persistent_plan(fl, T, pos0):
     assert max(loads) <= 1.04 * bound, (max(loads), bound)
 
 
+@pytest.mark.parametrize("n_q,n_kv,n_cu", [(24, 4, 256), (8, 1, 256), (16, 8, 64), (24, 2, 304)])
+def test_prefill_pieces_cover_every_walk(fl, n_q, n_kv, n_cu):
+    """The equal runs of a prefill call: every KV tile of every row tile in
+    exactly one piece, the slots one a piece in KV order as the kernel counts
+    them (a run's first piece's given, a later piece's its row tile's first), no
+    more runs than workgroups a kv head, and the longest run within a piece of
+    the mean where there are enough tiles for all."""
+    lib = fl._lib.lib()
+    G, most = n_q // n_kv, n_cu // n_kv
+    buf = (ctypes.c_ushort * 1024)()
+    bins, slots = ctypes.c_int(), ctypes.c_int()
+    shapes = [(1, 0), (5, 0), (33, 0), (43, 0), (64, 63), (100, 9000), (777, 3001), (1000, 0),
+              (1024, 98000), (2048, 0), (4096, 0), (8192, 0), (5000, 27000), (17, 1000000)]
+    for T, pos0 in shapes:
+        n = lib.fl_attention_prefill_pieces(T, pos0, n_q, n_kv, n_cu, buf, 1024, bins, slots)
+        rows = T * G
+        N = -(-rows // 256)
+        if N + 1 + 3 * most + 2 > 1024:
+            assert n == 0, (T, pos0)
+            continue
+        B = bins.value
+        assert n == 3 * B + 2 + N + 1 <= 1024 and 1 <= B <= most, (T, pos0)
+        v = list(buf[:n])
+        walk = [-(-(pos0 + min(256 * t + 255, rows - 1) // G + 1) // 32) for t in range(N)]
+        at, seen, runs = (0, 0), {}, []
+        slot0 = v[3 * B + 2:]
+        for b in range(B):
+            tile, j, end, j_end = v[2 * b:2 * b + 4]
+            assert (tile, j) == at, (T, pos0, b)
+            n_items = end - tile + (1 if j_end else 0)
+            assert n_items >= 1
+            run = 0
+            for it in range(n_items):
+                t, lo = tile + it, j if it == 0 else 0
+                hi = j_end if it == n_items - 1 and j_end else walk[t]
+                assert 0 <= lo < hi <= walk[t], (T, pos0, b, t)
+                slot = v[2 * (B + 1) + b] if it == 0 else slot0[t]
+                assert slot == slot0[t] + seen.get(t, 0), (T, pos0, b, t)
+                seen[t] = seen.get(t, 0) + 1
+                run += hi - lo
+            runs.append(run)
+            at = (end, j_end)
+        assert at == (N, 0) and sum(runs) == sum(walk)
+        assert slot0[0] == 0 and all(slot0[t + 1] - slot0[t] == seen[t] for t in range(N))
+        assert slots.value == slot0[N]
+        if B == most:
+            assert max(runs) <= sum(walk) / B + 8 * (1 + N / B) + 8, (T, pos0, max(runs))
+
+
 def test_prefill_plan_falls_back_to_the_tile_grid(fl):
     """No plan (a grid of row tiles x kv heads) where the kernel does not run
     (short prompts, the KV-split chunk), where the row tiles do not outnumber

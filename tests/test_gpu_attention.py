@@ -445,6 +445,57 @@ def test_prefill_r64_kv_split_vs_fp32(fl, dev, T, pos0, split):
         assert float(err.max()) <= 1e-2 * float(want.float().abs().max()), name
 
 
+# calls left to the library that take the equal runs: a ragged last row tile,
+# runs that start mid-tile, one row tile over 64 runs (16 tokens at 30000: the
+# merge's batches of eight), more row tiles than runs (3000 tokens); over an int8
+# cache with its rows staged first
+@pytest.mark.parametrize("kv8,T,pos0", [
+    (False, 777, 3001), (False, 683, 1024), (False, 512, 3072), (False, 1500, 1025),
+    (False, 16, 30000), (False, 3000, 1000), (True, 1000, 0), (True, 1000, 1024), (True, 300, 8001)])
+def test_prefill_left_to_the_library_vs_fp32(fl, dev, kv8, T, pos0):
+    """Every row against oracle/torch_ref.attention_prefill (fp32 on the GPU) and
+    the unsplit call at the attention bar, gated equal to ungated then attn_gate
+    bit for bit, and too small a work buffer for any split refused."""
+    from oracle import torch_ref as tr
+
+    L = pos0 + T
+    g = torch.Generator(device=dev).manual_seed(T + pos0)
+    qg = torch.randn((T, 24, 512), generator=g, device=dev)
+    qg[..., :256] /= 16
+    qg = qg.half()
+    kd = torch.randn((L, 4, 256), generator=g, device=dev).half()
+    vd = torch.randn((L, 4, 256), generator=g, device=dev).half()
+    need = int(fl._lib.lib().fl_attention_prefill_auto_work_bytes(T, pos0, 24, 4, 256, int(kv8)))
+    assert need > 0
+    if kv8:
+        k8, v8 = fl.ops.kv8_cache(L), fl.ops.kv8_cache(L)
+        fl.ops.kv_store_q8(kd, vd, k8, v8, pos0=0, max_pos=L)
+        n = L * 4 * 256
+        kd, vd = ((c[:n].view(-1, 32).float() * c[n:].view(torch.float16).float()[:, None])
+                  .half().view(L, 4, 256) for c in (k8, v8))
+
+    def call(**kw):
+        if kv8:
+            return fl.ops.attention_prefill_q8(qg, k8, v8, pos0=pos0, max_pos=L, scale=1.0, **kw)
+        return fl.ops.attention_prefill(qg, kd, vd, pos0=pos0, scale=1.0, **kw)
+
+    z, z1, zg = call(), call(split=1), call(gated=True)
+    want = tr.attention_prefill(qg[..., :256].contiguous(), kd, vd, pos0, 1.0, block=256)
+    torch.cuda.synchronize()
+    for name, got in (("library's split", z), ("split 1", z1)):
+        err = (got.float() - want.float()).abs()
+        bad = int((err > ATOL + RTOL * want.float().abs()).sum())
+        assert torch.isfinite(got.float()).all() and bad == 0, (name, float(err.max()))
+        assert float(err.max()) <= 1e-2 * float(want.float().abs().max()), name
+    fl.ops.attn_gate(z, qg, T=T)
+    torch.cuda.synchronize()
+    assert torch.equal(zg, z)
+    count = (fl.ops.prefill_split_count_q8 if kv8 else fl.ops.prefill_split_count)(T, pos0)
+    if count > 1:
+        with pytest.raises(fl._lib.FlError):
+            call(work=torch.empty(256, dtype=torch.uint8, device=dev))
+
+
 def test_prefill_kv_split_chunk_deep_in_prompt(fl, dev):
     """The reference's own prefill shape: a 1024-token chunk (MAX_CHUNK,
     runtime.py:196) at pos0 = 98000, where the 256-row workgroups (96) are
