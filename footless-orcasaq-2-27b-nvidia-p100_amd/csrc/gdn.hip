@@ -23,6 +23,8 @@
 
 #include "gdn_gates.hpp"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int GR_ROWS = 32;       // state rows a workgroup
@@ -920,6 +922,164 @@ gdn_decode_normed_kernel(const f16* __restrict__ x, int x_stride, const f16* __r
     }
 }
 
+// ---------------------------------------------------------------------------
+// A verify round's rows (one sequence, T = 2 or 3) from the raw q|k|v rows, in
+// two launches where conv rows, step and norm were three. gdn_verify_kernel:
+// the step of gdn_decode_kernel (32 state rows a workgroup, 8 lanes a row) with
+// the conv of all T rows in it. Nothing but the state passes from row to row,
+// so the conv, the sums of squares, the gates and the norms of every row are
+// formed together, two barriers in all (a row at a time: 3 T - 1), and the T
+// delta rules follow each other on registers. The conv frames are only read
+// here -- the 12 workgroups of a k head share its channels, and row 0's new
+// frames go where the old ones are -- and written by the second launch,
+// gdn_verify_finish_kernel: the output norm of the T rows, a wave a row, and the
+// frames after each row, a thread a channel. The values of conv1d_causal_rows,
+// gdn_decode and rmsnorm_gated bit for bit. One sequence, T = 3, 48 v heads:
+// bound by its launches and the chain inside the step, not by its 13 MB: the round
+// of 12 such layers and 4 attention layers at 32k went 291 -> 231 us.
+// ---------------------------------------------------------------------------
+template <int T>
+struct ConvRowsIn {
+    f16 h[3], x[T];
+    f16x4 w;
+};
+template <int T>
+__device__ __forceinline__ ConvRowsIn<T> conv_rows_load(const f16* __restrict__ x, int x_stride,
+                                                        const f16* __restrict__ w,
+                                                        const f16* __restrict__ st_in, int d) {
+    ConvRowsIn<T> c;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) c.h[j] = st_in[(size_t)d * 3 + j];
+#pragma unroll
+    for (int t = 0; t < T; ++t) c.x[t] = x[(size_t)t * x_stride + d];
+    c.w = *(const f16x4*)(w + (size_t)d * 4);
+    return c;
+}
+// the conv's fp16-rounded outputs of every row (a row's x enters the later rows'
+// window rounded by f16_sat, as conv_window_kernel's row form)
+template <int T>
+__device__ __forceinline__ void conv_rows_apply(const ConvRowsIn<T>& c, bool hist, float (&y)[T]) {
+    float e[3 + T];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) e[j] = hist ? (float)c.h[j] : 0.f;
+#pragma unroll
+    for (int t = 0; t < T; ++t) e[3 + t] = (float)f16_sat((float)c.x[t]);
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        float acc = 0.f;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) acc = fmaf((float)c.w[j], e[t + j], acc);
+        acc = fmaf((float)c.w[3], (float)c.x[t], acc);
+        y[t] = (float)f16_sat(silu_f(acc));
+    }
+}
+
+template <int T>
+__global__ void __launch_bounds__(GR_THREADS)
+gdn_verify_kernel(const f16* __restrict__ x, int x_stride, const f16* __restrict__ conv_w,
+                  const f16* __restrict__ st_in, int pos0, const float* __restrict__ ga,
+                  const float* __restrict__ gb, int ab_stride, const float* __restrict__ A_log,
+                  const float* __restrict__ dt_bias, float* __restrict__ S, f16* __restrict__ y,
+                  float* __restrict__ Ck, long long ck_step, int n_kheads, int n_vheads,
+                  float out_scale, float l2eps, int group) {
+    __shared__ __attribute__((aligned(16))) float ssq[T][8];
+    __shared__ __attribute__((aligned(16))) float snorm[T][2 * GR_K];
+    __shared__ float sv[T][GR_ROWS];
+    __shared__ float sg[T][2];
+    const int rb = blockIdx.x, hv = blockIdx.y, hk = hv / group;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ri = tid >> 3, c0 = 4 * (tid & 7);
+    const int vi = rb * GR_ROWS + ri;
+    const size_t srow = ((size_t)hv * GN_ROWS + vi) * GR_K + c0;
+    const int half_ = tid >> 7, i = tid & 127;
+    const int ch = (half_ ? hk * GR_K : n_kheads * GR_K + hk * GR_K) + i;   // q | k channel
+    const int gw = (rb + hv) & 3, vw = gw ^ 2;
+    const int ch_v = 2 * n_kheads * GR_K + hv * GN_ROWS + rb * GR_ROWS + (lane & 31);
+    // the small inputs first, then the state, as in gdn_decode_kernel
+    const ConvRowsIn<T> cq = conv_rows_load<T>(x, x_stride, conv_w, st_in, ch);
+    const ConvRowsIn<T> cv = conv_rows_load<T>(x, x_stride, conv_w, st_in, ch_v);
+    const int vz = opaque_zero();
+    const float dtb = dt_bias[hv + vz], A = A_log[hv + vz];
+    float a_t[T], b_t[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        a_t[t] = ga[(size_t)t * ab_stride + hv + vz];
+        b_t[t] = gb[(size_t)t * ab_stride + hv + vz];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float reg[16];
+    load_row16_nt(reg, S + srow);
+    __builtin_amdgcn_sched_barrier(0);
+    float xv[T], vv[T];
+    conv_rows_apply<T>(cq, pos0 > 0, xv);
+    conv_rows_apply<T>(cv, pos0 > 0, vv);
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        const float tr = warp32_tree_lane0(xv[t] * xv[t]);
+        if ((lane & 31) == 0) ssq[t][tid >> 5] = tr;
+        if (w == vw && lane < GR_ROWS) sv[t][lane] = vv[t];
+        if (w == gw) {
+            const float bt = gdn_beta(b_t[t]), dt = gdn_decay(a_t[t] + dtb, A);
+            if (lane == 0) {
+                sg[t][0] = bt;
+                sg[t][1] = dt;
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < T; ++t) {   // the reference's order (r0 + r2) + (r1 + r3)
+        const f32x4 r = *(const f32x4*)&ssq[t][4 * (w >> 1)];
+        const float den = sqrtf(((r[0] + r[2]) + (r[1] + r[3])) + l2eps);
+        snorm[t][tid] = (float)f16_sat(xv[t] / den);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        float kk[16], qq[16];
+        gather16(kk, snorm[t], c0);
+        gather16(qq, snorm[t] + GR_K, c0);
+        __builtin_amdgcn_sched_barrier(0);
+        delta_update(reg, kk, sv[t][ri], sg[t][0], sg[t][1]);
+        store_row16_nt(t == T - 1 ? S + srow : Ck + (size_t)t * ck_step + srow, reg);
+        const float o = delta_out(reg, qq);
+        if (c0 == 0) y[((size_t)t * n_vheads + hv) * GN_ROWS + vi] = f16_sat(o * out_scale);
+    }
+}
+
+// grid: norm_wgs workgroups of 4 rows' waves, then dim / 256 of channels
+template <int T>
+__global__ void __launch_bounds__(GR_THREADS)
+gdn_verify_finish_kernel(const f16* __restrict__ o, const f16* __restrict__ z,
+                         const float* __restrict__ nw, f16* __restrict__ y, int n_rows, float eps,
+                         int norm_wgs, const f16* __restrict__ x, int x_stride, const f16* st_in,
+                         f16* st0, f16* st1, f16* st2, int dim, int pos0) {
+    if ((int)blockIdx.x < norm_wgs) {
+        const int lane = threadIdx.x & 63;
+        const int rid = blockIdx.x * (GR_THREADS / 64) + (threadIdx.x >> 6);
+        if (rid >= n_rows) return;
+        const size_t base = (size_t)rid * GR_K + 2 * lane;
+        const f16x2 ov = *(const f16x2*)(o + base);
+        const f16x2 zv = *(const f16x2*)(z + base);
+        *(f16x2*)(y + base) = gated_rms_pair((float)ov[0], (float)ov[1], (float)zv[0],
+                                             (float)zv[1], nw[2 * lane], nw[2 * lane + 1], eps);
+        return;
+    }
+    const int d = (blockIdx.x - norm_wgs) * GR_THREADS + threadIdx.x;
+    if (d >= dim) return;
+    f16 e[3 + T];   // the window's frames, oldest first
+#pragma unroll
+    for (int j = 0; j < 3; ++j) e[j] = pos0 > 0 ? f16_sat((float)st_in[(size_t)d * 3 + j]) : (f16)0.f;
+#pragma unroll
+    for (int t = 0; t < T; ++t) e[3 + t] = f16_sat((float)x[(size_t)t * x_stride + d]);
+    f16* const st[3] = {st0, st1, st2};
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) st[t][(size_t)d * 3 + j] = e[t + 1 + j];
+}
+
 // The same norm, 16-byte aligned rows: 16 lanes a row (lane j of the row holds
 // o[8 j .. 8 j + 7], one 16-byte load), 4 rows a wave per pass and GR_PASSES
 // passes (all loads issued first), so a wave carries 4 GR_PASSES rows.
@@ -1297,6 +1457,52 @@ int fl_gdn_decode_normed(const void* x, int x_stride, int conv_fused, const void
     return fl::check_launch("gdn_decode_normed");
 }
 
+
+int fl_gdn_verify_normed(const void* x, int x_stride, const void* conv_w, const void* st_in,
+                         void* st0, void* st1, void* st2, int pos0, const float* a,
+                         const float* b, int ab_stride, const float* A_log, const float* dt_bias,
+                         float* S, float* Ck, long long ck_step, const void* z,
+                         const float* norm_w, void* y, int T, int n_kheads, int n_vheads, int K,
+                         int V, float out_scale, float l2eps, float norm_eps, void* work,
+                         size_t work_bytes, fl_stream_t stream) {
+    FL_REQUIRE(x && conv_w && st_in && a && b && A_log && dt_bias && S && Ck && z && norm_w && y &&
+                   work,
+               "null pointer");
+    FL_REQUIRE(T == 2 || T == 3, "T is 2 or 3");
+    FL_REQUIRE(st0 && st1 && (T < 3 || st2), "a state buffer per row");
+    FL_REQUIRE(K == GR_K && V == GN_ROWS, "K and V must be 128");
+    FL_REQUIRE(n_kheads >= 1 && n_vheads >= 1 && n_vheads % n_kheads == 0,
+               "n_vheads % n_kheads == 0");
+    const int dim = 2 * n_kheads * K + n_vheads * V;
+    FL_REQUIRE(x_stride >= dim && ab_stride >= n_vheads && pos0 >= 0, "x_stride, ab_stride, pos0");
+    FL_REQUIRE(aligned16(S) && aligned16(Ck) && ck_step % 4 == 0, "16-byte aligned S / Ck");
+    FL_REQUIRE(((uintptr_t)z & 3u) == 0 && ((uintptr_t)y & 3u) == 0 &&
+                   ((uintptr_t)work & 3u) == 0 && ((uintptr_t)norm_w & 7u) == 0 && norm_eps >= 0.f,
+               "aligned z, y, work, norm_w");
+    const size_t need = (size_t)T * n_vheads * V * sizeof(f16);
+    if (work_bytes < need) {
+        fl::set_error("work: %zu bytes, T * n_vheads * V halves are %zu", work_bytes, need);
+        return FL_ESCRATCH;
+    }
+    const dim3 grid(V / GR_ROWS, n_vheads);
+    const int n_rows = T * n_vheads, norm_wgs = (n_rows + 3) / 4;
+    const int wgs = norm_wgs + (dim + GR_THREADS - 1) / GR_THREADS;
+    auto run = [&](auto tt) {
+        constexpr int TT = decltype(tt)::value;
+        hipLaunchKernelGGL(gdn_verify_kernel<TT>, grid, dim3(GR_THREADS), 0, (hipStream_t)stream,
+                           (const f16*)x, x_stride, (const f16*)conv_w, (const f16*)st_in, pos0, a,
+                           b, ab_stride, A_log, dt_bias, S, (f16*)work, Ck, ck_step, n_kheads,
+                           n_vheads, out_scale, l2eps, n_vheads / n_kheads);
+        const int rc = fl::check_launch("gdn_verify");
+        if (rc) return rc;
+        hipLaunchKernelGGL(gdn_verify_finish_kernel<TT>, dim3(wgs), dim3(GR_THREADS), 0,
+                           (hipStream_t)stream, (const f16*)work, (const f16*)z, norm_w, (f16*)y,
+                           n_rows, norm_eps, norm_wgs, (const f16*)x, x_stride,
+                           (const f16*)st_in, (f16*)st0, (f16*)st1, (f16*)st2, dim, pos0);
+        return fl::check_launch("gdn_verify_finish");
+    };
+    return T == 2 ? run(std::integral_constant<int, 2>()) : run(std::integral_constant<int, 3>());
+}
 
 int fl_rmsnorm_gated(const void* o, const void* z, const float* w, void* y, int n, int rows,
                      int pitch, int T, float eps, fl_stream_t stream) {

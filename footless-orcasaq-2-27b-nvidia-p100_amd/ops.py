@@ -671,6 +671,35 @@ def gdn_decode_normed(x, S, a, b, A_log, dt_bias, z, norm_w, y=None, *, pos0s, T
     return y
 
 
+def gdn_verify_normed(x, conv_w, st_in, st0, st1, st2, a, b, A_log, dt_bias, S, ck, ck_step, z,
+                      norm_w, y=None, *, T: int, pos0: int, n_kheads: int = GDN_K_HEADS,
+                      n_vheads: int = GDN_V_HEADS, K: int = GDN_K, V: int = GDN_V,
+                      x_stride: int = QKV_ROWS, ab_stride: int = GDN_V_HEADS,
+                      out_scale: float = Q_SCALE, l2eps: float = L2_EPS,
+                      norm_eps: float = GDN_NORM_EPS):
+    """A verify round's T = 2 or 3 rows of one sequence (runtime.py:3021-3065):
+    conv1d_causal_rows, gdn_decode with the checkpoints (ck + t * ck_step) and
+    rmsnorm_gated in one call. x [T, x_stride] fp16 the raw q|k|v rows; st0 may
+    be st_in. Returns y [T, n_vheads, V] fp16."""
+    _contig(S, "S")
+    if y is None:
+        y = torch.empty((T, n_vheads, V), dtype=F16, device=x.device)
+    work = torch.empty_like(y)
+    dim, state, rows = 2 * n_kheads * K + n_vheads * V, n_vheads * V * K, T * n_vheads * V
+    _lib.call("fl_gdn_verify_normed", _ptr(x, F16, "x", (T - 1) * x_stride + dim), x_stride,
+              _ptr(conv_w, F16, "conv_w", dim * 4), _ptr(st_in, F16, "st_in", dim * 3),
+              _ptr(st0, F16, "st0", dim * 3), _ptr(st1, F16, "st1", dim * 3),
+              _ptr(st2, F16, "st2", dim * 3), pos0,
+              _ptr(a, F32, "a", (T - 1) * ab_stride + n_vheads),
+              _ptr(b, F32, "b", (T - 1) * ab_stride + n_vheads), ab_stride,
+              _ptr(A_log, F32, "A_log", n_vheads), _ptr(dt_bias, F32, "dt_bias", n_vheads),
+              _ptr(S, F32, "S", state), _ptr(ck, F32, "ck", (T - 2) * ck_step + state), ck_step,
+              _ptr(z, F16, "z", rows), _ptr(norm_w, F32, "norm_w", V), _ptr(y, F16, "y", rows), T,
+              n_kheads, n_vheads, K, V, float(out_scale), float(l2eps), float(norm_eps),
+              _ptr(work, F16, "work", rows), 2 * work.numel(), _stream())
+    return y
+
+
 def gdn_chunked_work_bytes(T: int, n_vheads: int = GDN_V_HEADS, K: int = GDN_K, V: int = GDN_V,
                            chunk: int = GDN_CHUNK) -> int:
     return int(_lib.lib().fl_gdn_chunked_work_bytes(T, n_vheads, K, V, chunk))

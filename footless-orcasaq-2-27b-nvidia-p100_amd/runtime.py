@@ -334,9 +334,9 @@ class HybridRuntime:
         gated output norm. Verify (T <= 1 + mtp_k): the conv rows leave row
         0's state in place in conv[phase], row 1's in conv[phase ^ 1], row 2's
         in the spare; the fused step keeps the recurrent state after each row
-        but the last as a checkpoint; then the gated output norm. Prefill:
-        conv over the chunk, the q / k L2 norm, the chunked WY scan with the
-        gates, then the gated output norm."""
+        but the last as a checkpoint; then the gated output norm (two
+        launches). Prefill: conv over the chunk, the q / k L2 norm, the chunked
+        WY scan with the gates, then the gated output norm."""
         g = self.gdn_ord[i]
         wt = self.w[i]
         S = st.s[g]
@@ -346,15 +346,10 @@ class HybridRuntime:
                                          pos0s=[pos0], conv_w=wt.conv_w, cst_in=[cin],
                                          cst_out=[cout]).view(1, GDN_V_HEADS, GDN_V)
         if verify:
-            c = torch.empty_like(qkv)
-            # the one-launch step + norm gives one sequence's rows 48 workgroups
-            # (a v head each): slower here than the 192 of the step alone
-            ops.conv1d_causal_rows(qkv, wt.conv_w, cin, c, cin, cout, self.snap_c[g], T=T,
-                                   pos0=pos0)
-            y = ops.gdn_decode(c[None], [S], a[None], b[None], wt.A_log, wt.dt_bias, T=T,
-                               pos0s=[pos0], ck=[self.snap_s[0, g]],
-                               ck_step=self.n_gdn * self.layer_s_elems)[0]
-            return ops.rmsnorm_gated(y.view(T, GDN_V_HEADS, GDN_V), zg, wt.norm_w, T=T)
+            return ops.gdn_verify_normed(qkv, wt.conv_w, cin, cin, cout, self.snap_c[g], a, b,
+                                         wt.A_log, wt.dt_bias, S, self.snap_s[0, g],
+                                         self.n_gdn * self.layer_s_elems, zg, wt.norm_w, T=T,
+                                         pos0=pos0)
         # conv, q / k norm, the chunked scan with its gates and the output norm
         return ops.gdn_prefill_layer(qkv, wt.conv_w, cin, cout, a, b, wt.A_log, wt.dt_bias, S, zg,
                                      wt.norm_w, T=T, pos0=pos0)

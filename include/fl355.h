@@ -460,6 +460,21 @@ int fl_gdn_decode_normed(const void* x, int x_stride, int conv_fused, const void
                          int V, float out_scale, float l2eps, float norm_eps,
                          fl_stream_t stream);
 
+/* A verify round's rows of one sequence (T = 2 or 3) from the raw q|k|v rows:
+ * fl_conv1d_causal_rows, fl_gdn_decode with a checkpoint after every row but
+ * the last, then fl_rmsnorm_gated -- the sequence runtime.py:3021-3065 launches,
+ * the same values -- in two launches. x [T][x_stride] f16; st_in, st0 .. st2 as
+ * fl_conv1d_causal_rows' (st0 may be st_in; st2 with T == 3); Ck / ck_step as
+ * fl_gdn_scan's; z, y [T][n_vheads][V] f16. work: T * n_vheads * V halves.
+ * K == V == 128, S and Ck 16-byte aligned. */
+int fl_gdn_verify_normed(const void* x, int x_stride, const void* conv_w, const void* st_in,
+                         void* st0, void* st1, void* st2, int pos0, const float* a,
+                         const float* b, int ab_stride, const float* A_log, const float* dt_bias,
+                         float* S, float* Ck, long long ck_step, const void* z,
+                         const float* norm_w, void* y, int T, int n_kheads, int n_vheads, int K,
+                         int V, float out_scale, float l2eps, float norm_eps, void* work,
+                         size_t work_bytes, fl_stream_t stream);
+
 /* ---- GDN chunked prefill --------------------------------------------------
  * Chunked (WY / UT transform) GDN prefill: the same recurrence as
  * fl_gdn_scan over T tokens in chunks of `chunk` tokens, fp32 state carried

@@ -734,3 +734,38 @@ def test_prefill_layer_equals_separate_calls(fl, dev, rng, T, pos0, x_off):
     assert torch.equal(so1, so2), "conv frames differ"
     assert torch.equal(S1, S2), "state differs"
     assert torch.equal(y1, y2), "normed rows differ"
+
+
+@pytest.mark.parametrize("T,pos0", [(2, 0), (3, 0), (2, 9), (3, 9)])
+def test_verify_round_equals_separate_calls(fl, dev, rng, T, pos0):
+    """A verify round's rows in one call against conv1d_causal_rows, gdn_decode
+    with checkpoints and rmsnorm_gated: the normed rows, the state, every
+    checkpoint and the frames after every row (row 0's in place) bit for bit."""
+    x = to_dev((rng.standard_normal((T, ROW)) * 1.5).astype(np.float16), dev)
+    w = to_dev((rng.standard_normal((ROW, 4)) * 0.5).astype(np.float16), dev)
+    ad = to_dev(rng.standard_normal((T, NV)).astype(np.float32), dev)
+    bd = to_dev(rng.standard_normal((T, NV)).astype(np.float32), dev)
+    A_log = to_dev((rng.standard_normal(NV) * 0.3).astype(np.float32), dev)
+    dt = to_dev((rng.standard_normal(NV) * 0.3).astype(np.float32), dev)
+    z = to_dev(rng.standard_normal((T, NV, 128)).astype(np.float16), dev)
+    nw = to_dev((1 + rng.standard_normal(128) * 0.2).astype(np.float32), dev)
+    st = to_dev(rng.standard_normal((ROW, 3)).astype(np.float16), dev)
+    S = to_dev((rng.standard_normal((NV, 128, 128)) * 0.05).astype(np.float32), dev)
+    state = NV * 128 * 128
+    f = [st.clone()] + [torch.full_like(st, 9.0) for _ in range(2)]
+    u = [t.clone() for t in f]
+    Sf, Su = S.clone(), S.clone()
+    ckf = torch.full((2, NV, 128, 128), 7.0, device=dev)
+    cku = ckf.clone()
+    yf = fl.ops.gdn_verify_normed(x, w, f[0], f[0], f[1], f[2], ad, bd, A_log, dt, Sf, ckf, state,
+                                  z, nw, T=T, pos0=pos0)
+    c = torch.empty_like(x)
+    fl.ops.conv1d_causal_rows(x, w, u[0], c, u[0], u[1], u[2], T=T, pos0=pos0)
+    yu = fl.ops.gdn_decode(c[None], [Su], ad[None], bd[None], A_log, dt, T=T, pos0s=[pos0],
+                           ck=[cku], ck_step=state)
+    yn = fl.ops.rmsnorm_gated(yu.view(T, NV, 128), z, nw, T=T)
+    torch.cuda.synchronize()
+    assert torch.equal(yf, yn), "normed rows differ"
+    assert torch.equal(Sf, Su) and torch.equal(ckf, cku), "state or checkpoints differ"
+    for t in range(3):
+        assert torch.equal(f[t], u[t]), f"frames after row {t} differ"
