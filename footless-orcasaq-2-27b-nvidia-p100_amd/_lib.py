@@ -126,7 +126,7 @@ def lib() -> ctypes.CDLL:
 
 def call(name: str, *args) -> None:
     """Call an int-returning entry point; raise FlError on a non-zero status."""
-    rc = getattr(lib(), name)(*args)
+    rc = getattr(_lib or lib(), name)(*args)
     if rc != FL_OK:
         detail = lib().fl_last_error().decode(errors="replace")
         if rc == FL_EINVAL:
@@ -134,15 +134,16 @@ def call(name: str, *args) -> None:
         raise FlError(name, rc, detail)
 
 
+# array types by length: making one costs more than filling it
+_PTRS = [ctypes.c_void_p * max(1, n) for n in range(FL_MAX_SEQS + 1)]
+_INTS = [ctypes.c_int * max(1, n) for n in range(FL_MAX_SEQS + 1)]
+
+
 def ptr_array(ptrs) -> ctypes.Array:
-    arr = (ctypes.c_void_p * max(1, len(ptrs)))()
-    for i, p in enumerate(ptrs):
-        arr[i] = p
-    return arr
+    n = len(ptrs)
+    return (_PTRS[n] if n <= FL_MAX_SEQS else ctypes.c_void_p * n)(*ptrs)
 
 
 def int_array(vals) -> ctypes.Array:
-    arr = (ctypes.c_int * max(1, len(vals)))()
-    for i, v in enumerate(vals):
-        arr[i] = int(v)
-    return arr
+    n = len(vals)
+    return (_INTS[n] if n <= FL_MAX_SEQS else ctypes.c_int * n)(*map(int, vals))

@@ -29,13 +29,29 @@ from .geometry import (ATTN_SCALE, DEC_SMAX, DEC_SPLIT_ROWS, DEC_TMIN, GATE_OFF,
 F16, F32, I8 = torch.float16, torch.float32, torch.int8
 
 
+# The current stream's handle without building a torch.cuda.Stream around it
+# (8 us of a call's 29: a decode step of 16 layers makes 20 calls).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device_index = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    if _raw_stream is None or _device_index is None:
+        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return _raw_stream(_device_index())
 
 
 def _ptr(t: torch.Tensor | None, dtype, name: str, span: int = 0):
     """Device pointer of `t` after checking dtype / device and that its
     storage holds `span` elements from its start."""
+    # a dense tensor of at least `span` elements (every other case below)
+    if (isinstance(t, torch.Tensor) and t.dtype is dtype and t.is_cuda and t.numel() >= span
+            and t.is_contiguous()):
+        return t.data_ptr()
+    return _ptr_any(t, dtype, name, span)
+
+
+def _ptr_any(t, dtype, name, span):
     if t is None:
         return None
     if not isinstance(t, torch.Tensor):
@@ -786,4 +802,49 @@ def gdn_prefill_layer(x, conv_w, st_in, st_out, a, b, A_log, dt_bias, S, z, norm
               _ptr(norm_w, F32, "norm_w", V), _ptr(y, F16, "y", T * n_vheads * V), T, n_kheads,
               n_vheads, K, V, float(out_scale), float(l2eps), float(norm_eps),
               _ptr(work, torch.uint8, "work", need), work.numel(), _stream())
+    return y
+
+
+# ---------------------------------------------------------------------------
+# A decode step's layers as the runtime calls them, one row a sequence: the
+# checks and values of attn_prep_rows + attn_decode(_q8) and of
+# gdn_decode_normed, with the sequences' pointers, positions and capacities
+# already in ctypes arrays that the layers share.
+# ---------------------------------------------------------------------------
+
+def attn_step(qg, k, v, wq, wk, kps, vps, pos, caps, *, B: int, kv8: bool, split_rows: int, work):
+    """qg [B, 24, 512], k / v [B, 4, 256] fp16; kps / vps, pos, caps: arrays of
+    this layer's cache pointers, the positions and the capacities. Returns z
+    [B, 24, 256] fp16, gated."""
+    if qg.shape[0] != B:
+        raise ValueError("one cache pair, position and capacity per row")
+    _contig(qg, "qg")
+    call, st = _lib.call, _stream()
+    qp = _ptr(qg, F16, "qg", B * N_HEADS * Q_PITCH)
+    row = N_KV * HEAD_DIM
+    call("fl_attn_prep_rows", qp, Q_PITCH, _ptr(k, F16, "k", B * row), _ptr(v, F16, "v", B * row),
+         _ptr(wq, F32, "wq", HEAD_DIM), _ptr(wk, F32, "wk", HEAD_DIM), kps, vps, pos, caps, B,
+         int(kv8), N_HEADS, N_KV, HEAD_DIM, ROPE_DIM, ROPE_THETA, NORM_EPS, st)
+    z = torch.empty((B, N_HEADS, HEAD_DIM), dtype=F16, device=qg.device)
+    call("fl_attn_decode_q8" if kv8 else "fl_attn_decode", qp, Q_PITCH, kps, vps, pos, caps, B, 1,
+         N_HEADS, N_KV, HEAD_DIM, ATTN_SCALE, split_rows, SPLIT_MAX, qp, Q_PITCH, GATE_OFF,
+         z.data_ptr(), HEAD_DIM, work.data_ptr(), work.numel(), st)
+    return z
+
+
+def gdn_step(x, a, b, A_log, dt_bias, z, norm_w, conv_w, sps, cins, couts, pos, *, B: int):
+    """x [B, 10240], z [B, 48, 128] fp16, a, b [B, 48] fp32; sps, cins, couts, pos:
+    arrays of the layer's state and conv frame pointers and of the positions.
+    Returns y [B, 48, 128] fp16."""
+    width = GDN_V_HEADS * GDN_V
+    _contig(x, "x"), _contig(a, "a"), _contig(b, "b")
+    pitch = width if z.is_contiguous() else z.view(B, width).stride(0)
+    y = torch.empty((B, GDN_V_HEADS, GDN_V), dtype=F16, device=x.device)
+    _lib.call("fl_gdn_decode_normed", _ptr(x, F16, "x", B * QKV_ROWS), QKV_ROWS, 1,
+              _ptr(conv_w, F16, "conv_w", QKV_ROWS * 4), cins, couts, pos,
+              _ptr(a, F32, "a", B * GDN_V_HEADS), _ptr(b, F32, "b", B * GDN_V_HEADS), GDN_V_HEADS,
+              _ptr(A_log, F32, "A_log", GDN_V_HEADS), _ptr(dt_bias, F32, "dt_bias", GDN_V_HEADS),
+              sps, None, 0, _ptr(z, F16, "z", (B - 1) * pitch + width), pitch,
+              _ptr(norm_w, F32, "norm_w", GDN_V), y.data_ptr(), width, B, 1, GDN_K_HEADS,
+              GDN_V_HEADS, GDN_K, GDN_V, Q_SCALE, L2_EPS, GDN_NORM_EPS, _stream())
     return y

@@ -38,7 +38,7 @@ from typing import Protocol, Sequence
 
 import torch
 
-from . import ops, state_blob
+from . import _lib, ops, state_blob
 from .geometry import (DEC_SPLIT_ROWS, GDN_K, GDN_K_HEADS, GDN_V, GDN_V_HEADS, HEAD_DIM,
                        N_KV, QKV_ROWS, SPLIT_T_MAX, kv8_nbytes)
 
@@ -329,9 +329,8 @@ class HybridRuntime:
 
     def _gdn(self, st: SeqState, i: int, qkv, zg, a, b, T: int, pos0: int,
              verify: bool) -> torch.Tensor:
-        """runtime.py:2961-3112 for one sequence. Decode (T = 1): one launch
-        runs the conv (conv[phase] -> conv[phase ^ 1]), the fused step and the
-        gated output norm. Verify (T <= 1 + mtp_k): the conv rows leave row
+        """runtime.py:2961-3112 for one sequence's verify or prefill (a decode
+        row: _decode_layers). Verify (T <= 1 + mtp_k): the conv rows leave row
         0's state in place in conv[phase], row 1's in conv[phase ^ 1], row 2's
         in the spare; the fused step keeps the recurrent state after each row
         but the last as a checkpoint; then the gated output norm (two
@@ -341,10 +340,6 @@ class HybridRuntime:
         wt = self.w[i]
         S = st.s[g]
         cin, cout = st.conv[st.phase, g], st.conv[st.phase ^ 1, g]
-        if T == 1 and not verify:   # the step and its output norm, one launch
-            return ops.gdn_decode_normed(qkv, [S], a, b, wt.A_log, wt.dt_bias, zg, wt.norm_w,
-                                         pos0s=[pos0], conv_w=wt.conv_w, cst_in=[cin],
-                                         cst_out=[cout]).view(1, GDN_V_HEADS, GDN_V)
         if verify:
             return ops.gdn_verify_normed(qkv, wt.conv_w, cin, cin, cout, self.snap_c[g], a, b,
                                          wt.A_log, wt.dt_bias, S, self.snap_s[0, g],
@@ -378,14 +373,17 @@ class HybridRuntime:
                 raise ValueError(f"a verify carries 2..{1 + self.mtp_k} rows")
             self._ensure_verify_buffers()
         self.grow(st, pos0 + T)
-        for i, kind in enumerate(self.layer_types):
-            if kind == "full_attention":
-                qg, k, v = proj.full_attn_in(i, T)
-                out = self._full_attn(st, i, qg, k, v, T, pos0)
-            else:
-                qkv, zg, a, b = proj.gdn_in(i, T)
-                out = self._gdn(st, i, qkv, zg, a, b, T, pos0, verify)
-            proj.layer_out(i, out)
+        if T == 1 and not verify:
+            self._decode_layers([st], proj, [pos0])
+        else:
+            for i, kind in enumerate(self.layer_types):
+                if kind == "full_attention":
+                    qg, k, v = proj.full_attn_in(i, T)
+                    out = self._full_attn(st, i, qg, k, v, T, pos0)
+                else:
+                    qkv, zg, a, b = proj.gdn_in(i, T)
+                    out = self._gdn(st, i, qkv, zg, a, b, T, pos0, verify)
+                proj.layer_out(i, out)
         if verify:
             self.verify_T, self._verify_pos0 = T, pos0
             return
@@ -425,6 +423,61 @@ class HybridRuntime:
         st.fed = 0
         return r
 
+    # -- one decode step's layers ------------------------------------------------
+
+    def _decode_layers(self, states: Sequence[SeqState], proj: Projections,
+                       pos0s: Sequence[int]) -> None:
+        """The layers of a decode step of one token a sequence: per full-attention
+        layer one launch of every row's prep into its own cache, then one
+        attention call over all rows; per GDN layer one fused conv + delta rule
+        + output norm launch over all rows. The states are checked once a step
+        and their layers addressed by stride: a tensor view and its checks for
+        every layer, sequence and buffer cost the host more than the kernels
+        take (a 16-layer step of one sequence at 4k: 579 us)."""
+        B = len(states)
+        if any(len(st.kk or ()) < self.n_full for st in states):
+            raise ValueError("a state without the layers' caches")
+        pos = _lib.int_array(pos0s)
+        g_state, ring = self.layer_s_elems, QKV_ROWS * 3
+        sps, cins, couts = (_lib.ptr_array([None] * B) for _ in range(3))
+        at = []   # per sequence: state, frames in, frames out, and their layer strides (bytes)
+        for st in states if self.n_gdn else ():
+            s, c = st.s, st.conv
+            span = (self.n_gdn - 1) * s.stride(0) + g_state
+            last = c.stride(0) + (self.n_gdn - 1) * c.stride(1) + ring
+            sp, cp = ops._ptr(s, F32, "S[b]", span), ops._ptr(c, F16, "conv[b]", last)
+            ph = 2 * c.stride(0)
+            at.append((sp, cp + st.phase * ph, cp + (st.phase ^ 1) * ph, 4 * s.stride(0),
+                       2 * c.stride(1)))
+        work = None
+        if self.n_full:
+            work = torch.empty(ops.attn_decode_work_bytes(B, 1), dtype=torch.uint8,
+                               device=states[0].kk[0].device)
+        kv8 = self.kv8
+        kv_type = torch.int8 if kv8 else F16
+        for i, kind in enumerate(self.layer_types):
+            wt = self.w[i]
+            if kind == "full_attention":
+                li = self.full_ord[i]
+                qg, k, v = proj.full_attn_in(i, B)
+                lcaps = [st.lcap[li] for st in states]
+                spans = [kv8_nbytes(n) if kv8 else n * N_KV * HEAD_DIM for n in lcaps]
+                kps = _lib.ptr_array([ops._ptr(st.kk[li], kv_type, "kcache", n)
+                                      for st, n in zip(states, spans)])
+                vps = _lib.ptr_array([ops._ptr(st.kv[li], kv_type, "vcache", n)
+                                      for st, n in zip(states, spans)])
+                out = ops.attn_step(qg, k, v, wt.q_norm, wt.k_norm, kps, vps, pos,
+                                    _lib.int_array(lcaps), B=B, kv8=kv8,
+                                    split_rows=self.split_rows, work=work)
+            else:
+                g = self.gdn_ord[i]
+                qkv, zg, a, b = proj.gdn_in(i, B)
+                for j, (sp, ci, co, ds, dc) in enumerate(at):
+                    sps[j], cins[j], couts[j] = sp + g * ds, ci + g * dc, co + g * dc
+                out = ops.gdn_step(qkv, a, b, wt.A_log, wt.dt_bias, zg, wt.norm_w, wt.conv_w, sps,
+                                   cins, couts, pos, B=B)
+            proj.layer_out(i, out)
+
     # -- batched decode --------------------------------------------------------
 
     def forward_batch(self, states: Sequence[SeqState], proj: Projections,
@@ -444,32 +497,7 @@ class HybridRuntime:
                 raise ValueError("a state holds a replay")
             pos0s.append(len(st.tokens))
             self.grow(st, len(st.tokens) + 1)
-        for i, kind in enumerate(self.layer_types):
-            if kind == "full_attention":
-                li, wt = self.full_ord[i], self.w[i]
-                qg, k, v = proj.full_attn_in(i, B)
-                kcs = [st.kk[li] for st in states]
-                vcs = [st.kv[li] for st in states]
-                # every row's prep into its own cache, one launch (the same values
-                # as a prep a row)
-                ops.attn_prep_rows(qg, k, v, wt.q_norm, wt.k_norm, kcs, vcs, pos0s,
-                                   [st.lcap[li] for st in states], kv8=self.kv8)
-                if self.kv8:
-                    z = ops.attn_decode_q8(qg[:, None], kcs, vcs, pos0s,
-                                           [st.lcap[li] for st in states],
-                                           split_rows=self.split_rows)
-                else:
-                    z = ops.attn_decode(qg[:, None], kcs, vcs, pos0s, split_rows=self.split_rows)
-                proj.layer_out(i, z[:, 0])
-            else:
-                g, wt = self.gdn_ord[i], self.w[i]
-                qkv, zg, a, b = proj.gdn_in(i, B)
-                yn = ops.gdn_decode_normed(qkv, [st.s[g] for st in states], a, b, wt.A_log,
-                                           wt.dt_bias, zg, wt.norm_w, pos0s=pos0s,
-                                           conv_w=wt.conv_w,
-                                           cst_in=[st.conv[st.phase, g] for st in states],
-                                           cst_out=[st.conv[st.phase ^ 1, g] for st in states])
-                proj.layer_out(i, yn.view(B, GDN_V_HEADS, GDN_V))
+        self._decode_layers(states, proj, pos0s)
         for st, t in zip(states, tokens):
             st.tokens.append(int(t))
             st.fed = len(st.tokens)
