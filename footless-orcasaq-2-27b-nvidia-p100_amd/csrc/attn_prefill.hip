@@ -807,18 +807,24 @@ attn_prefill_r64_kernel(const f16* __restrict__ q, int q_pitch, const f16* __res
                 r64_issue(lds_base + d * R64_STAGE, kb, vb, rsb, (j_lo + d) * R64_BK, kv_end, w,
                           lane, loff);
 
-        f16x8 qreg[2][16];   // Q[row nb][128 hh + 8 ks + 0..7]
+        // Q[row nb][128 hh + 8 ks + 0..7] (a lane past the rows reads token 0's; its
+        // column is never stored)
+        f16x8 qreg[2][16];
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
             const f16* qrow = q + ((size_t)t[nb] * n_q_heads + h * G + g[nb]) * q_pitch + 128 * hh;
 #pragma unroll
             for (int ks = 0; ks < 16; ++ks)
-                // (STREAM: unconditional, a lane past the rows reads token 0's row and
-                // its column is never stored: 3 % at T = 777 from 3001; the other
-                // modes' tile loop is scheduled 2 - 3 % worse without the select)
-                qreg[nb][ks] = STREAM || rvalid[nb] ? *(const f16x8*)(qrow + 8 * ks) : (f16x8)(0);
+                qreg[nb][ks] = *(const f16x8*)(qrow + 8 * ks);
         }
-        WAIT_VMCNT(0);   // Q and the first tiles: the wait left to the compiler lands in the loop
+        WAIT_VMCNT(0);   // the first tiles, and Q ...
+        // ... whose values are pinned here: a load the compiler moves below that
+        // wait is waited for at its use, inside the tile loop and with vmcnt(0)
+        // at the last one, on every tile and for the next tiles' copies with it
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+            for (int ks = 0; ks < 16; ++ks) asm volatile("" : "+v"(qreg[nb][ks]));
 
         f32x16 o[2][8];
 #pragma unroll
