@@ -26,9 +26,10 @@
 // gates, and T and M o QK^T written as fp16 MFMA operands.
 // chunk_state_kernel: a state wavefront per 16 state rows (v) of a v head,
 // all 128 k columns of them in fp32 registers, sequential over the chunks; a
-// paired output wavefront takes its Q S0^T and Delta through LDS a chunk later,
-// forms O and stores y, and issues the HBM -> LDS copies of the operands one
-// chunk ahead, so the state chain carries only its own products.
+// paired output wavefront takes its split S0 and Delta through LDS a chunk
+// later, forms Q S0^T and O and stores y; a copy wavefront issues the HBM ->
+// LDS copies of the operands one chunk ahead, so the state chain carries only
+// its own products.
 //
 // Precision. Every product runs on v_mfma_f32_16x16x32_f16 (fp16 inputs,
 // fp32 accumulate: the product of two fp16 values is exact in fp32). K, Q and
@@ -716,23 +717,27 @@ gdn_front_kernel(const f16* __restrict__ x, const f16* __restrict__ conv_w,
 }
 
 // ---------------------------------------------------------------------------
-// chunk_state_kernel: 32 state rows (v) of a v head a workgroup, 4 wavefronts.
-// Waves 0 and 1 (state waves) each hold 16 rows of S and run the recurrence's
-// chain: X = K S^T and Q S^T, Y, Delta = T Y, the state update. Waves 2 and 3
-// (output waves) each take a state wave's Q S^T and Delta a chunk later, form
-// O and store y, and issue every HBM -> LDS copy, so the state waves' chain
-// carries neither.
+// chunk_state_kernel: 32 state rows (v) of a v head a workgroup. Waves 0 and 1
+// (state waves) each hold 16 rows of S and run the recurrence's chain: X = K
+// S^T, Y, Delta = T Y, the state update. Waves 2 and 3 (output waves) each take
+// a state wave's split S and Delta a chunk later, form Q S^T and O and store y.
+// Waves 6 and 7 (copy waves) issue every HBM -> LDS copy, a chunk ahead and
+// more. (A wave's SIMD is its number modulo 4: waves 4 and 5, which would share
+// the state waves', leave at once.) The state waves' chain is what the kernel
+// takes, so what is not part of it lies elsewhere, and within it the VALU work
+// that a product does not wait for lies between the MFMAs of another: 42 -> 37.5
+// us for 1024 tokens of 48 heads, with the output waves issuing the copies and
+// the state waves forming Q S^T -> as here (4900 clocks a chunk).
 // ---------------------------------------------------------------------------
 constexpr int CS_ROWS = 32;   // state rows (v) a workgroup
-// A stage (the state waves' operands of a chunk): K and Q rows [64][256 B]
-// (16-byte chunk c of row r at c ^ (r & 15)), V columns [64][CS_ROWS] fp16,
-// T's hi / lo operands and the gates KiB (workspace bytes 0 .. 16 KiB and
-// 32 .. 33 KiB, as in HBM)
-constexpr int SA_K = 0, SA_Q = 16384, SA_V = 32768, SA_T = SA_V + CK_C * CS_ROWS * 2,
+// A stage (the state waves' operands of a chunk): K rows [64][256 B] (16-byte
+// chunk c of row r at c ^ (r & 15)), V columns [64][CS_ROWS] fp16, T's hi / lo
+// operands and the gates KiB (as in the workspace)
+constexpr int SA_K = 0, SA_V = 16384, SA_T = SA_V + CK_C * CS_ROWS * 2,
               SA_G = SA_T + 2 * WS_OP, SA_BYTES = SA_G + 1024;
-// B stage (the output waves'): M o QK^T's hi / lo operands (workspace bytes
-// 16 .. 32 KiB) and the gates KiB
-constexpr int SB_Q = 0, SB_G = 2 * WS_OP, SB_BYTES = SB_G + 1024;
+// B stage (the output waves'): Q rows as K's, M o QK^T's hi / lo operands and
+// the gates KiB
+constexpr int SB_Q = 0, SB_M = 16384, SB_G = SB_M + 2 * WS_OP, SB_BYTES = SB_G + 1024;
 // offsets in the gates KiB: beta, e^g, e^{g_C - g} [64] f32, then e^{g_C},
 // 2^-tau, 2^-kappa
 constexpr int G_BETA = WS_BETA - WS_BETA, G_EG = WS_EG - WS_BETA, G_DK = WS_DK - WS_BETA,
@@ -741,19 +746,23 @@ static_assert(WS_T_LO == WS_T_HI + WS_OP && WS_Q_HI == WS_T_LO + WS_OP &&
                   WS_Q_LO == WS_Q_HI + WS_OP && WS_BETA == WS_Q_LO + WS_OP &&
                   CK_BLK == WS_BETA + 1024 && WS_OP % 2048 == 0,
               "workspace block: T, then M o QK^T, then the gates KiB, whole copy pairs");
-// LDS: two A stages, two B stages, the hand-over (each state wave's Q S^T
-// 2^-s and Delta, [8][64 lanes] f32x4) and each output wave's y tile
-// [64 tokens][16 rows] fp16
-constexpr int L_A = 0, L_B = 2 * SA_BYTES, L_X = L_B + 2 * SB_BYTES, X_WAVE = 8 * 64 * 16,
+// LDS: two A stages, two B stages, the hand-over (each state wave's S as its
+// hi and lo B operands and Delta, [12][64 lanes] 16 bytes, then the lanes' 1 / s
+// and Delta's scale) and each output wave's y tile [64 tokens][16 rows] fp16
+constexpr int X_SL = 4 * 1024, X_DL = 8 * 1024, X_SC = 12 * 1024, X_WAVE = X_SC + 1024;
+constexpr int L_A = 0, L_B = 2 * SA_BYTES, L_X = L_B + 2 * SB_BYTES,
               L_Y = L_X + 2 * X_WAVE, CS_LDS = L_Y + 2 * CK_C * 16 * 2;
 static_assert(CS_LDS <= 160 * 1024, "the state pass's LDS fits 160 KiB");
-// y stores an output wave issues a chunk, after that chunk's copies
-constexpr int CS_NSTORE = 2;
+constexpr int CS_THREADS = 512;
 
 typedef __attribute__((address_space(3))) f32x4 lds_f32x4w;
+typedef __attribute__((address_space(3))) f16x8 lds_f16x8w;
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) f32x2 lds_f32x2w;
+typedef __attribute__((address_space(3))) float lds_f32w;
 typedef __attribute__((address_space(3))) f16 lds_f16w;
 
-// Per-lane source offsets of output wave wb's copies of a 64-token chunk (the
+// Per-lane source offsets of copy wave wb's copies of a 64-token chunk (the
 // base is scalar): K / Q copy n (n = 2 j + wb) brings rows 4 n .. 4 n + 3,
 // lane -> row 8 j + rr, rr = 4 wb + lane / 16, and 16-byte chunk
 // (lane % 16) ^ (row & 15), row & 15 = rr + 8 (j & 1); V copy n rows
@@ -769,23 +778,35 @@ __device__ __forceinline__ CsOff cs_offsets(int qk_bytes, int v_bytes, int wb, i
             (uint32_t)((lane >> 2) * v_bytes + 16 * (lane & 3)), (uint32_t)(16 * lane)};
 }
 
-// Output wave wb's half of the copies of chunk c's A stage into dst: 8 K, 8 Q,
-// 2 V and 6 T copies, and (wb = 0) the gates KiB. Rows past the last token
-// repeat it (beta is 0 there).
-__device__ __forceinline__ void cs_copy_a(uint32_t dst, const char* kb, const char* qb,
-                                          const char* vb, const char* wk, int t0, int T,
-                                          int qk_bytes, int v_bytes, int wb, int lane,
-                                          const CsOff& o) {
+// Copy wave wb's half of the 64 rows of K or Q of a chunk at t0 into dst: 8
+// copies. Rows past the last token repeat it (beta is 0 there).
+__device__ __forceinline__ void cs_copy_rows(uint32_t dst, const char* base, int t0, int T,
+                                             int qk_bytes, int wb, int lane, const CsOff& o) {
     if (T - t0 >= CK_C) {
-        const char* kt = kb + (size_t)t0 * qk_bytes;
-        const char* qt = qb + (size_t)t0 * qk_bytes;
-        const char* vt = vb + (size_t)t0 * v_bytes;
+        const char* at = base + (size_t)t0 * qk_bytes;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            copy16(at + (size_t)(8 * j) * qk_bytes, o.kq[j & 1], dst + 1024 * (2 * j + wb));
+    } else {
+        const int last = T - t0 - 1;
+        const int rr = 4 * wb + (lane >> 4), p = lane & 15;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const int n = 2 * j + wb;
-            copy16(kt + (size_t)(8 * j) * qk_bytes, o.kq[j & 1], dst + SA_K + 1024 * n);
-            copy16(qt + (size_t)(8 * j) * qk_bytes, o.kq[j & 1], dst + SA_Q + 1024 * n);
+            const int r = 8 * j + rr;
+            copy16_v(base + (size_t)(t0 + min(r, last)) * qk_bytes + 16 * (p ^ (r & 15)),
+                     __builtin_amdgcn_readfirstlane(dst + 1024 * (2 * j + wb)));
         }
+    }
+}
+
+// Copy wave wb's half of the copies of chunk c's A stage into dst: 8 K, 2 V and
+// 6 T copies, and (wb = 0) the gates KiB.
+__device__ __forceinline__ void cs_copy_a(uint32_t dst, const char* kb, const char* vb,
+                                          const char* wk, int t0, int T, int qk_bytes, int v_bytes,
+                                          int wb, int lane, const CsOff& o) {
+    cs_copy_rows(dst + SA_K, kb, t0, T, qk_bytes, wb, lane, o);
+    if (T - t0 >= CK_C) {
+        const char* vt = vb + (size_t)t0 * v_bytes;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int n = 2 * j + wb;
@@ -793,14 +814,6 @@ __device__ __forceinline__ void cs_copy_a(uint32_t dst, const char* kb, const ch
         }
     } else {
         const int last = T - t0 - 1;
-        const int rr = 4 * wb + (lane >> 4), p = lane & 15;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int n = 2 * j + wb, r = 8 * j + rr;
-            const size_t ro = (size_t)(t0 + min(r, last)) * qk_bytes + 16 * (p ^ (r & 15));
-            copy16_v(kb + ro, __builtin_amdgcn_readfirstlane(dst + SA_K + 1024 * n));
-            copy16_v(qb + ro, __builtin_amdgcn_readfirstlane(dst + SA_Q + 1024 * n));
-        }
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int n = 2 * j + wb, r = 16 * n + (lane >> 2);
@@ -816,34 +829,43 @@ __device__ __forceinline__ void cs_copy_a(uint32_t dst, const char* kb, const ch
     if (wb == 0) copy16(wk + WS_BETA, o.w, dst + SA_G);
 }
 
-// Output wave wb's half of the copies of chunk c's B stage: 6 M o QK^T copies
-// and (wb = 1) the gates KiB.
-__device__ __forceinline__ void cs_copy_b(uint32_t dst, const char* wk, int wb, const CsOff& o) {
+// Copy wave wb's half of the copies of chunk c's B stage: 8 Q and 6 M o QK^T
+// copies and (wb = 1) the gates KiB.
+__device__ __forceinline__ void cs_copy_b(uint32_t dst, const char* qb, const char* wk, int t0,
+                                          int T, int qk_bytes, int wb, int lane, const CsOff& o) {
+    cs_copy_rows(dst + SB_Q, qb, t0, T, qk_bytes, wb, lane, o);
 #pragma unroll
     for (int j = 0; j < WS_OP / 1024; ++j) {
         const int n = 2 * j + wb;
-        copy16(wk + WS_Q_HI + 1024 * n, o.w, dst + SB_Q + 1024 * n);
+        copy16(wk + WS_Q_HI + 1024 * n, o.w, dst + SB_M + 1024 * n);
     }
     if (wb == 1) copy16(wk + WS_BETA, o.w, dst + SB_G);
 }
 
-// The lane's parts of the swizzled K / Q row addresses, fixed for the kernel:
+// The lane's part of the swizzled K / Q row addresses, fixed for the kernel:
 // the A operand of X = K S^T (or Q S^T) for row block mb, k-step js holds row
 // 16 mb + i at k = 32 js + kap(g, e), two 8-byte reads at 16-byte chunks
 // (4 js + 2 h + (g >> 1)) ^ i, h = 0, 1 (row & 15 = i for every mb; mb adds
-// 16 rows = 4096 bytes)
-__device__ __forceinline__ void row_offsets(int g, int i, uint32_t (&ro)[8]) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-        ro[j] = i * 256 + 8 * (g & 1) + 16 * ((2 * j + (g >> 1)) ^ i);
+// 16 rows = 4096 bytes): this is chunk (g >> 1) ^ i, the others' addresses
+// differ from it by an exclusive or with 32 (2 js + h)
+__device__ __forceinline__ uint32_t row_offset(int g, int i) {
+    return i * 256 + 8 * (g & 1) + 16 * ((g >> 1) ^ i);
 }
-// stage base (scalar) + lane part, once a chunk: an opaque vector sum, so the
-// constant parts of each read (row block, K or Q, k step) stay in the LDS
-// instruction's offset field instead of each read adding its own base
+// Stage base (scalar) + lane part, once a chunk: opaque, so the constant parts
+// of each read (row block, k step, operand) stay in the LDS instruction's
+// offset field instead of each read forming its own address
 __device__ __forceinline__ uint32_t lane_addr(uint32_t sbase, uint32_t lane_part) {
     uint32_t r;
     asm("v_add_u32 %0, %1, %2" : "=v"(r) : "s"(sbase), "v"(lane_part));
     return r;
+}
+// the eight 16-byte chunks' addresses of a row or column offset (sbase a
+// multiple of 256): the loop holds one register of them, not eight
+__device__ __forceinline__ void lane_addrs(uint32_t sbase, uint32_t lane_part, uint32_t (&ra)[8]) {
+    ra[0] = lane_addr(sbase, lane_part);
+#pragma unroll
+    for (int j = 1; j < 8; ++j)
+        asm("v_xor_b32 %0, %1, %2" : "=v"(ra[j]) : "i"(32 * j), "v"(ra[0]));
 }
 __device__ __forceinline__ f16x8 row_frag(const uint32_t (&ra)[8], uint32_t off, int mb, int js) {
     const f16x4 a = *(volatile lds_f16x4*)(uintptr_t)(ra[2 * js] + off + 4096 * mb);
@@ -858,11 +880,9 @@ __device__ __forceinline__ f16x8 row_frag(const uint32_t (&ra)[8], uint32_t off,
 // i of the four rows). r & 15 = 4 g + i / 4 for both reads and every kq, so the
 // lane's part of the address is fixed per kb; kq and the second read add
 // 8192 and 4096 bytes.
-__device__ __forceinline__ void col_offsets(int g, int i, uint32_t (&co)[8]) {
+__device__ __forceinline__ uint32_t col_offset(int g, int i) {
     const int rr = 4 * g + (i >> 2);
-#pragma unroll
-    for (int kb = 0; kb < 8; ++kb)
-        co[kb] = rr * 256 + 16 * ((2 * kb + ((i & 3) >> 1)) ^ rr) + 8 * (i & 1);
+    return rr * 256 + 16 * (((i & 3) >> 1) ^ rr) + 8 * (i & 1);
 }
 __device__ __forceinline__ f16x8 col_frag(const uint32_t (&ca)[8], int kb, int kq) {
     const uint32_t a0 = ca[kb] + SA_K + 8192 * kq;
@@ -872,15 +892,28 @@ __device__ __forceinline__ f16x8 col_frag(const uint32_t (&ca)[8], int kb, int k
     return (f16x8){ah[0], ah[1], ah[2], ah[3], bh[0], bh[1], bh[2], bh[3]};
 }
 
+// A scheduling region's order: an LDS read behind each of the first R of its M
+// MFMAs (left alone, the reads gather at one end of the region, where they are
+// waited for or hold the MFMAs back)
+template <int R, int M>
+__device__ __forceinline__ void between_mfmas() {
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    if constexpr (M > R) __builtin_amdgcn_sched_group_barrier(0x8, M - R, 0);
+}
+
 // A state wave: 16 rows v0 .. v0 + 15 of the state, chunk after chunk.
 // Barriers (every wave of the workgroup passes the same sequence): E(-1),
-// then per chunk c: M(c-1) (the output wave has read the hand-over of c-1),
-// E(c) (the hand-over of c written; A stage c free for the copies of c + 2).
+// then per chunk c: M(c-1) (the output wave has read the hand-over of c-1; the
+// copies of A stage c + 1 and B stage c have landed), E(c) (the hand-over of c
+// written; A stage c free for the copies of c + 2).
 __device__ __forceinline__ void cs_state_wave(float* __restrict__ S, uint32_t lds0, int hv, int v0,
                                               int wa, int g, int i, int l, int n_chunks) {
-    uint32_t ro[8], co[8];
-    row_offsets(g, i, ro);
-    col_offsets(g, i, co);
+    const uint32_t ro = row_offset(g, i), co = col_offset(g, i);
+    const uint32_t vo = (4 * g + (i >> 2)) * (CS_ROWS * 2) + 32 * wa + 8 * (i & 3);
     // the state, st[kb][r] = S[v0 + i][16 kb + 4 g + r]: the result layout of
     // the 16 x 16 blocks of S^T
     float* Sv = S + ((size_t)hv * CK_V + v0 + i) * CK_K + 4 * g;
@@ -888,88 +921,85 @@ __device__ __forceinline__ void cs_state_wave(float* __restrict__ S, uint32_t ld
 #pragma unroll
     for (int kb8 = 0; kb8 < 8; ++kb8) st[kb8] = *(const f32x4*)(Sv + 16 * kb8);
     tile_done();   // E(-1): stages 0 and 1 landed
-    for (int c = 0; c < n_chunks; ++c) {
+    // Each phase's LDS operands are read a phase ahead, behind a scheduling
+    // fence, so no phase waits on LDS latency; X's K fragments, which do not
+    // wait for the state, ahead of the hand-over of the chunk before.
+    f16x8 kx[4][4];
+    auto read_k = [&](int c) {
         const uint32_t sb = lds0 + L_A + (c & 1) * SA_BYTES;
-        const uint32_t sg = sb + SA_G;
         uint32_t ra[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) ra[j] = lane_addr(sb, ro[j]);
-        // Each phase's LDS operands are read a phase ahead, behind a
-        // scheduling fence, so no phase waits on LDS latency. First X's K
-        // fragments, which do not wait for the state.
-        f16x8 kx[4][4];
+        lane_addrs(sb, ro, ra);
 #pragma unroll
         for (int js = 0; js < 4; ++js)
 #pragma unroll
             for (int mb = 0; mb < 4; ++mb) kx[js][mb] = row_frag(ra, SA_K, mb, js);
-        const f32x4 sc = *(lds_f32x4*)(uintptr_t)(sg + G_SC);   // e^{g_C}, 2^-tau, 2^-kappa
+    };
+    read_k(0);
+    float ms = 0.f;   // the lane's part of max |S| of row v0 + i
+#pragma unroll
+    for (int kb8 = 0; kb8 < 8; ++kb8)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ms = fmaxf(ms, fabsf(st[kb8][r]));
+    for (int c = 0; c < n_chunks; ++c) {
+        const uint32_t sb = lds0 + L_A + (c & 1) * SA_BYTES;
+        // e^{g_C} and 2^-tau
+        const float eg_c = *(const lds_f32w*)(uintptr_t)(sb + SA_G + G_SC);
+        const float t_un = *(const lds_f32w*)(uintptr_t)(sb + SA_G + G_SC + 4);
         __builtin_amdgcn_sched_barrier(0);
 
         // the state, scaled and split: B operands of the four k-steps
-        float ms = 0.f;
-#pragma unroll
-        for (int kb8 = 0; kb8 < 8; ++kb8)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) ms = fmaxf(ms, fabsf(st[kb8][r]));
         float s_inv;
         const float s_sc = pow2_scale<7>(col_max(ms), s_inv);
         f16x8 sh[4], sl[4];
-#pragma unroll
-        for (int js = 0; js < 4; ++js) split8(st[2 * js], st[2 * js + 1], s_sc, sh[js], sl[js]);
+        split8(st[0], st[1], s_sc, sh[0], sl[0]);
         __builtin_amdgcn_sched_barrier(0);
 
-        // Y's inputs and Q S^T's first fragments, then X = K S^T (two
-        // passes), 64 tokens x 16 rows, on four accumulators
+        // Y's inputs, then X = K S^T (two passes), 64 tokens x 16 rows, on four
+        // accumulators
+        const uint32_t va = lane_addr(sb, vo), ga = lane_addr(sb, 16 * g);
         f16x4 vv[4];
         f32x4 be[4], eg[4];
 #pragma unroll
         for (int mb = 0; mb < 4; ++mb) {
-            const int tok = 16 * mb + 4 * g;
-            const int vr = tok + (i >> 2);
             vv[mb] = __builtin_bit_cast(
                 f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(
-                           sb + SA_V + vr * (CS_ROWS * 2) + 32 * wa + 8 * (i & 3))));
-            be[mb] = *(lds_f32x4*)(uintptr_t)(sg + G_BETA + 4 * tok);
-            eg[mb] = *(lds_f32x4*)(uintptr_t)(sg + G_EG + 4 * tok);
+                           va + SA_V + 16 * CS_ROWS * 2 * mb)));
+            be[mb] = *(lds_f32x4*)(uintptr_t)(ga + SA_G + G_BETA + 64 * mb);
+            eg[mb] = *(lds_f32x4*)(uintptr_t)(ga + SA_G + G_EG + 64 * mb);
         }
-        f16x8 qa[2][4];
+        f32x4 x[4];
 #pragma unroll
-        for (int m2 = 0; m2 < 4; ++m2) qa[0][m2] = row_frag(ra, SA_Q, m2, 0);
-        f32x4 x[4], qs[4];
-#pragma unroll
-        for (int mb = 0; mb < 4; ++mb) x[mb] = qs[mb] = (f32x4)(0.f);
+        for (int mb = 0; mb < 4; ++mb) x[mb] = (f32x4)(0.f);
 #pragma unroll
         for (int js = 0; js < 4; ++js) {
+            if (js < 3) split8(st[2 * js + 2], st[2 * js + 3], s_sc, sh[js + 1], sl[js + 1]);
 #pragma unroll
             for (int mb = 0; mb < 4; ++mb) x[mb] = mfma16(kx[js][mb], sh[js], x[mb]);
 #pragma unroll
             for (int mb = 0; mb < 4; ++mb) x[mb] = mfma16(kx[js][mb], sl[js], x[mb]);
         }
+#pragma unroll
+        for (int j = 0; j < 24; ++j) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);
+            if (j >= 12) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x8, 8, 0);
         __builtin_amdgcn_sched_barrier(0);
 
-        // T's operands for Delta; then Q S^T, which only the output wave
-        // needs, issued between the blocks of Y = beta (V - e^g X) (tokens
-        // 16 mb + 4 g + r, column v0 + i), its next fragments read a k-step
-        // ahead
+        // T's operands for Delta; then Y = beta (V - e^g X) (tokens 16 mb + 4 g
+        // + r, column v0 + i)
+        const uint32_t ta = lane_addr(sb, 16 * l);
         f16x8 th[CK_NF], tl[CK_NF];
 #pragma unroll
         for (int f = 0; f < CK_NF; ++f) {
-            const uint32_t fo = (f * 64 + l) * 16;
-            th[f] = *(lds_f16x8*)(uintptr_t)(sb + SA_T + fo);
-            tl[f] = *(lds_f16x8*)(uintptr_t)(sb + SA_T + WS_OP + fo);
+            th[f] = *(lds_f16x8*)(uintptr_t)(ta + SA_T + 1024 * f);
+            tl[f] = *(lds_f16x8*)(uintptr_t)(ta + SA_T + WS_OP + 1024 * f);
         }
         f32x4 yv[4];
         float my = 0.f;
 #pragma unroll
         for (int mb = 0; mb < 4; ++mb) {
-            if (mb < 3) {
-#pragma unroll
-                for (int m2 = 0; m2 < 4; ++m2) qa[(mb + 1) & 1][m2] = row_frag(ra, SA_Q, m2, mb + 1);
-            }
-#pragma unroll
-            for (int m2 = 0; m2 < 4; ++m2) qs[m2] = mfma16(qa[mb & 1][m2], sh[mb], qs[m2]);
-#pragma unroll
-            for (int m2 = 0; m2 < 4; ++m2) qs[m2] = mfma16(qa[mb & 1][m2], sl[mb], qs[m2]);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 yv[mb][r] = be[mb][r] * fmaf(-(eg[mb][r] * s_inv), x[mb][r], (float)vv[mb][r]);
@@ -987,8 +1017,7 @@ __device__ __forceinline__ void cs_state_wave(float* __restrict__ S, uint32_t ld
         // Delta = T Y (three passes; T is zero above the diagonal, so rows
         // 0..31 take no columns 32..63)
         uint32_t ca[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) ca[j] = lane_addr(sb, co[j]);
+        lane_addrs(sb, co, ca);
         f16x8 kt[2][2][4];
 #pragma unroll
         for (int kq = 0; kq < 2; ++kq)
@@ -997,7 +1026,7 @@ __device__ __forceinline__ void cs_state_wave(float* __restrict__ S, uint32_t ld
         f32x4 dk[4];
 #pragma unroll
         for (int mb = 0; mb < 4; ++mb)
-            dk[mb] = *(lds_f32x4*)(uintptr_t)(sg + G_DK + 4 * (16 * mb + 4 * g));
+            dk[mb] = *(lds_f32x4*)(uintptr_t)(ga + SA_G + G_DK + 64 * mb);
         f32x4 dl[4];
 #pragma unroll
         for (int mb = 0; mb < 4; ++mb) dl[mb] = (f32x4)(0.f);
@@ -1016,6 +1045,7 @@ __device__ __forceinline__ void cs_state_wave(float* __restrict__ S, uint32_t ld
             const int mb = f_mb(f), kq = f_kq(f);
             dl[mb] = mfma16(tl[f], yh[kq], dl[mb]);
         }
+        between_mfmas<18, 18>();
         __builtin_amdgcn_sched_barrier(0);
 
         // the second half's K^T fragments; Delta' = e^{g_C - g} Delta for
@@ -1024,14 +1054,15 @@ __device__ __forceinline__ void cs_state_wave(float* __restrict__ S, uint32_t ld
         for (int kq = 0; kq < 2; ++kq)
 #pragma unroll
             for (int b = 0; b < 4; ++b) kt[1][kq][b] = col_frag(ca, 4 + b, kq);
-        const float d_un = sc[1] * y_inv;
+        __builtin_amdgcn_sched_barrier(0);
+        // (dl is Delta in T's and Y's scales, powers of two: 1 / d_un of it)
+        const float d_un = t_un * y_inv;
         float md = 0.f;
         f32x4 dp[4];
 #pragma unroll
         for (int mb = 0; mb < 4; ++mb) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                dl[mb][r] *= d_un;
                 dp[mb][r] = dk[mb][r] * dl[mb][r];
                 md = fmaxf(md, fabsf(dp[mb][r]));
             }
@@ -1041,54 +1072,87 @@ __device__ __forceinline__ void cs_state_wave(float* __restrict__ S, uint32_t ld
         f16x8 ph[2], pl[2];
 #pragma unroll
         for (int kq = 0; kq < 2; ++kq) split8(dp[2 * kq], dp[2 * kq + 1], p_sc, ph[kq], pl[kq]);
+        const float p_un = p_inv * d_un;
 
         // S^T = e^{g_C} S^T + K^T Delta' (K exact: two passes), in two halves
-        // of 4 k blocks
+        // of 4 k blocks, the first's sums formed between the second's MFMAs;
+        // the rows' next maximum with it
+        f32x4 u[2][4];
+        auto update_mfmas = [&](int h) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            f32x4 u[4];
-#pragma unroll
-            for (int b = 0; b < 4; ++b) u[b] = (f32x4)(0.f);
+            for (int b = 0; b < 4; ++b) u[h][b] = (f32x4)(0.f);
 #pragma unroll
             for (int kq = 0; kq < 2; ++kq) {
 #pragma unroll
-                for (int b = 0; b < 4; ++b) u[b] = mfma16(kt[h][kq][b], ph[kq], u[b]);
+                for (int b = 0; b < 4; ++b) u[h][b] = mfma16(kt[h][kq][b], ph[kq], u[h][b]);
 #pragma unroll
-                for (int b = 0; b < 4; ++b) u[b] = mfma16(kt[h][kq][b], pl[kq], u[b]);
+                for (int b = 0; b < 4; ++b) u[h][b] = mfma16(kt[h][kq][b], pl[kq], u[h][b]);
             }
+        };
+        ms = 0.f;
+        auto update_sums = [&](int h) {
 #pragma unroll
-            for (int b = 0; b < 4; ++b)
+            for (int b = 0; b < 4; ++b) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    st[4 * h + b][r] = fmaf(u[b][r], p_inv, sc[0] * st[4 * h + b][r]);
+                for (int r = 0; r < 4; ++r) {
+                    st[4 * h + b][r] = fmaf(u[h][b][r], p_un, st[4 * h + b][r]);
+                    ms = fmaxf(ms, fabsf(st[4 * h + b][r]));
+                }
+                // here, not past the barriers on the way to the next chunk
+                asm volatile("" : "+v"(st[4 * h + b]));
+            }
+        };
+#pragma unroll
+        for (int kb8 = 0; kb8 < 8; ++kb8) st[kb8] *= eg_c;
+        update_mfmas(0);
+        __builtin_amdgcn_sched_barrier(0);
+        update_mfmas(1);
+        update_sums(0);
+#pragma unroll
+        for (int j = 0; j < 12; ++j) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);
         }
+        __builtin_amdgcn_sched_group_barrier(0x8, 4, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        update_sums(1);
+        asm volatile("" : "+v"(ms));
         __builtin_amdgcn_sched_barrier(0);
 
-        // hand Q S0^T and Delta to the output wave (after it has read the
-        // previous chunk's)
+        // hand S0 and Delta to the output wave (after it has read the previous
+        // chunk's), the next chunk's K fragments on their way
         tile_done();   // M(c-1)
-        const uint32_t xo = lds0 + L_X + wa * X_WAVE + l * 16;
+        const uint32_t xo = lane_addr(lds0 + L_X + wa * X_WAVE, 16 * l);
 #pragma unroll
-        for (int mb = 0; mb < 4; ++mb) {
-            *(lds_f32x4w*)(uintptr_t)(xo + 1024 * mb) = qs[mb] * s_inv;
-            *(lds_f32x4w*)(uintptr_t)(xo + 1024 * (4 + mb)) = dl[mb];
+        for (int js = 0; js < 4; ++js) {
+            *(lds_f16x8w*)(uintptr_t)(xo + 1024 * js) = sh[js];
+            *(lds_f16x8w*)(uintptr_t)(xo + X_SL + 1024 * js) = sl[js];
+            *(lds_f32x4w*)(uintptr_t)(xo + X_DL + 1024 * js) = dl[js];
         }
-        tile_done();   // E(c)
+        *(lds_f32x2w*)(uintptr_t)(xo + X_SC) = (f32x2){s_inv, d_un};
+        asm volatile("" ::: "memory");
+        // LDS operations end in order: with 15 of the 32 reads left, the
+        // hand-over is written (a stage's reads are waited for ahead of M)
+        if (c + 1 < n_chunks) {
+            read_k(c + 1);
+            asm volatile("s_waitcnt lgkmcnt(15)\n\ts_barrier" ::: "memory");   // E(c)
+        } else {
+            tile_done();   // E(c)
+        }
     }
+    // (the lane's part anew: the loop has no register left for it)
+    const int le = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    float* Se = S + ((size_t)hv * CK_V + v0) * CK_K + (le & 15) * CK_K + 4 * (le >> 4);
 #pragma unroll
-    for (int kb8 = 0; kb8 < 8; ++kb8) *(f32x4*)(Sv + 16 * kb8) = st[kb8];
+    for (int kb8 = 0; kb8 < 8; ++kb8) *(f32x4*)(Se + 16 * kb8) = st[kb8];
 }
 
-// An output wave: the paired state wave's rows, a chunk behind it. y at token
-// t = 16 mb + 4 g + r, row v0 + i: O = e^g Q S0^T + (M o QK^T) Delta (three
-// passes), accumulated scaled by 2^(kappa + eps). Barriers: E(-1), M(-1), then
-// per chunk c: E(c), and M(c) but for the last chunk.
-__device__ __forceinline__ void cs_output_wave(const f16* q, const f16* k, const f16* v,
-                                               f16* __restrict__ y, const char* work,
-                                               uint32_t lds0, int T, int n_vheads, int hv, int hk,
-                                               int vw0, int v0, int wb, int g, int i, int l,
-                                               int n_chunks, int qk_bytes, int v_bytes,
-                                               int y_stride, float out_scale) {
+// A copy wave. Barriers as the state waves'; every copy of an iteration has
+// landed before its M.
+__device__ __forceinline__ void cs_copy_wave(const f16* q, const f16* k, const f16* v,
+                                             const char* work, uint32_t lds0, int T, int n_vheads,
+                                             int hv, int hk, int vw0, int wb, int l, int n_chunks,
+                                             int qk_bytes, int v_bytes) {
     const char* kb = uniform_ptr((const char*)(k + (size_t)hk * CK_K));
     const char* qb = uniform_ptr((const char*)(q + (size_t)hk * CK_K));
     const char* vb = uniform_ptr((const char*)(v + (size_t)hv * CK_V + vw0));
@@ -1097,31 +1161,71 @@ __device__ __forceinline__ void cs_output_wave(const f16* q, const f16* k, const
     };
     const CsOff off = cs_offsets(qk_bytes, v_bytes, wb, l);
     auto copy_a = [&](int c) {
-        cs_copy_a(lds0 + L_A + (c & 1) * SA_BYTES, kb, qb, vb, wblock(c), c * CK_C, T, qk_bytes,
+        cs_copy_a(lds0 + L_A + (c & 1) * SA_BYTES, kb, vb, wblock(c), c * CK_C, T, qk_bytes,
                   v_bytes, wb, l, off);
     };
-    auto copy_b = [&](int c) { cs_copy_b(lds0 + L_B + (c & 1) * SB_BYTES, wblock(c), wb, off); };
+    auto copy_b = [&](int c) {
+        cs_copy_b(lds0 + L_B + (c & 1) * SB_BYTES, qb, wblock(c), c * CK_C, T, qk_bytes, wb, l, off);
+    };
     copy_a(0);
     copy_b(0);
     if (n_chunks > 1) copy_a(1);
     WAIT_VMCNT(0);
     tile_done();   // E(-1)
     tile_done();   // M(-1)
+    for (int c = 0; c < n_chunks; ++c) {
+        tile_done();   // E(c): A stage c and B stage c - 1 are free
+        if (c + 2 < n_chunks) copy_a(c + 2);
+        if (c + 1 < n_chunks) {
+            copy_b(c + 1);
+            WAIT_VMCNT(0);
+            tile_done();   // M(c)
+        }
+    }
+}
+
+// An output wave: the paired state wave's rows, a chunk behind it. y at token
+// t = 16 mb + 4 g + r, row v0 + i: O = e^g Q S0^T (two passes, S split as the
+// state wave did) + (M o QK^T) Delta (three passes), accumulated scaled by
+// 2^(kappa + eps). Barriers: E(-1), M(-1), then per chunk c: E(c), and M(c) but
+// for the last chunk.
+__device__ __forceinline__ void cs_output_wave(f16* __restrict__ y, uint32_t lds0, int T, int hv,
+                                               int v0, int wb, int g, int i, int l, int n_chunks,
+                                               int y_stride, float out_scale) {
+    const uint32_t ro = row_offset(g, i);
+    tile_done();   // E(-1)
+    tile_done();   // M(-1)
     const uint32_t yt = lds0 + L_Y + wb * (CK_C * 32);
     for (int c = 0; c < n_chunks; ++c) {
-        // this wave's copies for chunk c (B stage) and c + 1 (A stage) landed;
-        // only this wave's y stores of chunk c - 1 were issued after them
-        WAIT_VMCNT(CS_NSTORE);
         tile_done();   // E(c)
-        if (c + 2 < n_chunks) copy_a(c + 2);
-        if (c + 1 < n_chunks) copy_b(c + 1);
         const uint32_t xo = lds0 + L_X + wb * X_WAVE + l * 16;
         const uint32_t sbb = lds0 + L_B + (c & 1) * SB_BYTES;
+        f16x8 sh[4], sl[4];
         f32x4 qs[4], dl[4];
 #pragma unroll
+        for (int js = 0; js < 4; ++js) {
+            sh[js] = *(lds_f16x8*)(uintptr_t)(xo + 1024 * js);
+            sl[js] = *(lds_f16x8*)(uintptr_t)(xo + X_SL + 1024 * js);
+            dl[js] = *(lds_f32x4*)(uintptr_t)(xo + X_DL + 1024 * js);
+            qs[js] = (f32x4)(0.f);
+        }
+        const f32x2 un = *(const lds_f32x2w*)(uintptr_t)(xo + X_SC);
+        uint32_t ra[8];
+        lane_addrs(sbb, ro, ra);
+#pragma unroll
+        for (int js = 0; js < 4; ++js) {
+            f16x8 qa[4];
+#pragma unroll
+            for (int mb = 0; mb < 4; ++mb) qa[mb] = row_frag(ra, SB_Q, mb, js);
+#pragma unroll
+            for (int mb = 0; mb < 4; ++mb) qs[mb] = mfma16(qa[mb], sh[js], qs[mb]);
+#pragma unroll
+            for (int mb = 0; mb < 4; ++mb) qs[mb] = mfma16(qa[mb], sl[js], qs[mb]);
+        }
+#pragma unroll
         for (int mb = 0; mb < 4; ++mb) {
-            qs[mb] = *(lds_f32x4*)(uintptr_t)(xo + 1024 * mb);
-            dl[mb] = *(lds_f32x4*)(uintptr_t)(xo + 1024 * (4 + mb));
+            qs[mb] *= un[0];
+            dl[mb] *= un[1];
         }
         const f32x4 sc = *(lds_f32x4*)(uintptr_t)(sbb + SB_G + G_SC);
         float mo = 0.f;
@@ -1157,8 +1261,8 @@ __device__ __forceinline__ void cs_output_wave(const f16* q, const f16* k, const
 #pragma unroll
         for (int f = 0; f < CK_NF; ++f) {
             const uint32_t fo = (f * 64 + l) * 16;
-            qh[f] = *(lds_f16x8*)(uintptr_t)(sbb + SB_Q + fo);
-            ql[f] = *(lds_f16x8*)(uintptr_t)(sbb + SB_Q + WS_OP + fo);
+            qh[f] = *(lds_f16x8*)(uintptr_t)(sbb + SB_M + fo);
+            ql[f] = *(lds_f16x8*)(uintptr_t)(sbb + SB_M + WS_OP + fo);
         }
 #pragma unroll
         for (int f = 0; f < CK_NF; ++f) o[f_mb(f)] = mfma16(qh[f], oh[f_kq(f)], o[f_mb(f)]);
@@ -1187,12 +1291,12 @@ __device__ __forceinline__ void cs_output_wave(const f16* q, const f16* k, const
     }
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+__global__ void __launch_bounds__(CS_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 chunk_state_kernel(const f16* __restrict__ q, const f16* __restrict__ k,
                    const f16* __restrict__ v, float* __restrict__ S, f16* __restrict__ y, int T,
                    int n_vheads, int qk_stride, int v_stride, int y_stride, float out_scale,
                    int group, const char* __restrict__ work) {
-    extern __shared__ __attribute__((aligned(16))) char smem[];
+    extern __shared__ __attribute__((aligned(256))) char cs_smem[];
     // a v head's workgroups are n_vheads apart in the flat id, so with
     // n_vheads a multiple of 8 (48 here) they land on one XCD (dispatch goes
     // round robin over the 8) and share its L2
@@ -1201,13 +1305,16 @@ chunk_state_kernel(const f16* __restrict__ q, const f16* __restrict__ k,
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = l >> 4, i = l & 15;
     const int vw0 = part * CS_ROWS;
-    const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) char*)smem);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) char*)cs_smem);
     const int n_chunks = (T + CK_C - 1) / CK_C;
     if (w < 2)
         cs_state_wave(S, lds0, hv, vw0 + 16 * w, w, g, i, l, n_chunks);
-    else
-        cs_output_wave(q, k, v, y, work, lds0, T, n_vheads, hv, hk, vw0, vw0 + 16 * (w - 2),
-                       w - 2, g, i, l, n_chunks, 2 * qk_stride, 2 * v_stride, y_stride, out_scale);
+    else if (w < 4)
+        cs_output_wave(y, lds0, T, hv, vw0 + 16 * (w - 2), w - 2, g, i, l, n_chunks, y_stride,
+                       out_scale);
+    else if (w >= 6)
+        cs_copy_wave(q, k, v, work, lds0, T, n_vheads, hv, hk, vw0, w - 6, l, n_chunks,
+                     2 * qk_stride, 2 * v_stride);
 }
 
 // The front kernel's and the state pass's dynamic LDS is above the 64 KiB
@@ -1255,7 +1362,7 @@ int launch_state(const void* q, const void* k, const void* v, float* S, void* y,
                  int group, const void* work, fl_stream_t stream) {
     const int rc = raise_lds_limit();
     if (rc) return rc;
-    hipLaunchKernelGGL(chunk_state_kernel, dim3(n_vheads * (CK_V / CS_ROWS)), dim3(256),
+    hipLaunchKernelGGL(chunk_state_kernel, dim3(n_vheads * (CK_V / CS_ROWS)), dim3(CS_THREADS),
                        CS_LDS, (hipStream_t)stream, (const f16*)q, (const f16*)k, (const f16*)v, S,
                        (f16*)y, T, n_vheads, qk_stride, v_stride, y_stride, out_scale, group,
                        (const char*)work);
