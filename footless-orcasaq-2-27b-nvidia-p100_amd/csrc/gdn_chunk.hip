@@ -727,11 +727,13 @@ gdn_front_kernel(const f16* __restrict__ x, const f16* __restrict__ conv_w,
 // takes, so what is not part of it lies elsewhere, and within it the VALU work
 // that a product does not wait for lies between the MFMAs of another: 42 -> 37.5
 // us for 1024 tokens of 48 heads, with the output waves issuing the copies and
-// the state waves forming Q S^T -> as here (4900 clocks a chunk).
+// the state waves forming Q S^T -> as here. (Measured and slower by 1 us: the
+// hand-over written between X's MFMAs, or behind Delta, with M before it. Its
+// 25 KB then meet the K reads and the y tiles in the LDS.)
 // ---------------------------------------------------------------------------
 constexpr int CS_ROWS = 32;   // state rows (v) a workgroup
 // A stage (the state waves' operands of a chunk): K rows [64][256 B] (16-byte
-// chunk c of row r at c ^ (r & 15)), V columns [64][CS_ROWS] fp16, T's hi / lo
+// chunk c of row r at c ^ row_swz(r)), V columns [64][CS_ROWS] fp16, T's hi / lo
 // operands and the gates KiB (as in the workspace)
 constexpr int SA_K = 0, SA_V = 16384, SA_T = SA_V + CK_C * CS_ROWS * 2,
               SA_G = SA_T + 2 * WS_OP, SA_BYTES = SA_G + 1024;
@@ -768,13 +770,17 @@ typedef __attribute__((address_space(3))) f16 lds_f16w;
 // (lane % 16) ^ (row & 15), row & 15 = rr + 8 (j & 1); V copy n rows
 // 16 n + lane / 4, 16 bytes (lane % 4) of the workgroup's 64-byte slice; a
 // workspace copy 16 bytes a lane.
+// (rows 4 g .. 4 g + 3 and chunks 4 js .. 4 js + 3 fall on 16 different chunks,
+// as do the rows 0 .. 15 of any one chunk)
+__device__ __forceinline__ int row_swz(int r) { return 4 * (r & 3) + ((r >> 2) & 3); }
+
 struct CsOff {
     uint32_t kq[2], v, w;
 };
 __device__ __forceinline__ CsOff cs_offsets(int qk_bytes, int v_bytes, int wb, int lane) {
     const int rr = 4 * wb + (lane >> 4), p = lane & 15;
-    return {{(uint32_t)(rr * qk_bytes + 16 * (p ^ rr)),
-             (uint32_t)(rr * qk_bytes + 16 * (p ^ (rr + 8)))},
+    return {{(uint32_t)(rr * qk_bytes + 16 * (p ^ row_swz(rr))),
+             (uint32_t)(rr * qk_bytes + 16 * (p ^ row_swz(rr + 8)))},
             (uint32_t)((lane >> 2) * v_bytes + 16 * (lane & 3)), (uint32_t)(16 * lane)};
 }
 
@@ -793,7 +799,7 @@ __device__ __forceinline__ void cs_copy_rows(uint32_t dst, const char* base, int
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int r = 8 * j + rr;
-            copy16_v(base + (size_t)(t0 + min(r, last)) * qk_bytes + 16 * (p ^ (r & 15)),
+            copy16_v(base + (size_t)(t0 + min(r, last)) * qk_bytes + 16 * (p ^ row_swz(r)),
                      __builtin_amdgcn_readfirstlane(dst + 1024 * (2 * j + wb)));
         }
     }
@@ -842,14 +848,19 @@ __device__ __forceinline__ void cs_copy_b(uint32_t dst, const char* qb, const ch
     if (wb == 1) copy16(wk + WS_BETA, o.w, dst + SB_G);
 }
 
+// The state's k axis is held in another order than the tokens': block 2 js + h
+// holds, in its row 4 g + r, k = 32 js + 8 g + 4 h + r. A k-step's B operand
+// (blocks 2 js and 2 js + 1) then pairs with eight consecutive k of a K or Q
+// row, one 16-byte read where kap's order takes two of 8 bytes (the LDS is a
+// bound beside the chain: a chunk moves 280 KB through it). 37.5 -> 36 us for
+// 1024 tokens of 48 heads.
+//
 // The lane's part of the swizzled K / Q row addresses, fixed for the kernel:
 // the A operand of X = K S^T (or Q S^T) for row block mb, k-step js holds row
-// 16 mb + i at k = 32 js + kap(g, e), two 8-byte reads at 16-byte chunks
-// (4 js + 2 h + (g >> 1)) ^ i, h = 0, 1 (row & 15 = i for every mb; mb adds
-// 16 rows = 4096 bytes): this is chunk (g >> 1) ^ i, the others' addresses
-// differ from it by an exclusive or with 32 (2 js + h)
+// 16 mb + i's 16-byte chunk 4 js + g (mb adds 16 rows = 4096 bytes): this is
+// chunk g's, the others' differ from it by an exclusive or with 64 js
 __device__ __forceinline__ uint32_t row_offset(int g, int i) {
-    return i * 256 + 8 * (g & 1) + 16 * ((g >> 1) ^ i);
+    return i * 256 + 16 * (g ^ row_swz(i));
 }
 // Stage base (scalar) + lane part, once a chunk: opaque, so the constant parts
 // of each read (row block, k step, operand) stay in the LDS instruction's
@@ -859,33 +870,31 @@ __device__ __forceinline__ uint32_t lane_addr(uint32_t sbase, uint32_t lane_part
     asm("v_add_u32 %0, %1, %2" : "=v"(r) : "s"(sbase), "v"(lane_part));
     return r;
 }
-// the eight 16-byte chunks' addresses of a row or column offset (sbase a
-// multiple of 256): the loop holds one register of them, not eight
-__device__ __forceinline__ void lane_addrs(uint32_t sbase, uint32_t lane_part, uint32_t (&ra)[8]) {
+// the four k-steps' addresses of a row or column offset (sbase a multiple of
+// 256): the loop holds one register of them, not four
+__device__ __forceinline__ void lane_addrs(uint32_t sbase, uint32_t lane_part, uint32_t (&ra)[4]) {
     ra[0] = lane_addr(sbase, lane_part);
 #pragma unroll
-    for (int j = 1; j < 8; ++j)
-        asm("v_xor_b32 %0, %1, %2" : "=v"(ra[j]) : "i"(32 * j), "v"(ra[0]));
+    for (int j = 1; j < 4; ++j)
+        asm("v_xor_b32 %0, %1, %2" : "=v"(ra[j]) : "i"(64 * j), "v"(ra[0]));
 }
-__device__ __forceinline__ f16x8 row_frag(const uint32_t (&ra)[8], uint32_t off, int mb, int js) {
-    const f16x4 a = *(volatile lds_f16x4*)(uintptr_t)(ra[2 * js] + off + 4096 * mb);
-    const f16x4 b = *(volatile lds_f16x4*)(uintptr_t)(ra[2 * js + 1] + off + 4096 * mb);
-    return (f16x8){a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+__device__ __forceinline__ f16x8 row_frag(const uint32_t (&ra)[4], uint32_t off, int mb, int js) {
+    return *(lds_f16x8*)(uintptr_t)(ra[js] + off + 4096 * mb);
 }
 
-// A operand of K^T Delta' for k rows 16 kb .., token step kq: lane 16 g + i
-// gets K[32 kq + kap(g, e)][16 kb + i] by two transposed reads (each: the
-// group's 16 lanes read a 4-row x 16-column block, lane i addressing row
-// r = 32 kq + 4 g + i / 4 (+ 16), columns 4 (i % 4) .., and receiving column
-// i of the four rows). r & 15 = 4 g + i / 4 for both reads and every kq, so the
-// lane's part of the address is fixed per kb; kq and the second read add
-// 8192 and 4096 bytes.
+// A operand of K^T Delta' for block kb = 2 js + h of k rows, token step kq:
+// lane 16 g + i gets K[32 kq + kap(g, e)][the block's row i] by two transposed
+// reads (each: the group's 16 lanes read 4 rows x 16 columns, lane i addressing
+// row r = 32 kq + 4 g + i / 4 (+ 16), columns 32 js + 8 (i % 4) + 4 h .. + 3,
+// and receiving the block's column i of the four rows). r & 15 = 4 g + i / 4
+// for both reads and every kq, so the swizzled column part is fixed for the
+// lane; kq and the second read add 8192 and 4096 bytes.
 __device__ __forceinline__ uint32_t col_offset(int g, int i) {
     const int rr = 4 * g + (i >> 2);
-    return rr * 256 + 16 * (((i & 3) >> 1) ^ rr) + 8 * (i & 1);
+    return rr * 256 + 16 * ((i & 3) ^ row_swz(rr));
 }
-__device__ __forceinline__ f16x8 col_frag(const uint32_t (&ca)[8], int kb, int kq) {
-    const uint32_t a0 = ca[kb] + SA_K + 8192 * kq;
+__device__ __forceinline__ f16x8 col_frag(const uint32_t (&ca)[4], int kb, int kq) {
+    const uint32_t a0 = ca[kb >> 1] + SA_K + 8 * (kb & 1) + 8192 * kq;
     const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)a0);
     const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(a0 + 4096));
     const f16x4 ah = __builtin_bit_cast(f16x4, a), bh = __builtin_bit_cast(f16x4, b);
@@ -914,12 +923,13 @@ __device__ __forceinline__ void cs_state_wave(float* __restrict__ S, uint32_t ld
                                               int wa, int g, int i, int l, int n_chunks) {
     const uint32_t ro = row_offset(g, i), co = col_offset(g, i);
     const uint32_t vo = (4 * g + (i >> 2)) * (CS_ROWS * 2) + 32 * wa + 8 * (i & 3);
-    // the state, st[kb][r] = S[v0 + i][16 kb + 4 g + r]: the result layout of
-    // the 16 x 16 blocks of S^T
-    float* Sv = S + ((size_t)hv * CK_V + v0 + i) * CK_K + 4 * g;
+    // the state, st[2 js + h][r] = S[v0 + i][32 js + 8 g + 4 h + r]: the result
+    // layout of the 16 x 16 blocks of S^T
+    float* Sv = S + ((size_t)hv * CK_V + v0 + i) * CK_K + 8 * g;
     f32x4 st[8];
 #pragma unroll
-    for (int kb8 = 0; kb8 < 8; ++kb8) st[kb8] = *(const f32x4*)(Sv + 16 * kb8);
+    for (int kb8 = 0; kb8 < 8; ++kb8)
+        st[kb8] = *(const f32x4*)(Sv + 32 * (kb8 >> 1) + 4 * (kb8 & 1));
     tile_done();   // E(-1): stages 0 and 1 landed
     // Each phase's LDS operands are read a phase ahead, behind a scheduling
     // fence, so no phase waits on LDS latency; X's K fragments, which do not
@@ -927,7 +937,7 @@ __device__ __forceinline__ void cs_state_wave(float* __restrict__ S, uint32_t ld
     f16x8 kx[4][4];
     auto read_k = [&](int c) {
         const uint32_t sb = lds0 + L_A + (c & 1) * SA_BYTES;
-        uint32_t ra[8];
+        uint32_t ra[4];
         lane_addrs(sb, ro, ra);
 #pragma unroll
         for (int js = 0; js < 4; ++js)
@@ -970,21 +980,32 @@ __device__ __forceinline__ void cs_state_wave(float* __restrict__ S, uint32_t ld
         f32x4 x[4];
 #pragma unroll
         for (int mb = 0; mb < 4; ++mb) x[mb] = (f32x4)(0.f);
-#pragma unroll
-        for (int js = 0; js < 4; ++js) {
-            if (js < 3) split8(st[2 * js + 2], st[2 * js + 3], s_sc, sh[js + 1], sl[js + 1]);
+        auto x_mfmas = [&](int js) {
 #pragma unroll
             for (int mb = 0; mb < 4; ++mb) x[mb] = mfma16(kx[js][mb], sh[js], x[mb]);
 #pragma unroll
             for (int mb = 0; mb < 4; ++mb) x[mb] = mfma16(kx[js][mb], sl[js], x[mb]);
+        };
+#pragma unroll
+        for (int js = 0; js < 3; ++js) {
+            split8(st[2 * js + 2], st[2 * js + 3], s_sc, sh[js + 1], sl[js + 1]);
+            x_mfmas(js);
         }
 #pragma unroll
         for (int j = 0; j < 24; ++j) {
             __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            if (j < 12) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);
-            if (j >= 12) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
-        __builtin_amdgcn_sched_group_barrier(0x8, 8, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        x_mfmas(3);
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb) eg[mb] *= -s_inv;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);
+        }
         __builtin_amdgcn_sched_barrier(0);
 
         // T's operands for Delta; then Y = beta (V - e^g X) (tokens 16 mb + 4 g
@@ -1002,7 +1023,7 @@ __device__ __forceinline__ void cs_state_wave(float* __restrict__ S, uint32_t ld
         for (int mb = 0; mb < 4; ++mb) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                yv[mb][r] = be[mb][r] * fmaf(-(eg[mb][r] * s_inv), x[mb][r], (float)vv[mb][r]);
+                yv[mb][r] = be[mb][r] * fmaf(eg[mb][r], x[mb][r], (float)vv[mb][r]);
                 my = fmaxf(my, fabsf(yv[mb][r]));
             }
         }
@@ -1016,7 +1037,7 @@ __device__ __forceinline__ void cs_state_wave(float* __restrict__ S, uint32_t ld
         // the state update's first K^T fragments and the decays; then
         // Delta = T Y (three passes; T is zero above the diagonal, so rows
         // 0..31 take no columns 32..63)
-        uint32_t ca[8];
+        uint32_t ca[4];
         lane_addrs(sb, co, ca);
         f16x8 kt[2][2][4];
 #pragma unroll
@@ -1131,7 +1152,7 @@ __device__ __forceinline__ void cs_state_wave(float* __restrict__ S, uint32_t ld
         }
         *(lds_f32x2w*)(uintptr_t)(xo + X_SC) = (f32x2){s_inv, d_un};
         asm volatile("" ::: "memory");
-        // LDS operations end in order: with 15 of the 32 reads left, the
+        // LDS operations end in order: with 15 of the 16 reads left, the
         // hand-over is written (a stage's reads are waited for ahead of M)
         if (c + 1 < n_chunks) {
             read_k(c + 1);
@@ -1142,9 +1163,10 @@ __device__ __forceinline__ void cs_state_wave(float* __restrict__ S, uint32_t ld
     }
     // (the lane's part anew: the loop has no register left for it)
     const int le = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-    float* Se = S + ((size_t)hv * CK_V + v0) * CK_K + (le & 15) * CK_K + 4 * (le >> 4);
+    float* Se = S + ((size_t)hv * CK_V + v0) * CK_K + (le & 15) * CK_K + 8 * (le >> 4);
 #pragma unroll
-    for (int kb8 = 0; kb8 < 8; ++kb8) *(f32x4*)(Se + 16 * kb8) = st[kb8];
+    for (int kb8 = 0; kb8 < 8; ++kb8)
+        *(f32x4*)(Se + 32 * (kb8 >> 1) + 4 * (kb8 & 1)) = st[kb8];
 }
 
 // A copy wave. Barriers as the state waves'; every copy of an iteration has
@@ -1210,7 +1232,7 @@ __device__ __forceinline__ void cs_output_wave(f16* __restrict__ y, uint32_t lds
             qs[js] = (f32x4)(0.f);
         }
         const f32x2 un = *(const lds_f32x2w*)(uintptr_t)(xo + X_SC);
-        uint32_t ra[8];
+        uint32_t ra[4];
         lane_addrs(sbb, ro, ra);
 #pragma unroll
         for (int js = 0; js < 4; ++js) {
