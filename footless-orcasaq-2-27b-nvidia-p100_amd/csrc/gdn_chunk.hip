@@ -764,16 +764,17 @@ typedef __attribute__((address_space(3))) f32x2 lds_f32x2w;
 typedef __attribute__((address_space(3))) float lds_f32w;
 typedef __attribute__((address_space(3))) f16 lds_f16w;
 
+// The 16-byte chunk swizzle of staged K and Q rows: rows 4 g .. 4 g + 3 and
+// chunks 4 js .. 4 js + 3 fall on 16 different chunks (the transposed reads), as
+// do the rows 0 .. 15 of any one chunk (the row reads)
+__device__ __forceinline__ int row_swz(int r) { return 4 * (r & 3) + ((r >> 2) & 3); }
+
 // Per-lane source offsets of copy wave wb's copies of a 64-token chunk (the
 // base is scalar): K / Q copy n (n = 2 j + wb) brings rows 4 n .. 4 n + 3,
 // lane -> row 8 j + rr, rr = 4 wb + lane / 16, and 16-byte chunk
-// (lane % 16) ^ (row & 15), row & 15 = rr + 8 (j & 1); V copy n rows
+// (lane % 16) ^ row_swz(row), row & 15 = rr + 8 (j & 1); V copy n rows
 // 16 n + lane / 4, 16 bytes (lane % 4) of the workgroup's 64-byte slice; a
 // workspace copy 16 bytes a lane.
-// (rows 4 g .. 4 g + 3 and chunks 4 js .. 4 js + 3 fall on 16 different chunks,
-// as do the rows 0 .. 15 of any one chunk)
-__device__ __forceinline__ int row_swz(int r) { return 4 * (r & 3) + ((r >> 2) & 3); }
-
 struct CsOff {
     uint32_t kq[2], v, w;
 };
