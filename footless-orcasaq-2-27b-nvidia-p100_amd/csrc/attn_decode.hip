@@ -186,30 +186,42 @@ struct DecTileRegs {
 // two waves. In DecTileRegs, lane l = 16 g + i:
 //   k[ks] = K[row 16 (w & 1) + i][128 (w >> 1) + 32 g + 8 ks + 0..7]
 //   v[i'] = V[row 16 (w & 1) + 4 (l & 3) + i'][128 (w >> 1) + 8 (l >> 2) + 0..7]
-// One int8 tile in flight: the same elements as bytes, plus one dword of
-// scales a lane -- rows 16 (w & 1) + (l & 15), blocks 4 (w >> 1) + 2 ((l >>
-// 4) & 1) + 0, 1; K for l < 32, V above.
+// One int8 tile in flight: the same elements as bytes. Its scales come through
+// LDS (DecScales).
 struct DecTileQ8 {
     u32x4 k[2];
     u32x2 v[4];
-    uint32_t sc;
 };
+
+// The scales of one int8 tile in LDS: the 32 rows of K, then the 32 rows of V,
+// 16 bytes (this head's 8 blocks) a row. A row's scales are 16 bytes of a
+// 64-byte sector, and every wave loading its own rows' scales touches each
+// sector twice a workgroup, a quarter of all the lines its loads touch: so a
+// wave loads all 64 rows' scales of every fourth tile instead, 16 bytes a lane,
+// and the workgroup shares them. Against a dword a lane of each wave's own rows
+// (same box, us): B = 4, T = 1 at ~8k 24.6 -> 23.4, T = 3 at ~8k / ~32k / ~100k
+// 27.6 / 73.3 / 202.5 -> 26.7 / 70 / 194, B = 6, T = 1 at ~60k 164.6 -> 158;
+// under the length rule (three workgroups a CU before, two now, by LDS) 27.5 /
+// 74.4 / 201.5 -> 26.9 / 71 / 200; the same bits.
+typedef f16 DecScales[2 * DEC_TILE][8];
+constexpr int DEC_SC_TILES = 4;   // tiles a group: one a wave
+
+__device__ __forceinline__ u32x4 dec_load_scales(const char* __restrict__ sc, uint32_t rs, int j,
+                                                 int uhi, int lane) {
+    const uint32_t row = (uint32_t)min(j * DEC_TILE + (lane & 31), uhi - 1);
+    return *(const u32x4*)(sc + row * (rs / 16));
+}
 
 template <bool NT_V>
 __device__ __forceinline__ void dec_load_tile(DecTileQ8& r, const char* __restrict__ kbase,
-                                              const char* __restrict__ vbase,
-                                              const f16* __restrict__ ksb,
-                                              const f16* __restrict__ vsb, size_t row_stride,
+                                              const char* __restrict__ vbase, size_t row_stride,
                                               int j, int uhi, int lane, int w) {
-    const int hh = lane >> 5;
     const uint32_t rs = (uint32_t)row_stride;   // bytes between rows; caches < 2 GiB
     const int r0 = j * DEC_TILE + 16 * (w & 1), cb = 128 * (w >> 1);
     const uint32_t krow = (uint32_t)min(r0 + (lane & 15), uhi - 1);
     const u32x4* src = (const u32x4*)(kbase + (krow * rs + cb + 32 * ((lane >> 4) & 3)));
     r.k[0] = src[0];
     r.k[1] = src[1];
-    const char* sb = (const char*)(hh ? vsb : ksb);
-    r.sc = *(const uint32_t*)(sb + (krow * (rs / 16) + 2 * (4 * (w >> 1) + 2 * ((lane >> 4) & 1))));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const uint32_t vrow = (uint32_t)min(r0 + 4 * (lane & 3) + i, uhi - 1);
@@ -219,13 +231,13 @@ __device__ __forceinline__ void dec_load_tile(DecTileQ8& r, const char* __restri
 }
 
 // The int8 tile as the fp16 tile the MFMAs read: fp16(byte * scale).
-__device__ __forceinline__ DecTileRegs dec_dequant(const DecTileQ8& q, int lane) {
+__device__ __forceinline__ DecTileRegs dec_dequant(const DecTileQ8& q, const DecScales& sc,
+                                                   int lane, int w) {
     DecTileRegs r;
-    // K: row (l & 15), block 4 (w >> 1) + l / 16 -- lane (l & 15) + 16 (l / 32)'s
-    // dword, half (l / 16) & 1; V row 4 (l & 3) + i, the same block -- lane 32 + that
-    const int bh = (lane >> 4) & 1, bl = 16 * (lane >> 5);
-    const uint32_t kp = (uint32_t)__builtin_amdgcn_ds_bpermute(((lane & 15) + bl) << 2, (int)q.sc);
-    const f16 ksh = __builtin_bit_cast(f16x2, kp)[bh];
+    // K row 16 (w & 1) + (l & 15), V rows 16 (w & 1) + 4 (l & 3) + i; block 4 (w
+    // >> 1) + l / 16 of both
+    const int r0 = 16 * (w & 1), blk = 4 * (w >> 1) + (lane >> 4);
+    const f16 ksh = sc[r0 + (lane & 15)][blk];
     const f16x2 ks2 = {ksh, ksh};
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
@@ -236,9 +248,7 @@ __device__ __forceinline__ DecTileRegs dec_dequant(const DecTileQ8& q, int lane)
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const uint32_t vp = (uint32_t)__builtin_amdgcn_ds_bpermute(
-            (32 + bl + 4 * (lane & 3) + i) << 2, (int)q.sc);
-        const f16 vsh = __builtin_bit_cast(f16x2, vp)[bh];
+        const f16 vsh = sc[DEC_TILE + r0 + 4 * (lane & 3) + i][blk];
         const f16x2 vs2 = {vsh, vsh};
         const f16x4 lo = q8_deq4(q.v[i].x, vs2);
         const f16x4 hi = q8_deq4(q.v[i].y, vs2);
@@ -369,6 +379,7 @@ attn_decode_split_kernel(const f16* __restrict__ qg, DecSeqs seqs, float* __rest
     __shared__ __attribute__((aligned(16))) f32x4 s_part[2][SP_W][4][64];
     __shared__ __attribute__((aligned(16))) f16 s_vt[Q8 ? 2 : 1][DEC_WAVES][64][VTP];
     __shared__ __attribute__((aligned(16))) char s_stage[STAGE ? NBUF * Q8_STAGE_B : 16];
+    __shared__ __attribute__((aligned(16))) DecScales s_sc[2][Q8 && !STAGE ? DEC_SC_TILES : 1];
 
     const int s = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -611,25 +622,50 @@ attn_decode_split_kernel(const f16* __restrict__ qg, DecSeqs seqs, float* __rest
         typedef typename std::conditional<Q8, DecTileQ8, DecTileRegs>::type Raw;
         auto load = [&](Raw& r, int j) {
             if constexpr (Q8)
-                dec_load_tile<NT_V>(r, kbase8, vbase8, ksb, vsb, row_stride, j, uhi, lane, w);
+                dec_load_tile<NT_V>(r, kbase8, vbase8, row_stride, j, uhi, lane, w);
             else
                 dec_load_tile<NT_V>(r, kbase, vbase, row_stride, j, uhi, lane, w);
         };
         const int j0 = ulo / DEC_TILE;
         const int j1 = (uhi + DEC_TILE - 1) / DEC_TILE;
         Raw rbuf[NBUF];
+        if constexpr (Q8) {
+            // Group g's scales (tiles j0 + 4 g .. + 3, tile 4 g + w from wave w)
+            // are loaded in tile 4 g - 4 and written to s_sc[g & 1] ahead of the
+            // barrier of tile 4 g - 2. Every wave has by then passed the barrier
+            // of tile 4 g - 3, so none still reads group g - 2 there (tile 4 g - 5
+            // at the latest), and reads group g only past that of tile 4 g - 1.
+            static_assert(DEC_SC_TILES % NBUF == 0 && DEC_SC_TILES == DEC_WAVES, "");
+            const char* sc = (const char*)(hh ? vsb : ksb);
+            u32x4 scales = dec_load_scales(sc, (uint32_t)row_stride, min(j0 + w, j1 - 1), uhi, lane);
 #pragma unroll
-        for (int p = 0; p < NBUF - 1; ++p) load(rbuf[p], min(j0 + p, j1 - 1));
-        for (int j = j0; j < j1; j += NBUF) {
+            for (int p = 0; p < NBUF - 1; ++p) load(rbuf[p], min(j0 + p, j1 - 1));
+            *(u32x4*)s_sc[0][w][lane] = scales;
+            lds_barrier();
+            int g = 0;
+            for (int j = j0; j < j1; j += DEC_SC_TILES) {
 #pragma unroll
-            for (int u = 0; u < NBUF; ++u) {
-                const int jj = j + u;
-                load(rbuf[(u + NBUF - 1) % NBUF], min(jj + NBUF - 1, j1 - 1));
-                if (jj < j1) {
-                    if constexpr (Q8)
-                        body(dec_dequant(rbuf[u], lane), jj, none, none);
-                    else
-                        body(rbuf[u], jj, none, none);
+                for (int u = 0; u < DEC_SC_TILES; ++u) {
+                    const int jj = j + u;
+                    if (u == 0)
+                        scales = dec_load_scales(sc, (uint32_t)row_stride,
+                                                 min(j + DEC_SC_TILES + w, j1 - 1), uhi, lane);
+                    load(rbuf[(u + NBUF - 1) % NBUF], min(jj + NBUF - 1, j1 - 1));
+                    if (jj < j1)
+                        body(dec_dequant(rbuf[u % NBUF], s_sc[g][u], lane, w), jj,
+                             [&] { if (u == 2) *(u32x4*)s_sc[g ^ 1][w][lane] = scales; }, none);
+                }
+                g ^= 1;
+            }
+        } else {
+#pragma unroll
+            for (int p = 0; p < NBUF - 1; ++p) load(rbuf[p], min(j0 + p, j1 - 1));
+            for (int j = j0; j < j1; j += NBUF) {
+#pragma unroll
+                for (int u = 0; u < NBUF; ++u) {
+                    const int jj = j + u;
+                    load(rbuf[(u + NBUF - 1) % NBUF], min(jj + NBUF - 1, j1 - 1));
+                    if (jj < j1) body(rbuf[u], jj, none, none);
                 }
             }
         }
@@ -901,9 +937,10 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 #define DEC_SPLIT_FLOOR 32
 #endif
 
-// int8 register tiles: 2 buffers (168 VGPRs, three waves a SIMD) -- in the
-// int8 layout 3 buffers (two waves a SIMD) measured 83.4 / 30.9 us at ~32k /
-// ~8k against 77.5 / 28.0, 4 and 5 slower still
+// int8 register tiles: 2 buffers -- in the int8 layout 3 buffers measured 83.4
+// / 30.9 us at ~32k / ~8k against 77.5 / 28.0, 4 and 5 slower still (with each
+// wave's own scale loads; two workgroups a CU are resident now, by the 60 KiB
+// of LDS with the shared scales)
 #ifndef DEC_NBUF_Q8
 #define DEC_NBUF_Q8 2
 #endif
@@ -914,7 +951,7 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 // per-sequence launches of attention_dec_q8 (112 workgroups, ~100k rows
 // each) 478 against 525 us a step for the register tiles; B = 1 at 4k-16k
 // within 3 % of them (12.2 at 4k either way); larger grids keep the register
-// tiles, whose workgroups (three a CU) overlap each other's barriers (B = 4,
+// tiles, whose workgroups (two a CU) overlap each other's barriers (B = 4,
 // T = 3 at ~8k / ~100k: 33.3 / 223 us against 34.4 / 235 staged, measured
 // before the int8 layout). Both give the same bits.
 constexpr int DEC_STAGE_MAX_WGS = 256;

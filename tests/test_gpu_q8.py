@@ -164,6 +164,35 @@ def test_decode_q8_batched_vs_single_and_oracle(fl, dev, orc, rng):
         assert ok, f"seq {b} L={L}: {err}"
 
 
+# tiles a split: 1 .. 9 (the register tiles' scales are loaded for four tiles at
+# a time), the last one ragged or whole
+@pytest.mark.parametrize("T", [1, 3])
+@pytest.mark.parametrize("lens", [[31, 64, 95, 127, 128, 5120, 6150, 18432],
+                                  [7200, 8191, 10245, 4, 97, 33, 3, 16500]])
+def test_decode_q8_tiles_a_split_batched_equals_single(fl, dev, T, lens):
+    """One batched launch (register tiles) against each sequence alone (at most
+    256 workgroups: the staged tiles), bit for bit, over rows whose blocks differ
+    in scale by up to 2^6."""
+    g = torch.Generator(device=dev).manual_seed(sum(lens))
+    ks, vs = [], []
+    for n in lens:
+        rows = [torch.randn((n, 4, 8, 32), generator=g, device=dev) for _ in range(2)]
+        rows = [(r * torch.exp2(torch.randint(-6, 1, (n, 4, 8, 1), generator=g, device=dev))).half()
+                for r in rows]
+        ks.append(fl.ops.kv8_cache(n))
+        vs.append(fl.ops.kv8_cache(n))
+        fl.ops.kv_store_q8(rows[0].view(n, 4, 256), rows[1].view(n, 4, 256), ks[-1], vs[-1],
+                           pos0=0, max_pos=n)
+    qg = torch.randn((len(lens), T, 24, 512), generator=g, device=dev).half()
+    pos0s, sr = [n - T for n in lens], fl.geometry.SPLIT_ROWS
+    zb = fl.ops.attn_decode_q8(qg, ks, vs, pos0s, lens, split_rows=sr)
+    assert torch.isfinite(zb.float()).all()
+    for b, n in enumerate(lens):
+        z1 = fl.ops.attn_decode_q8(qg[b:b + 1].contiguous(), [ks[b]], [vs[b]], [n - T], [n],
+                                   split_rows=sr)
+        assert torch.equal(zb[b], z1[0]), (b, n)
+
+
 @pytest.mark.parametrize("B,T,Lmax", [(4, 3, 8192), (4, 3, 32768), (4, 3, 102400),
                                       (1, 1, 102400)])
 def test_decode_q8_config2_vs_oracle(fl, dev, orc, B, T, Lmax):
