@@ -49,6 +49,7 @@
 //     p = 0, corr = 1), so a token's partial is the same bits whichever other
 //     tokens share the launch: a verify row equals the T = 1 call at its
 //     position (the reference asserts this, runtime.py:2062-2069).
+#include "attn_pieces.hpp"
 #include "fl_common.hpp"
 
 #include <mutex>
@@ -891,6 +892,74 @@ attn_merge_rows_kernel(const float* __restrict__ pacc, const float* __restrict__
     *(f16x4*)(z + (size_t)rh * z_pitch + 4 * c) = out;
 }
 
+// The merge of a prefill's piece list (attn_pieces.hpp), with the output gate
+// (attn_gate) when `gate` (the call's q | gate rows, the gate 256 halves into a
+// head's row) is given: one wavefront a (token, q head), lane l holding dims
+// 4 l .. 4 l + 3, its row tile's pieces in batches of eight against one running
+// max (attn_merge_rows_kernel's arithmetic). It stands here and not beside the
+// kernel that leaves the partials because that file is compiled without NaNs,
+// under which f16_sat stores a NaN as a finite number and sigmoid_f takes a NaN
+// gate for an open one: a NaN leaves every merge as a NaN.
+constexpr int SM_PAIRS = 4;   // (token, head) pairs a workgroup
+constexpr int SM_BATCH = 8;
+__global__ void __launch_bounds__(64 * SM_PAIRS)
+attn_piece_merge_kernel(const fl::StreamOut so, f16* __restrict__ z, int z_pitch,
+                        const f16* __restrict__ gate, int g_pitch, int n_q_heads, int G, int bins,
+                        int n_pairs, const fl::R64Plan plan) {
+    using fl::PF_HD;
+    using fl::R64_BQ;
+    const int lane = threadIdx.x & 63;
+    const int rh = __builtin_amdgcn_readfirstlane(blockIdx.x * SM_PAIRS + (threadIdx.x >> 6));
+    if (rh >= n_pairs) return;   // wave-uniform
+    const int t = rh / n_q_heads, head = rh - t * n_q_heads, h = head / G;
+    const int row = t * G + head - h * G;   // among its kv head's rows
+    const int tile = row / R64_BQ;
+    const fl::StreamAt sa = {plan.v, bins};
+    const int s0 = sa.slot0(tile), ns = sa.slot0(tile + 1) - s0;
+    f16x4 gv = {};
+    if (gate != nullptr) gv = *(const f16x4*)(gate + (size_t)rh * g_pitch + PF_HD + 4 * lane);
+    const size_t p0 = (size_t)(h * so.n + s0) * R64_BQ + (row - tile * R64_BQ);
+    const f32x4* acc = (const f32x4*)(so.pacc + p0 * PF_HD) + lane;
+    f32x4 num = (f32x4)(0.f);
+    float den = 0.f, M = -1e30f;
+    for (int s = 0; s < ns; s += SM_BATCH) {
+        float mv[SM_BATCH], dv[SM_BATCH];
+        f32x4 av[SM_BATCH];
+#pragma unroll
+        for (int u = 0; u < SM_BATCH; ++u) {
+            if (s + u >= ns) break;   // uniform: no load past the row's pieces
+            const size_t si = (size_t)(s + u) * R64_BQ;
+            mv[u] = so.pm[p0 + si];
+            dv[u] = so.pd[p0 + si];
+            av[u] = acc[si * (PF_HD / 4)];
+        }
+        float bm = M;
+#pragma unroll
+        for (int u = 0; u < SM_BATCH; ++u)
+            if (s + u < ns) bm = fmaxf(bm, mv[u]);
+        const float corr = fast_exp2((M - bm) * FL_LOG2E);
+        num *= corr;
+        den *= corr;
+        M = bm;
+#pragma unroll
+        for (int u = 0; u < SM_BATCH; ++u) {
+            if (s + u >= ns) break;
+            const float e = fast_exp2((mv[u] - M) * FL_LOG2E);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) num[d] = fmaf(e, av[u][d], num[d]);
+            den = fmaf(e, dv[u], den);
+        }
+    }
+    const float inv = 1.f / den;
+    f16x4 out;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        out[d] = f16_sat(num[d] * inv);
+        if (gate != nullptr) out[d] = f16_sat((float)out[d] * sigmoid_f((float)gv[d]));
+    }
+    *(f16x4*)(z + (size_t)rh * z_pitch + 4 * lane) = out;
+}
+
 // The output gate for layouts the 8-a-lane kernel below does not take (odd
 // head_dim, pitches or offsets, unaligned buffers): one wavefront a (token,
 // head) row, lane l taking elements l, l + 64, ... of it, with the same
@@ -1144,6 +1213,16 @@ int scratch_on_current_device(void** out) {
     return FL_OK;
 }
 }  // namespace
+
+int fl::launch_piece_merge(const StreamOut& so, const R64Plan& plan, int bins, void* z, int z_pitch,
+                           const void* gate, int g_pitch, int T, int n_q_heads, int G,
+                           hipStream_t stream) {
+    const int n_pairs = T * n_q_heads;
+    hipLaunchKernelGGL(attn_piece_merge_kernel, dim3((n_pairs + SM_PAIRS - 1) / SM_PAIRS),
+                       dim3(64 * SM_PAIRS), 0, stream, so, (f16*)z, z_pitch, (const f16*)gate,
+                       g_pitch, n_q_heads, G, bins, n_pairs, plan);
+    return check_launch("attn_piece_merge");
+}
 
 extern "C" {
 

@@ -35,6 +35,7 @@
 // the other stage, in the same swizzled layout, so the compute is the fp16
 // kernel's. The reference dequantizes V the same way; its K stays fp32
 // (byte * scale exact), here it is rounded to fp16 once.
+#include "attn_pieces.hpp"
 #include "fl_common.hpp"
 
 #include <algorithm>
@@ -44,13 +45,19 @@
 #include <queue>
 #include <vector>
 
+using fl::PF_HD;
+using fl::R64_BQ;
+using fl::R64_PLAN_MAX;
+using fl::R64Plan;
+using fl::StreamAt;
+using fl::StreamOut;
+
 namespace {
 
 constexpr int PF_WAVES = 4;
 constexpr int PF_THREADS = 64 * PF_WAVES;
 constexpr int PF_BQ = 32 * PF_WAVES;   // rows a workgroup
 constexpr int PF_BK = 64;              // kv rows a tile
-constexpr int PF_HD = 256;
 constexpr int ROW_B = PF_HD * 2;       // bytes a K / V row
 constexpr int TILE_B = PF_BK * ROW_B;  // 32 KiB
 constexpr int LDS_B = 4 * TILE_B;      // K stage 0 | K stage 1 | V stage 0 | V stage 1
@@ -535,7 +542,6 @@ __device__ __forceinline__ void copy16_at(const char* sbase, uint32_t voff, uint
 // lazy rescale, P rounded to fp16); 32-row tiles move the rescale points,
 // so the two kernels agree to rounding, not bit for bit.
 // ---------------------------------------------------------------------------
-constexpr int R64_BQ = 256;                 // rows a workgroup
 constexpr int R64_BK = 32;                  // kv rows a tile
 constexpr int R64_TILE = R64_BK * ROW_B;    // 16 KiB: K (or V) of a tile
 constexpr int R64_STAGE = 2 * R64_TILE;     // K | V
@@ -562,12 +568,7 @@ constexpr int R64_MIN_WGS = 384;
 // The host balances the bins (kv tiles walked + a fixed cost a row tile).
 // Plan layout: v[0 .. bins] = offsets of each bin's list in the row-tile
 // indices at v[bins + 1 ..].
-constexpr int R64_PLAN_MAX = 1024;     // bins + 1 + row tiles a kv head: 2 KiB of arguments
 constexpr int R64_ITEM_COST = 5;       // a row tile's fixed cost in kv tiles (Q, pipeline fill, z)
-struct R64Plan {
-    uint16_t v[R64_PLAN_MAX];
-};
-
 // Copy tile kv0 (K and V, 32 rows each) into the stage at dst: wave w copies
 // rows 8 w .. 8 w + 7, two a copy instruction (as issue_rows: loff[n] = this
 // lane's source offset from row 8 w, row 2 n + lane / 32, swizzled chunk).
@@ -650,35 +651,6 @@ __device__ __forceinline__ void r64_vfrags(s16x4 (&vb)[8], const char* vt,
     for (int i = 0; i < 8; ++i)
         vb[i] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vt + b[i] + imm));
 }
-
-// A call's work over one kv head as a list of pieces (STREAM): the row tiles'
-// causal walks laid end to end and cut into `bins` runs of equal cost, one a
-// workgroup, wherever the cuts fall. Bin b runs from tile start[b].tile, KV tile
-// start[b].j, up to start[b + 1]. Every piece leaves a partial, a row tile's in
-// slots slot0[tile] .. slot0[tile + 1] - 1 of its kv head in KV order (an uncut
-// tile's in its one slot: a second epilogue for it costs more registers than
-// the kernel has); `first[b]` is bin b's first piece's slot. v[]: start (2 (bins
-// + 1)), first (bins), slot0 (row tiles + 1).
-struct StreamAt {
-    const uint16_t* v;
-    int bins;
-    __device__ __forceinline__ int at(int i) const {   // (uniform)
-        return __builtin_amdgcn_readfirstlane((int)v[i]);
-    }
-    __device__ __forceinline__ int tile(int b) const { return at(2 * b); }
-    __device__ __forceinline__ int j(int b) const { return at(2 * b + 1); }
-    __device__ __forceinline__ int first(int b) const { return at(2 * (bins + 1) + b); }
-    __device__ __forceinline__ int slot0(int t) const { return at(3 * bins + 2 + t); }
-};
-// The partials of all kv heads: O unnormalised [slot][256 rows][256], then the
-// running max (natural-log units) and sum [slot][256 rows]; kv head h's slots
-// start at h * n.
-struct StreamOut {
-    float* pacc;
-    float* pm;
-    float* pd;
-    int n;   // slots a kv head (R64_PIECES), splits (R64_SPLIT)
-};
 
 // R64_ROWS: whole row tiles, bins > 0 the persistent plan's lists or bins == 0 a
 // grid of row tiles x kv heads, to z. R64_SPLIT: that grid with the uniform KV
@@ -933,69 +905,6 @@ attn_prefill_r64_kernel(const f16* __restrict__ q, int q_pitch, const f16* __res
                         z_sat(o[nb][mb][4 * r4 + 2] * inv), z_sat(o[nb][mb][4 * r4 + 3] * inv)};
         }
     }
-}
-
-// The merge of a piece list's partials, with the output gate (attn_gate) when
-// `gate` (the call's q | gate rows, the gate 256 halves into a head's row) is
-// given: one wavefront a (token, q head), lane l holding dims 4 l .. 4 l + 3,
-// its row tile's pieces in batches of eight against one running max
-// (attn_merge_rows_kernel's arithmetic).
-constexpr int SM_PAIRS = 4;   // (token, head) pairs a workgroup
-constexpr int SM_BATCH = 8;
-__global__ void __launch_bounds__(64 * SM_PAIRS)
-attn_prefill_stream_merge_kernel(const StreamOut so, f16* __restrict__ z, int z_pitch,
-                                 const f16* __restrict__ gate, int g_pitch, int n_q_heads, int G,
-                                 int bins, int n_pairs, const R64Plan plan) {
-    const int lane = threadIdx.x & 63;
-    const int rh = __builtin_amdgcn_readfirstlane(blockIdx.x * SM_PAIRS + (threadIdx.x >> 6));
-    if (rh >= n_pairs) return;   // wave-uniform
-    const int t = rh / n_q_heads, head = rh - t * n_q_heads, h = head / G;
-    const int row = t * G + head - h * G;   // among its kv head's rows
-    const int tile = row / R64_BQ;
-    const StreamAt sa = {plan.v, bins};
-    const int s0 = sa.slot0(tile), ns = sa.slot0(tile + 1) - s0;
-    f16x4 gv = {};
-    if (gate != nullptr) gv = *(const f16x4*)(gate + (size_t)rh * g_pitch + PF_HD + 4 * lane);
-    const size_t p0 = (size_t)(h * so.n + s0) * R64_BQ + (row - tile * R64_BQ);
-    const f32x4* acc = (const f32x4*)(so.pacc + p0 * PF_HD) + lane;
-    f32x4 num = (f32x4)(0.f);
-    float den = 0.f, M = -1e30f;
-    for (int s = 0; s < ns; s += SM_BATCH) {
-        float mv[SM_BATCH], dv[SM_BATCH];
-        f32x4 av[SM_BATCH];
-#pragma unroll
-        for (int u = 0; u < SM_BATCH; ++u) {
-            if (s + u >= ns) break;   // uniform: no load past the row's pieces
-            const size_t si = (size_t)(s + u) * R64_BQ;
-            mv[u] = so.pm[p0 + si];
-            dv[u] = so.pd[p0 + si];
-            av[u] = acc[si * (PF_HD / 4)];
-        }
-        float bm = M;
-#pragma unroll
-        for (int u = 0; u < SM_BATCH; ++u)
-            if (s + u < ns) bm = fmaxf(bm, mv[u]);
-        const float corr = fast_exp2((M - bm) * FL_LOG2E);
-        num *= corr;
-        den *= corr;
-        M = bm;
-#pragma unroll
-        for (int u = 0; u < SM_BATCH; ++u) {
-            if (s + u >= ns) break;
-            const float e = fast_exp2((mv[u] - M) * FL_LOG2E);
-#pragma unroll
-            for (int d = 0; d < 4; ++d) num[d] = fmaf(e, av[u][d], num[d]);
-            den = fmaf(e, dv[u], den);
-        }
-    }
-    const float inv = 1.f / den;
-    f16x4 out;
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-        out[d] = f16_sat(num[d] * inv);
-        if (gate != nullptr) out[d] = f16_sat((float)out[d] * sigmoid_f((float)gv[d]));
-    }
-    *(f16x4*)(z + (size_t)rh * z_pitch + 4 * lane) = out;
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
@@ -1663,12 +1572,8 @@ int prefill(const void* q, int q_pitch, const void* k_new, const void* v_new, vo
                            scale * FL_LOG2E, r64_tiles, sp_plan.bins, sp_plan.plan, so);
         rc = fl::check_launch("attn_prefill_r64 (pieces)");
         if (rc) return rc;
-        const int n_pairs = T * n_q_heads;
-        hipLaunchKernelGGL(attn_prefill_stream_merge_kernel,
-                           dim3((n_pairs + SM_PAIRS - 1) / SM_PAIRS), dim3(64 * SM_PAIRS), 0,
-                           (hipStream_t)stream_, so, (f16*)z, z_pitch, (const f16*)gate, q_pitch,
-                           n_q_heads, n_q_heads / n_kv_heads, sp_plan.bins, n_pairs, sp_plan.plan);
-        return fl::check_launch("attn_prefill merge (pieces)");
+        return fl::launch_piece_merge(so, sp_plan.plan, sp_plan.bins, z, z_pitch, gate, q_pitch, T,
+                                      n_q_heads, n_q_heads / n_kv_heads, (hipStream_t)stream_);
     }
     if (!Q8 && split == 1 && use_r64(T, n_q_heads, n_kv_heads)) {
         R64Plan plan;

@@ -650,3 +650,51 @@ def test_prefill_gated_equals_prefill_then_gate(fl, dev, kv8, T, pos0, split, sp
     torch.cuda.synchronize()
     assert torch.isfinite(zg.float()).all()
     assert torch.equal(zg, z), f"kv8={kv8} T={T} pos0={pos0} split={split}"
+
+
+# calls the equal runs take: fp16, and an int8 cache with its rows staged first
+@pytest.mark.parametrize("kv8,T,pos0", [(False, 777, 3001), (False, 16, 30000), (True, 1000, 1024)])
+def test_prefill_pieces_keep_nan(fl, dev, kv8, T, pos0):
+    """A NaN gate value, a NaN value row and a NaN query row leave a call left to
+    the library as NaN exactly where the uniform split leaves them (its merge
+    and attn_gate keep a NaN as the reference's f16_sat does), and the call
+    gated equals ungated then attn_gate."""
+    L = pos0 + T
+    g = torch.Generator(device=dev).manual_seed(T + pos0)
+    qg = torch.randn((T, 24, 512), generator=g, device=dev)
+    qg[..., :256] /= 16
+    qg = qg.half()
+    k = torch.randn((L, 4, 256), generator=g, device=dev).half()
+    v = torch.randn((L, 4, 256), generator=g, device=dev).half()
+    nan = float("nan")
+    qg[T // 2, 3, 256 + 17] = nan        # a gate value
+    qg[T - 2, 20, 5] = nan               # a query row: its z whole
+    if kv8:
+        k8, v8 = fl.ops.kv8_cache(L), fl.ops.kv8_cache(L)
+        fl.ops.kv_store_q8(k, v, k8, v8, pos0=0, max_pos=L)
+        # the scale of V row 7, kv head 1, dims 32 .. 63 (every query sees the row)
+        v8[L * 4 * 256:].view(torch.float16).view(L, 4, 8)[7, 1, 1] = nan
+
+        def run(**kw):
+            return fl.ops.attention_prefill_q8(qg, k8, v8, pos0=pos0, max_pos=L, scale=1.0, **kw)
+    else:
+        v[7, 1, 32:64] = nan
+
+        def run(**kw):
+            return fl.ops.attention_prefill(qg, k, v, pos0=pos0, scale=1.0, **kw)
+    need = fl._lib.lib().fl_attention_prefill_auto_work_bytes
+    assert need(T, pos0, 24, 4, 256, int(kv8)) > 0
+    z, zg, want, want_g = run(), run(gated=True), run(split=2), run(split=2, gated=True)
+    fl.ops.attn_gate(z, qg, T=T)
+    torch.cuda.synchronize()
+    expect = torch.zeros((T, 24, 256), dtype=torch.bool, device=dev)
+    expect[:, 6:12, 32:64] = True
+    expect[T - 2, 20] = True
+    assert torch.equal(torch.isnan(want), expect)
+    expect[T // 2, 3, 17] = True
+    for name, got in (("split 2", want_g), ("left to the library", zg), ("then the gate", z)):
+        assert torch.equal(torch.isnan(got), expect), name
+        assert torch.isfinite(got[~expect].float()).all(), name
+    assert torch.equal(zg[~expect], z[~expect])
+    err = (zg.float() - want_g.float())[~expect].abs()
+    assert not (err > ATOL + RTOL * want_g.float()[~expect].abs()).any(), float(err.max())
