@@ -74,6 +74,13 @@ def _contig(t: torch.Tensor, name: str):
         raise ValueError(f"{name}: must be contiguous")
 
 
+def _pitched(t: torch.Tensor, name: str, pitch: int):
+    """A view's rows have to lie the `pitch` elements apart that the call reads
+    them at: a column slice of a wider tensor passes every span check."""
+    if not t.is_contiguous() and (t.dim() < 2 or t.stride(0) != pitch or not t[0].is_contiguous()):
+        raise ValueError(f"{name}: rows not {pitch} elements apart")
+
+
 # ---------------------------------------------------------------------------
 # full attention
 # ---------------------------------------------------------------------------
@@ -695,9 +702,9 @@ def gdn_verify_normed(x, conv_w, st_in, st0, st1, st2, a, b, A_log, dt_bias, S, 
                       norm_eps: float = GDN_NORM_EPS):
     """A verify round's T = 2 or 3 rows of one sequence (runtime.py:3021-3065):
     conv1d_causal_rows, gdn_decode with the checkpoints (ck + t * ck_step) and
-    rmsnorm_gated in one call. x [T, x_stride] fp16 the raw q|k|v rows; st0 may
-    be st_in. Returns y [T, n_vheads, V] fp16."""
-    _contig(S, "S")
+    rmsnorm_gated in one call. x [T, x_stride] fp16 the raw q|k|v rows; a, b
+    [T, ab_stride] fp32; st0 may be st_in. Returns y [T, n_vheads, V] fp16."""
+    _contig(S, "S"), _pitched(a, "a", ab_stride), _pitched(b, "b", ab_stride)
     if y is None:
         y = torch.empty((T, n_vheads, V), dtype=F16, device=x.device)
     work = torch.empty_like(y)
@@ -783,9 +790,9 @@ def gdn_prefill_layer(x, conv_w, st_in, st_out, a, b, A_log, dt_bias, S, z, norm
                       l2eps: float = L2_EPS, norm_eps: float = GDN_NORM_EPS, work=None):
     """A GDN layer over a prompt's rows (runtime.py:3035-3111): conv1d_causal,
     l2norm_scaled of q and k, gdn_prefill_chunked_logits and rmsnorm_gated in one
-    call. x [T, x_stride] fp16 the raw q|k|v rows, z [T, n_vheads, V] fp16; S
-    and st_out are written. Returns y [T, n_vheads, V] fp16."""
-    _contig(S, "S")
+    call. x [T, x_stride] fp16 the raw q|k|v rows, a, b [T, ab_stride] fp32, z [T,
+    n_vheads, V] fp16; S and st_out are written. Returns y [T, n_vheads, V] fp16."""
+    _contig(S, "S"), _pitched(a, "a", ab_stride), _pitched(b, "b", ab_stride)
     if y is None:
         y = torch.empty((T, n_vheads, V), dtype=F16, device=x.device)
     dim = 2 * n_kheads * K + n_vheads * V

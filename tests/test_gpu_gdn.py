@@ -769,3 +769,40 @@ def test_verify_round_equals_separate_calls(fl, dev, rng, T, pos0):
     assert torch.equal(Sf, Su) and torch.equal(ckf, cku), "state or checkpoints differ"
     for t in range(3):
         assert torch.equal(f[t], u[t]), f"frames after row {t} differ"
+
+
+@pytest.mark.parametrize("entry,T", [("verify", 2), ("verify", 3), ("prefill", 5), ("prefill", 70)])
+def test_gate_logits_of_a_fused_projection(fl, dev, rng, entry, T):
+    """The gate logits as column slices of one [T, 96] projection: refused where
+    the call reads rows of 48, and the contiguous tensors' bits at their own
+    stride."""
+    x = to_dev((rng.standard_normal((T, ROW)) * 1.5).astype(np.float16), dev)
+    w = to_dev((rng.standard_normal((ROW, 4)) * 0.5).astype(np.float16), dev)
+    ab = to_dev(rng.standard_normal((T, 2 * NV)).astype(np.float32), dev)
+    A_log = to_dev((rng.standard_normal(NV) * 0.3).astype(np.float32), dev)
+    dt = to_dev((rng.standard_normal(NV) * 0.3).astype(np.float32), dev)
+    z = to_dev(rng.standard_normal((T, NV, 128)).astype(np.float16), dev)
+    nw = to_dev((1 + rng.standard_normal(128) * 0.2).astype(np.float32), dev)
+    st = to_dev(rng.standard_normal((ROW, 3)).astype(np.float16), dev)
+    S0 = to_dev((rng.standard_normal((NV, 128, 128)) * 0.05).astype(np.float32), dev)
+    state = NV * 128 * 128
+
+    def run(a, b, **kw):
+        S, s0, s1, s2 = S0.clone(), st.clone(), st.clone(), st.clone()
+        ck = torch.zeros((2, NV, 128, 128), device=dev)
+        if entry == "verify":
+            y = fl.ops.gdn_verify_normed(x, w, s0, s0, s1, s2, a, b, A_log, dt, S, ck, state, z, nw,
+                                         T=T, pos0=9, **kw)
+        else:
+            y = fl.ops.gdn_prefill_layer(x, w, s0, s1, a, b, A_log, dt, S, z, nw, T=T, pos0=9, **kw)
+        return y, S, ck, s0, s1, s2
+
+    a, b = ab[:, :NV], ab[:, NV:]
+    want = run(a.contiguous(), b.contiguous())
+    got = run(a, b, ab_stride=2 * NV)
+    torch.cuda.synchronize()
+    for i, (p, q) in enumerate(zip(got, want)):
+        assert torch.equal(p, q), i
+    for la, lb in ((a, b), (a.contiguous(), b), (a, b.contiguous())):
+        with pytest.raises(ValueError, match="elements apart"):
+            run(la, lb)
