@@ -1491,20 +1491,19 @@ int prefill(const void* q, int q_pitch, const void* k_new, const void* v_new, vo
     int n_cu = 0;
     int rc = prefill_device_setup(n_cu);
     if (rc) return rc;
-    // the library's own choice (split 0, or the count it gives out): a piece list
-    // where that is cheaper and its partials fit in `work`
-    const int policy = split_policy(T, pos0, n_q_heads, n_kv_heads, Q8);
+    // the library's own choice (split 0 alone: a count the caller asks for runs as
+    // that, whatever `work` holds): a piece list where that is cheaper and its
+    // partials fit in `work`
     AutoChoice c;
     c.stage = c.stream = false;
-    if (split == 0 || (split > 1 && split == policy))
-        auto_choice(T, pos0, n_q_heads, n_kv_heads, n_cu, Q8, c);
+    if (split == 0) auto_choice(T, pos0, n_q_heads, n_kv_heads, n_cu, Q8, c);
     const StreamPlan& sp_plan = c.sp;
     const size_t copy = c.stage ? q8_copy_bytes(T, pos0, n_kv_heads) : 0;
     const bool staged_auto = c.stage && work != nullptr && aligned16(work) &&
                              work_bytes >= copy + auto_f16_bytes(T, pos0, n_q_heads, n_kv_heads, c);
     const bool stream = !Q8 && c.stream && work != nullptr && aligned16(work) &&
                         work_bytes >= stream_work_bytes(sp_plan, n_kv_heads);
-    if (split == 0) split = policy;
+    if (split == 0) split = split_policy(T, pos0, n_q_heads, n_kv_heads, Q8);
     if (split > 1 && !stream && !staged_auto) {
         FL_REQUIRE(work != nullptr && aligned16(work), "16-byte aligned work for a split");
         if (work_bytes < split_work_bytes(T, n_q_heads, head_dim, split)) {

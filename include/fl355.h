@@ -290,9 +290,9 @@ size_t fl_attention_prefill_work_bytes(int T, int n_q_heads, int head_dim, int s
 /* The `work` bytes of a call that leaves its split to the library (split 0):
  * beside a uniform split, the row tiles' causal walks cut into equal runs, one
  * a CU, whose cut tiles leave partials that one merge combines (gate included).
- * A split 0 call, or one with the count that fl_attention_prefill_split_count
- * gives, takes that where it is cheaper and `work` holds these bytes, else the
- * uniform split (or none). q8: over an int8 cache. 0: no work needed. */
+ * A split 0 call takes that where it is cheaper and `work` holds these bytes,
+ * else the uniform split (or none); a split >= 1 is run as asked. q8: over an
+ * int8 cache. 0: no work needed. */
 size_t fl_attention_prefill_auto_work_bytes(int T, int pos0, int n_q_heads, int n_kv_heads,
                                             int head_dim, int q8);
 /* That cut for n_cu CUs, for tests and tuning (as fl_attention_prefill_plan):

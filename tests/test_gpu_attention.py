@@ -698,3 +698,40 @@ def test_prefill_pieces_keep_nan(fl, dev, kv8, T, pos0):
     assert torch.equal(zg[~expect], z[~expect])
     err = (zg.float() - want_g.float())[~expect].abs()
     assert not (err > ATOL + RTOL * want_g.float()[~expect].abs()).any(), float(err.max())
+
+
+@pytest.mark.parametrize("kv8,T,pos0", [(False, 683, 1024), (False, 512, 3072), (True, 1024, 8000)])
+def test_prefill_split_asked_for_is_run(fl, dev, kv8, T, pos0):
+    """A call that asks for the uniform split by its count gets it, the same bits
+    whether `work` holds that split's bytes alone or all that a call left to
+    the library would take."""
+    L = pos0 + T
+    g = torch.Generator(device=dev).manual_seed(L)
+    q = torch.randn((T, 24, 512), generator=g, device=dev).half()
+    k = torch.randn((L, 4, 256), generator=g, device=dev).half()
+    v = torch.randn((L, 4, 256), generator=g, device=dev).half()
+    lib = fl._lib.lib()
+    auto = int(lib.fl_attention_prefill_auto_work_bytes(T, pos0, 24, 4, 256, int(kv8)))
+    count = (fl.ops.prefill_split_count_q8 if kv8 else fl.ops.prefill_split_count)(T, pos0)
+    own = int(lib.fl_attention_prefill_work_bytes(T, 24, 256, count))
+    assert count > 1 and auto > 0
+    if kv8:
+        k8, v8 = fl.ops.kv8_cache(L), fl.ops.kv8_cache(L)
+        fl.ops.kv_store_q8(k, v, k8, v8, pos0=0, max_pos=L)
+
+    def run(split, nbytes, gated):
+        work = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        if kv8:
+            return fl.ops.attention_prefill_q8(q, k8, v8, pos0=pos0, max_pos=L, split=split,
+                                               work=work, gated=gated)
+        return fl.ops.attention_prefill(q, k, v, pos0=pos0, split=split, work=work, gated=gated)
+
+    for gated in (False, True):
+        want, got = run(count, own, gated), run(count, own + auto, gated)
+        left = run(None, own + auto, gated)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), gated
+        # the call left to the library adds the same values in another order
+        assert not torch.equal(left, want), gated
+        err = (left.float() - want.float()).abs()
+        assert not (err > ATOL + RTOL * want.float().abs()).any(), float(err.max())
