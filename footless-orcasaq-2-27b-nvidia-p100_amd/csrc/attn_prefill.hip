@@ -1361,7 +1361,15 @@ long long plain_cost(int T, int pos0, int n_q_heads, int n_kv_heads, int n_cu, b
 // gated, staged against the int8 kernel: T = 1024 from 0 59 / 71 us, 3072 133 /
 // 202, 30000 784 / 1139; T = 512 at 1024 54 / 64, 256 at 8000 90 / 106, 16 at
 // 30000 86 / 107; a short call over few rows stays (T = 16 at 3072: 33 staged, 26;
-// 64 at 1024: 32, 29), which Q8_STAGE_COST is set for.
+// 64 at 1024: 32, 29), which Q8_STAGE_COST is set for. An int8 cache is chosen
+// for its memory: a call whose copy and partials would pass Q8_STAGE_MAX_BYTES
+// keeps to the int8 kernel and its split's ~100 MB (1024 tokens at 98000 take
+// 608 MB, 2478 against 3535 us; the limit is met at ~200000 rows of 4 kv heads).
+constexpr size_t Q8_STAGE_MAX_BYTES = (size_t)1 << 30;
+size_t q8_copy_bytes(int T, int pos0, int n_kv_heads);
+struct AutoChoice;
+size_t auto_f16_bytes(int T, int pos0, int n_q_heads, int n_kv_heads, const AutoChoice& c);
+
 struct AutoChoice {
     bool stage, stream;
     StreamPlan sp;
@@ -1379,7 +1387,10 @@ void choose(int T, int pos0, int n_q_heads, int n_kv_heads, int n_cu, bool q8, A
     if (!q8) return;
     if (c.stream) cost = 10 * (long long)c.sp.cost;
     cost += Q8_STAGE_COST + (pos0 + (long long)T) * n_kv_heads / Q8_STAGE_ROWS;
-    c.stage = cost < plain_cost(T, pos0, n_q_heads, n_kv_heads, n_cu, true);
+    c.stage = cost < plain_cost(T, pos0, n_q_heads, n_kv_heads, n_cu, true) &&
+              q8_copy_bytes(T, pos0, n_kv_heads) +
+                      auto_f16_bytes(T, pos0, n_q_heads, n_kv_heads, c) <=
+                  Q8_STAGE_MAX_BYTES;
     c.stream = c.stream && c.stage;
 }
 

@@ -312,15 +312,26 @@ def prefill_split_count_q8(T: int, pos0: int, n_q_heads: int = N_HEADS,
 
 def _prefill_split(T, pos0, n_q_heads, n_kv_heads, head_dim, split, work, device, q8=False):
     """(split, work) of a prefill call: a split left to the library goes down as 0,
-    with the work its choice needs where none is given."""
+    with the work its choice needs where none is given. Where that cannot be
+    allocated (over an int8 cache it may hold an fp16 copy of the cached rows),
+    the library gets the uniform split's, and takes that."""
+    lib = _lib.lib()
+    if work is not None:
+        return (0 if split is None else split), work
     if split is None:
-        split = 0
-        if work is None:
-            need = int(_lib.lib().fl_attention_prefill_auto_work_bytes(
-                T, pos0, n_q_heads, n_kv_heads, head_dim, int(q8)))
-            work = torch.empty(need, dtype=torch.uint8, device=device) if need else None
-    elif split > 1 and work is None:
-        need = int(_lib.lib().fl_attention_prefill_work_bytes(T, n_q_heads, head_dim, split))
+        need = int(lib.fl_attention_prefill_auto_work_bytes(T, pos0, n_q_heads, n_kv_heads,
+                                                            head_dim, int(q8)))
+        try:
+            return 0, (torch.empty(need, dtype=torch.uint8, device=device) if need else None)
+        except torch.OutOfMemoryError:
+            count = (prefill_split_count_q8 if q8 else prefill_split_count)(T, pos0, n_q_heads,
+                                                                            n_kv_heads)
+            less = int(lib.fl_attention_prefill_work_bytes(T, n_q_heads, head_dim, count))
+            if less >= need:
+                raise
+            return 0, (torch.empty(less, dtype=torch.uint8, device=device) if less else None)
+    if split > 1:
+        need = int(lib.fl_attention_prefill_work_bytes(T, n_q_heads, head_dim, split))
         work = torch.empty(need, dtype=torch.uint8, device=device)
     return split, work
 
@@ -502,7 +513,8 @@ def attention_prefill_q8(q, kcache, vcache, *, pos0: int, max_pos: int, T: int |
     if split <= 1:
         stage = int(_lib.lib().fl_attention_prefill_q8_stage_bytes(T, pos0, n_q_heads, n_kv_heads,
                                                                    HEAD_DIM))
-    if stage > 0 and (work is None or work.numel() < stage):
+    # (split 0 without work: there was no room for the copy)
+    if stage > 0 and (split == 1 if work is None else work.numel() < stage):
         work = torch.empty(stage, dtype=torch.uint8, device=q.device)
     if gated:
         _prefill_gated(args, 1, split, zargs, work)

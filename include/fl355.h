@@ -292,7 +292,10 @@ size_t fl_attention_prefill_work_bytes(int T, int n_q_heads, int head_dim, int s
  * a CU, whose cut tiles leave partials that one merge combines (gate included).
  * A split 0 call takes that where it is cheaper and `work` holds these bytes,
  * else the uniform split (or none); a split >= 1 is run as asked. q8: over an
- * int8 cache. 0: no work needed. */
+ * int8 cache, where the bytes hold an fp16 copy of the rows [0, pos0 + T) when
+ * that pays (see fl_attention_prefill_kv_q8): 4 KiB a row at 4 kv heads, up to 1
+ * GiB with the partials for a chunk that would else split its KV range. A caller
+ * short of memory passes what the uniform split needs. 0: no work needed. */
 size_t fl_attention_prefill_auto_work_bytes(int T, int pos0, int n_q_heads, int n_kv_heads,
                                             int head_dim, int q8);
 /* That cut for n_cu CUs, for tests and tuning (as fl_attention_prefill_plan):

@@ -197,6 +197,36 @@ def test_prefill_split_policy(fl):
     assert lib.fl_attention_prefill_work_bytes(1024, 24, 256, 1) == 0
 
 
+def test_prefill_q8_staging_is_bounded(fl, monkeypatch):
+    """A chunk left to the library over an int8 cache takes an fp16 copy of the
+    cached rows up to 1 GiB of work, past that the int8 kernel's split; and where
+    its work cannot be allocated, the wrapper passes on the split's instead."""
+    import torch
+
+    lib = fl._lib.lib()
+    uniform = 1024 * 24 * lib.fl_attention_prefill_split_count_q8(1024, 98000, 24, 4) * 1032
+    staged = lib.fl_attention_prefill_auto_work_bytes(1024, 98000, 24, 4, 256, 1)
+    assert staged > 2 * 99024 * 4 * 256 * 2 > uniform
+    for T, pos0 in ((1024, 150000), (1024, 260000), (200, 262000), (16, 500000), (700, 10 ** 6)):
+        need = lib.fl_attention_prefill_auto_work_bytes(T, pos0, 24, 4, 256, 1)
+        count = lib.fl_attention_prefill_split_count_q8(T, pos0, 24, 4)
+        assert need <= 1 << 30, (T, pos0)
+        if (pos0 + T) * 4096 > 1 << 30:
+            assert need == lib.fl_attention_prefill_work_bytes(T, 24, 256, count), (T, pos0)
+
+    def full(n, **kw):
+        if n > uniform:
+            raise torch.OutOfMemoryError("full")
+        return ("work", n)
+
+    monkeypatch.setattr(torch, "empty", full)
+    args = (24, 4, 256, None, None, "cpu")
+    assert fl.ops._prefill_split(1024, 98000, *args, q8=True) == (0, ("work", uniform))
+    assert fl.ops._prefill_split(8192, 98000, *args, q8=True) == (0, None)   # staged, else whole
+    with pytest.raises(torch.OutOfMemoryError):   # nothing smaller to fall back to
+        fl.ops._prefill_split(1024, 98000, *args, q8=False)
+
+
 
 def _plan_weights(T, pos0, G):
     RT = T * G

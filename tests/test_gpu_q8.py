@@ -337,3 +337,37 @@ def test_prefill_q8_config3_sampled_rows(fl, dev, orc, L):
                                       scale=1.0, T=1)
         err, ok = close_rel(zh[t:t + 1], want, ATOL, RTOL)
         assert ok, f"L={L} row {t}: max|err| {err}"
+
+
+@pytest.mark.parametrize("T,pos0", [(1024, 8000), (4096, 512)])
+def test_prefill_without_room_for_the_staging_copy(fl, dev, monkeypatch, T, pos0):
+    """A prefill over an int8 cache whose fp16 staging copy cannot be allocated
+    (the allocator made to refuse it) runs the int8 kernel: the bits of its
+    uniform split, or of the unsplit call without work."""
+    L = pos0 + T
+    g = torch.Generator(device=dev).manual_seed(L)
+    q = torch.randn((T, 24, 512), generator=g, device=dev).half()
+    k = torch.randn((L, 4, 256), generator=g, device=dev).half()
+    v = torch.randn((L, 4, 256), generator=g, device=dev).half()
+    k8, v8 = fl.ops.kv8_cache(L), fl.ops.kv8_cache(L)
+    fl.ops.kv_store_q8(k, v, k8, v8, pos0=0, max_pos=L)
+    count = fl.ops.prefill_split_count_q8(T, pos0)
+    want = torch.empty((T, 24, 256), dtype=torch.float16, device=dev)
+    if count > 1:
+        fl.ops.attention_prefill_q8(q, k8, v8, pos0=pos0, max_pos=L, z=want, split=count)
+    else:
+        fl._lib.call("fl_attention_prefill_q8", q.data_ptr(), 512, None, None, k8.data_ptr(),
+                     v8.data_ptr(), 0, 24, 4, 256, pos0, L, fl.geometry.ATTN_SCALE, T,
+                     want.data_ptr(), 256, torch.cuda.current_stream().cuda_stream)
+    z = torch.empty_like(want)
+    room, empty = int(fl._lib.lib().fl_attention_prefill_work_bytes(T, 24, 256, count)), torch.empty
+
+    def full(*shape, **kw):
+        if kw.get("dtype") is torch.uint8 and shape[0] > room:
+            raise torch.OutOfMemoryError("full")
+        return empty(*shape, **kw)
+
+    monkeypatch.setattr(torch, "empty", full)
+    fl.ops.attention_prefill_q8(q, k8, v8, pos0=pos0, max_pos=L, z=z)
+    torch.cuda.synchronize()
+    assert torch.isfinite(want.float()).all() and torch.equal(z, want)
