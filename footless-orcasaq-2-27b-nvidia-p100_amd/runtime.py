@@ -462,6 +462,8 @@ class HybridRuntime:
                 qg, k, v = proj.full_attn_in(i, B)
                 lcaps = [st.lcap[li] for st in states]
                 spans = [kv8_nbytes(n) if kv8 else n * N_KV * HEAD_DIM for n in lcaps]
+                for st in states:
+                    ops._contig(st.kk[li], "kcache"), ops._contig(st.kv[li], "vcache")
                 kps = _lib.ptr_array([ops._ptr(st.kk[li], kv_type, "kcache", n)
                                       for st, n in zip(states, spans)])
                 vps = _lib.ptr_array([ops._ptr(st.kv[li], kv_type, "vcache", n)

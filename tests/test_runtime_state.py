@@ -138,3 +138,34 @@ def test_accept_verify_bookkeeping(T, kept):
     assert live == {1: 10.0, 2: 11.0, 3: 12.0}[kept]
     with pytest.raises(ValueError):                       # only once a verify
         rt.accept_verify(st, [7, 8, 9][:T], kept)
+
+
+@pytest.mark.parametrize("kv8", [False, True])
+@pytest.mark.parametrize("which", ["kk", "kv"])
+def test_decode_step_refuses_strided_caches(kv8, which):
+    """A decode step addresses a layer's cache rows from its first element: a
+    buffer put in its place that is not dense is refused, one sequence or a
+    batch."""
+    layers = ("full_attention",)
+    g = torch.Generator().manual_seed(0)
+
+    class Proj:
+        def full_attn_in(self, layer, T):
+            return (torch.randn((T, 24, 512), generator=g).half(), torch.zeros((T, 4, 256)).half(),
+                    torch.zeros((T, 4, 256)).half())
+
+        def layer_out(self, layer, out):
+            pass
+
+    rt = small_rt(kv8, layers)
+    st = rt.new_state()
+    rt.grow(st, 8)
+    cap = st.lcap[0]
+    if kv8:
+        getattr(st, which)[0] = torch.zeros(2 * st.kk[0].numel(), dtype=torch.int8)[::2]
+    else:
+        getattr(st, which)[0] = torch.zeros((4, cap, 256), dtype=torch.float16).transpose(0, 1)
+    with pytest.raises(ValueError, match="must be contiguous"):
+        rt.forward(st, Proj(), [1])
+    with pytest.raises(ValueError, match="must be contiguous"):
+        rt.forward_batch([st], Proj(), [1])
