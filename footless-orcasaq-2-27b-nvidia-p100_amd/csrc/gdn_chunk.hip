@@ -1478,6 +1478,10 @@ int fl_gdn_prefill_layer(const void* x, int x_stride, const void* conv_w, const 
     FL_REQUIRE(ab_stride >= n_vheads, "ab_stride >= n_vheads");
     FL_REQUIRE(st_in != st_out, "st_in and st_out must be distinct buffers");
     FL_REQUIRE(((uintptr_t)S & 15u) == 0 && ((uintptr_t)work & 15u) == 0, "16-byte aligned S, work");
+    // (the output norm's conditions, before anything is written)
+    FL_REQUIRE(((uintptr_t)z & 3u) == 0 && ((uintptr_t)y & 3u) == 0 &&
+                   ((uintptr_t)norm_w & 7u) == 0 && norm_eps >= 0.f,
+               "aligned z, y, norm_w; norm_eps >= 0");
     const size_t need = fl_gdn_prefill_layer_work_bytes(T, x_stride, n_vheads, K, V);
     if (work_bytes < need) {
         fl::set_error("work: %zu bytes, fl_gdn_prefill_layer_work_bytes asks %zu", work_bytes, need);

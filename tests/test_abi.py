@@ -176,6 +176,20 @@ def test_noalloc_decode_refuses_beyond_its_static_scratch(fl):
     assert b"static scratch" in lib.fl_last_error()
 
 
+@pytest.mark.parametrize("bad", ["z", "y", "norm_w", "norm_eps"])
+def test_prefill_layer_refuses_its_norm_up_front(fl, bad):
+    """The one-call GDN layer checks the output norm's conditions before its first
+    launch writes the state and the conv frames."""
+    p = {n: ctypes.c_void_p(0x1000 * (i + 1)) for i, n in enumerate(
+        ("x", "w", "in", "out", "a", "b", "A", "dt", "S", "z", "norm_w", "y", "work"))}
+    if bad in p:
+        p[bad] = ctypes.c_void_p(0x100002)   # never dereferenced
+    rc = _call(fl, "fl_gdn_prefill_layer", p["x"], 10240, p["w"], p["in"], p["out"], 0, p["a"],
+               p["b"], 48, p["A"], p["dt"], p["S"], p["z"], p["norm_w"], p["y"], 5, 16, 48, 128,
+               128, 0.088, 1e-6, -1.0 if bad == "norm_eps" else 1e-6, p["work"], 1 << 40, None)
+    assert rc == 1 and b"norm" in fl._lib.lib().fl_last_error()
+
+
 def test_prefill_split_policy(fl):
     """The KV split the prefill takes: none where the grid fills the CUs (an 8k
     or 2k fresh prompt, a 4k chunk deep in a prompt: the 64-rows-a-wave kernel
