@@ -518,6 +518,14 @@ chunk_prep_kernel(const f16* __restrict__ q, const f16* __restrict__ k, const Pr
 constexpr int FG = 3;                        // v heads a k head
 constexpr int FR_THREADS = 256 * FG;
 constexpr int FR_TB = 4;                     // tokens a conv task
+// The front kernel from this many workgroups up. One takes its ~20 us however
+// few there are (a workgroup's own chain), while the three launches that it
+// replaces spread a short call over more of the chip. Same box, both sides, four
+// layers of 16 k heads, us, front / separate: 1 chunk 108 / 82, 2 (32
+// workgroups) 128 / 114, 5 (80) 166 / 163, 6 (96) 173 / 177, 8 (128) 186 / 201, 16
+// (256) 259 / 306; a layer of 8 k heads at 80 workgroups 50.5 / 49.5, 96 53.5 /
+// 54.5; of 32 at 64 43.5 / 42.3, 96 47.5 / 51.3.
+constexpr int FR_MIN_WGS = 96;
 constexpr int FR_TILE = CK_C * PK_P * 2;     // staged K or Q rows; A or M o QK^T of a team
 constexpr int FR_LDS = 2 * FR_TILE + FG * 2 * FR_TILE + FG * (2 * CK_C + 8) * 4;
 static_assert(FR_LDS <= 160 * 1024, "the front kernel's LDS fits 160 KiB");
@@ -1498,12 +1506,13 @@ int fl_gdn_prefill_layer(const void* x, int x_stride, const void* conv_w, const 
     auto al16 = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
     int rc;
     // the one-launch front takes the model's three v heads a k head with 16-byte
-    // rows; anything else the conv and norm kernels, then the chunked scan's
-    // own prep
-    if (group == FG && al16(x) && al16(conv_w) && al16(st_in) && al16(st_out)) {
+    // rows and enough chunks; anything else the conv and norm kernels, then the
+    // chunked scan's own prep
+    const int n_chunks = (T + CK_C - 1) / CK_C;
+    if (group == FG && (long long)n_chunks * n_kheads >= FR_MIN_WGS && al16(x) && al16(conv_w) &&
+        al16(st_in) && al16(st_out)) {
         rc = raise_lds_limit();
         if (rc) return rc;
-        const int n_chunks = (T + CK_C - 1) / CK_C;
         hipLaunchKernelGGL(gdn_front_kernel, dim3(n_chunks, n_kheads), dim3(FR_THREADS), FR_LDS,
                            (hipStream_t)stream, (const f16*)x, (const f16*)conv_w,
                            (const f16*)st_in, (f16*)st_out, cx, gates, T, pos0, n_kheads, x_stride,

@@ -806,3 +806,45 @@ def test_gate_logits_of_a_fused_projection(fl, dev, rng, entry, T):
     for la, lb in ((a, b), (a.contiguous(), b), (a, b.contiguous())):
         with pytest.raises(ValueError, match="elements apart"):
             run(la, lb)
+
+
+# the one-launch front (three v heads a k head, 96 chunks x k heads or more): one
+# chunk of 96 k heads around the conv's 4-token tasks and the frames of history, the
+# model's heads on both sides of the rule and with ragged last chunks; one, two and
+# four v heads a k head (the separate kernels inside the call)
+@pytest.mark.parametrize("nk,nv,T,pos0", [
+    (96, 288, 1, 0), (96, 288, 2, 7), (96, 288, 3, 0), (96, 288, 5, 9), (96, 288, 63, 0),
+    (96, 288, 64, 5), (48, 144, 65, 3), (16, 48, 320, 7), (16, 48, 321, 0), (16, 48, 323, 64),
+    (16, 48, 1000, 5), (4, 4, 70, 3), (4, 8, 70, 0), (4, 16, 200, 9)])
+def test_prefill_layer_head_counts_equal_separate_calls(fl, dev, rng, nk, nv, T, pos0):
+    """The GDN layer's prefill in one call at other head counts against the
+    separate calls: the normed rows, the state and the conv frames bit for bit."""
+    W = (2 * nk + nv) * 128
+    x = to_dev((rng.standard_normal((T, W)) * 1.5).astype(np.float16), dev)
+    w = to_dev((rng.standard_normal((W, 4)) * 0.5).astype(np.float16), dev)
+    st = to_dev(rng.standard_normal((W, 3)).astype(np.float16), dev)
+    ad = to_dev(rng.standard_normal((T, nv)).astype(np.float32), dev)
+    bd = to_dev(rng.standard_normal((T, nv)).astype(np.float32), dev)
+    A_log = to_dev((rng.standard_normal(nv) * 0.3).astype(np.float32), dev)
+    dt = to_dev((rng.standard_normal(nv) * 0.3).astype(np.float32), dev)
+    z = to_dev(rng.standard_normal((T, nv, 128)).astype(np.float16), dev)
+    nw = to_dev((1 + rng.standard_normal(128) * 0.2).astype(np.float32), dev)
+    S1 = to_dev((rng.standard_normal((nv, 128, 128)) * 0.05).astype(np.float32), dev)
+    S2 = S1.clone()
+    so1, so2 = torch.full_like(st, 9.0), torch.full_like(st, 9.0)
+    heads = dict(ab_stride=nv, n_kheads=nk, n_vheads=nv)
+    y1 = fl.ops.gdn_prefill_layer(x, w, st, so1, ad, bd, A_log, dt, S1, z, nw, T=T, pos0=pos0,
+                                  x_stride=W, **heads)
+    c, kd = torch.empty_like(x), nk * 128
+    ln = torch.empty_like(c)
+    fl.ops.conv1d_causal(x, w, st, c, so2, dim=W, T=T, pos0=pos0, row_stride=W)
+    fl.ops.l2norm_scaled_strided(c, ln, rows=2 * nk, token_stride=W, T=T)
+    yr = fl.ops.gdn_prefill_chunked_logits(ln[:, :kd], ln[:, kd:2 * kd], c[:, 2 * kd:], ad, bd,
+                                           A_log, dt, S2, T=T, qk_stride=W, v_stride=W,
+                                           group=nv // nk, **heads)
+    y2 = fl.ops.rmsnorm_gated(yr.view(T, nv, 128), z, nw, T=T, rows=nv)
+    torch.cuda.synchronize()
+    assert torch.isfinite(y1.float()).all()
+    assert torch.equal(so1, so2), "conv frames differ"
+    assert torch.equal(S1, S2), "state differs"
+    assert torch.equal(y1, y2), "normed rows differ"
