@@ -199,11 +199,11 @@ struct DecTileQ8 {
 // 64-byte sector, and every wave loading its own rows' scales touches each
 // sector twice a workgroup, a quarter of all the lines its loads touch: so a
 // wave loads all 64 rows' scales of every fourth tile instead, 16 bytes a lane,
-// and the workgroup shares them. Against a dword a lane of each wave's own rows
-// (same box, us): B = 4, T = 1 at ~8k 24.6 -> 23.4, T = 3 at ~8k / ~32k / ~100k
-// 27.6 / 73.3 / 202.5 -> 26.7 / 70 / 194, B = 6, T = 1 at ~60k 164.6 -> 158;
-// under the length rule (three workgroups a CU before, two now, by LDS) 27.5 /
-// 74.4 / 201.5 -> 26.9 / 71 / 200; the same bits.
+// and the workgroup shares them. Their 8 KiB of LDS leave two workgroups a CU
+// where a dword a lane of each wave's own rows (dec_load_own_scales) leaves three:
+// launch_split picks by the grid. Same box, own -> shared, us: B = 4, T = 1 at
+// 8192 23.5 -> 22.7, 33000 63.7 -> 59.5, 100000 180.4 -> 173.0; B = 6 at 60000 166.7
+// -> 160.6; B = 8 at 3000 19.8 -> 19.0; the same bits.
 typedef f16 DecScales[2 * DEC_TILE][8];
 constexpr int DEC_SC_TILES = 4;   // tiles a group: one a wave
 
@@ -231,14 +231,22 @@ __device__ __forceinline__ void dec_load_tile(DecTileQ8& r, const char* __restri
     }
 }
 
-// The int8 tile as the fp16 tile the MFMAs read: fp16(byte * scale).
-__device__ __forceinline__ DecTileRegs dec_dequant(const DecTileQ8& q, const DecScales& sc,
-                                                   int lane, int w) {
+// Each wave's own scales of a tile: rows 16 (w & 1) + (l & 15), blocks 4 (w >> 1)
+// + 2 ((l >> 4) & 1) + 0, 1; K for l < 32, V above (`sc` that cache's scales).
+__device__ __forceinline__ uint32_t dec_load_own_scales(const char* __restrict__ sc, uint32_t rs,
+                                                        int j, int uhi, int lane, int w) {
+    const uint32_t row = (uint32_t)min(j * DEC_TILE + 16 * (w & 1) + (lane & 15), uhi - 1);
+    return *(const uint32_t*)(sc + (row * (rs / 16) + 2 * (4 * (w >> 1) + 2 * ((lane >> 4) & 1))));
+}
+
+// The int8 tile as the fp16 tile the MFMAs read, fp16(byte * scale), block 4 (w
+// >> 1) + l / 16 of K row 16 (w & 1) + (l & 15), scale ks(), and of V rows 16 (w &
+// 1) + 4 (l & 3) + i, scale vs(i).
+template <class KScale, class VScale>
+__device__ __forceinline__ DecTileRegs dec_dequant(const DecTileQ8& q, KScale&& kscale,
+                                                   VScale&& vscale) {
     DecTileRegs r;
-    // K row 16 (w & 1) + (l & 15), V rows 16 (w & 1) + 4 (l & 3) + i; block 4 (w
-    // >> 1) + l / 16 of both
-    const int r0 = 16 * (w & 1), blk = 4 * (w >> 1) + (lane >> 4);
-    const f16 ksh = sc[r0 + (lane & 15)][blk];
+    const f16 ksh = kscale();
     const f16x2 ks2 = {ksh, ksh};
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
@@ -249,13 +257,29 @@ __device__ __forceinline__ DecTileRegs dec_dequant(const DecTileQ8& q, const Dec
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const f16 vsh = sc[DEC_TILE + r0 + 4 * (lane & 3) + i][blk];
+        const f16 vsh = vscale(i);
         const f16x2 vs2 = {vsh, vsh};
         const f16x4 lo = q8_deq4(q.v[i].x, vs2);
         const f16x4 hi = q8_deq4(q.v[i].y, vs2);
         r.v[i] = (f16x8){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     }
     return r;
+}
+__device__ __forceinline__ DecTileRegs dec_dequant_shared(const DecTileQ8& q, const DecScales& sc,
+                                                          int lane, int w) {
+    const int r0 = 16 * (w & 1), blk = 4 * (w >> 1) + (lane >> 4);
+    return dec_dequant(q, [&] { return sc[r0 + (lane & 15)][blk]; },
+                       [&](int i) { return sc[DEC_TILE + r0 + 4 * (lane & 3) + i][blk]; });
+}
+__device__ __forceinline__ DecTileRegs dec_dequant_own(const DecTileQ8& q, uint32_t sc, int lane) {
+    // lane (l & 15) + 16 (l / 32)'s dword, half (l / 16) & 1; V 32 lanes above
+    const int bl = 16 * (lane >> 5);
+    auto of = [&](int from) {
+        const uint32_t p = (uint32_t)__builtin_amdgcn_ds_bpermute(from << 2, (int)sc);
+        return __builtin_bit_cast(f16x2, p)[(lane >> 4) & 1];
+    };
+    return dec_dequant(q, [&] { return of((lane & 15) + bl); },
+                       [&](int i) { return of(32 + bl + 4 * (lane & 3) + i); });
 }
 
 // int8 tiles are copied HBM -> LDS (global_load_lds) into stages of
@@ -366,8 +390,9 @@ __device__ __forceinline__ void lds_barrier() {
 // DEC: attention_dec_q8's split rule and partials -- (split, split_rows) are
 // (smax, tmin), pm in log2 units, no partial written for s >= St; otherwise
 // attention_split_gqa's -- pm in natural-log units, empty partials written.
-template <int NBUF, bool NT_V, bool Q8, bool DEC, bool STAGE>
-__global__ void __launch_bounds__(DEC_THREADS)
+// SHARED: the register tiles of an int8 cache take their scales through LDS.
+template <int NBUF, bool NT_V, bool Q8, bool DEC, bool STAGE, bool SHARED>
+__global__ void __launch_bounds__(DEC_THREADS, Q8 && !STAGE && !SHARED ? 3 : 1)
 attn_decode_split_kernel(const f16* __restrict__ qg, DecSeqs seqs, float* __restrict__ pacc,
                          float* __restrict__ pm, float* __restrict__ pd, int n_q_heads,
                          int n_kv, int q_pitch, int T, int split, int split_rows,
@@ -380,7 +405,7 @@ attn_decode_split_kernel(const f16* __restrict__ qg, DecSeqs seqs, float* __rest
     __shared__ __attribute__((aligned(16))) f32x4 s_part[2][SP_W][4][64];
     __shared__ __attribute__((aligned(16))) f16 s_vt[Q8 ? 2 : 1][DEC_WAVES][64][VTP];
     __shared__ __attribute__((aligned(16))) char s_stage[STAGE ? NBUF * Q8_STAGE_B : 16];
-    __shared__ __attribute__((aligned(16))) DecScales s_sc[2][Q8 && !STAGE ? DEC_SC_TILES : 1];
+    __shared__ __attribute__((aligned(16))) DecScales s_sc[2][SHARED ? DEC_SC_TILES : 1];
 
     const int s = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -616,8 +641,8 @@ attn_decode_split_kernel(const f16* __restrict__ qg, DecSeqs seqs, float* __rest
     } else if (uhi > ulo) {
         // NBUF register tile buffers: the loads of tile j + NBUF - 1 are issued
         // before the math of tile j. Every load is issued unconditionally (rows
-        // and tiles clamped into the range: a row past uhi reads row uhi - 1,
-        // masked to p = 0; a tile past the end re-reads the last one), so the
+        // clamped into the range: a row past uhi reads row uhi - 1, masked to p =
+        // 0; past the last tile the fp16 tiles re-read it), so the
         // compiler's wait before tile j's math counts exactly the loads of the
         // tiles behind it instead of draining them all.
         typedef typename std::conditional<Q8, DecTileQ8, DecTileRegs>::type Raw;
@@ -630,17 +655,21 @@ attn_decode_split_kernel(const f16* __restrict__ qg, DecSeqs seqs, float* __rest
         const int j0 = ulo / DEC_TILE;
         const int j1 = (uhi + DEC_TILE - 1) / DEC_TILE;
         Raw rbuf[NBUF];
-        if constexpr (Q8) {
+        if constexpr (SHARED) {
             // Group g's scales (tiles j0 + 4 g .. + 3, tile 4 g + w from wave w)
             // are loaded in tile 4 g - 4 and written to s_sc[g & 1] ahead of the
             // barrier of tile 4 g - 2. Every wave has by then passed the barrier
             // of tile 4 g - 3, so none still reads group g - 2 there (tile 4 g - 5
             // at the latest), and reads group g only past that of tile 4 g - 1.
+            // Loads past the last tile are not clamped to it: every lane's row is then
+            // row uhi - 1, a line or two instead of a tile's or a group's (a split of
+            // few tiles would pay for them: B = 3 at 6000, 5 tiles a split, 22.1 us
+            // with the last tile read again up to a whole group, 19.0 so).
             static_assert(DEC_SC_TILES % NBUF == 0 && DEC_SC_TILES == DEC_WAVES, "");
             const char* sc = (const char*)(hh ? vsb : ksb);
-            u32x4 scales = dec_load_scales(sc, (uint32_t)row_stride, min(j0 + w, j1 - 1), uhi, lane);
+            u32x4 scales = dec_load_scales(sc, (uint32_t)row_stride, j0 + w, uhi, lane);
 #pragma unroll
-            for (int p = 0; p < NBUF - 1; ++p) load(rbuf[p], min(j0 + p, j1 - 1));
+            for (int p = 0; p < NBUF - 1; ++p) load(rbuf[p], j0 + p);
             *(u32x4*)s_sc[0][w][lane] = scales;
             lds_barrier();
             int g = 0;
@@ -648,15 +677,33 @@ attn_decode_split_kernel(const f16* __restrict__ qg, DecSeqs seqs, float* __rest
 #pragma unroll
                 for (int u = 0; u < DEC_SC_TILES; ++u) {
                     const int jj = j + u;
+                    if (jj >= j1) break;
                     if (u == 0)
-                        scales = dec_load_scales(sc, (uint32_t)row_stride,
-                                                 min(j + DEC_SC_TILES + w, j1 - 1), uhi, lane);
-                    load(rbuf[(u + NBUF - 1) % NBUF], min(jj + NBUF - 1, j1 - 1));
-                    if (jj < j1)
-                        body(dec_dequant(rbuf[u % NBUF], s_sc[g][u], lane, w), jj,
-                             [&] { if (u == 2) *(u32x4*)s_sc[g ^ 1][w][lane] = scales; }, none);
+                        scales = dec_load_scales(sc, (uint32_t)row_stride, j + DEC_SC_TILES + w,
+                                                 uhi, lane);
+                    load(rbuf[(u + NBUF - 1) % NBUF], jj + NBUF - 1);
+                    body(dec_dequant_shared(rbuf[u % NBUF], s_sc[g][u], lane, w), jj,
+                         [&] { if (u == 2) *(u32x4*)s_sc[g ^ 1][w][lane] = scales; }, none);
                 }
                 g ^= 1;
+            }
+        } else if constexpr (Q8) {
+            const char* sc = (const char*)(hh ? vsb : ksb);
+            uint32_t sbuf[NBUF];
+            auto load_own = [&](int p, int j) {
+                load(rbuf[p], j);
+                sbuf[p] = dec_load_own_scales(sc, (uint32_t)row_stride, j, uhi, lane, w);
+            };
+#pragma unroll
+            for (int p = 0; p < NBUF - 1; ++p) load_own(p, j0 + p);
+            for (int j = j0; j < j1; j += NBUF) {
+#pragma unroll
+                for (int u = 0; u < NBUF; ++u) {
+                    const int jj = j + u;
+                    if (jj >= j1) break;
+                    load_own((u + NBUF - 1) % NBUF, jj + NBUF - 1);
+                    body(dec_dequant_own(rbuf[u], sbuf[u], lane), jj, none, none);
+                }
             }
         } else {
 #pragma unroll
@@ -1008,8 +1055,7 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 // int8 register tiles: 2 buffers -- in the int8 layout 3 buffers measured 83.4
 // / 30.9 us at ~32k / ~8k against 77.5 / 28.0, 4 and 5 slower still (with each
-// wave's own scale loads; two workgroups a CU are resident now, by the 60 KiB
-// of LDS with the shared scales)
+// wave's own scale loads)
 #ifndef DEC_NBUF_Q8
 #define DEC_NBUF_Q8 2
 #endif
@@ -1020,11 +1066,26 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 // per-sequence launches of attention_dec_q8 (112 workgroups, ~100k rows
 // each) 478 against 525 us a step for the register tiles; B = 1 at 4k-16k
 // within 3 % of them (12.2 at 4k either way); larger grids keep the register
-// tiles, whose workgroups (two a CU) overlap each other's barriers (B = 4,
+// tiles, whose workgroups (two or three a CU) overlap each other's barriers (B = 4,
 // T = 3 at ~8k / ~100k: 33.3 / 223 us against 34.4 / 235 staged, measured
 // before the int8 layout). Both give the same bits.
 constexpr int DEC_STAGE_MAX_WGS = 256;
 constexpr int DEC_NBUF_STAGE = 2;
+
+// The current device's compute-unit count, looked up once per device.
+int dec_cu_count() {
+    static int cached[64] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    if (cached[dev] == 0) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+            n <= 0)
+            n = 256;
+        cached[dev] = n;
+    }
+    return cached[dev];
+}
 
 // grid_split blocks a (sequence, kv head); `split` the partials' stride;
 // split_floor the floor of split_count (0: the reference's rule).
@@ -1033,15 +1094,25 @@ int launch_split(const f16* qg, const DecSeqs& seqs, float* pacc, float* pm, flo
                  int T, int n_q_heads, int n_kv, int q_pitch, int grid_split, int split,
                  int split_rows, float sl2, hipStream_t stream, int split_floor = 0) {
     dim3 grid(grid_split, n_kv, B);
-    if (Q8 && (long long)grid_split * n_kv * B <= DEC_STAGE_MAX_WGS)
-        hipLaunchKernelGGL((attn_decode_split_kernel<DEC_NBUF_STAGE, false, true, DEC, true>),
-                           grid, dim3(DEC_THREADS), 0, stream, qg, seqs, pacc, pm, pd, n_q_heads,
-                           n_kv, q_pitch, T, split, split_rows, split_floor, sl2);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(DEC_THREADS), 0, stream, qg, seqs, pacc, pm, pd,
+                           n_q_heads, n_kv, q_pitch, T, split, split_rows, split_floor, sl2);
+    };
+    // int8 register tiles: the shared scales (two workgroups a CU), but for the
+    // grids that each wave's own (three a CU) run in one round and the shared ones
+    // in two. Same box, shared / own, us: 736 workgroups (B = 4 at 12000, splits of
+    // 256 rows) 36.5 / 32.7, 744 (B = 3 at 16000) 36.2 / 32.7, 768 (B = 6 at 6000)
+    // 27.6 / 26.0, 640 (B = 5 at 3000) 19.4 / 19.0; 920 (B = 5 at 12000) 40.0 / 42.0,
+    // 992 (B = 4 at 16000) 40.8 / 45.5, 1024 (B = 4 at 33000) 62.4 / 66.8.
+    const long long wgs = (long long)grid_split * n_kv * B;
+    if constexpr (!Q8)
+        launch(attn_decode_split_kernel<DEC_NBUF, DEC_NT_V, false, DEC, false, false>);
+    else if (wgs <= DEC_STAGE_MAX_WGS)
+        launch(attn_decode_split_kernel<DEC_NBUF_STAGE, false, true, DEC, true, false>);
+    else if (wgs > 2LL * dec_cu_count() && wgs <= 3LL * dec_cu_count())
+        launch(attn_decode_split_kernel<DEC_NBUF_Q8, DEC_NT_V, true, DEC, false, false>);
     else
-        hipLaunchKernelGGL((attn_decode_split_kernel<Q8 ? DEC_NBUF_Q8 : DEC_NBUF, DEC_NT_V, Q8, DEC,
-                                                     false>),
-                           grid, dim3(DEC_THREADS), 0, stream, qg, seqs, pacc, pm, pd, n_q_heads,
-                           n_kv, q_pitch, T, split, split_rows, split_floor, sl2);
+        launch(attn_decode_split_kernel<DEC_NBUF_Q8, DEC_NT_V, true, DEC, false, true>);
     return fl::check_launch("attn_decode_split");
 }
 
@@ -1077,21 +1148,6 @@ int check_decode_geometry(int T, int n_q_heads, int n_kv, int head_dim, int q_pi
     FL_REQUIRE(split >= 1 && split <= 65535, "split in [1, 65535]");
     FL_REQUIRE(split_rows >= DEC_TILE, "split_rows >= 32");
     return FL_OK;
-}
-
-// The current device's compute-unit count, looked up once per device.
-int dec_cu_count() {
-    static int cached[64] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (cached[dev] == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            n <= 0)
-            n = 256;
-        cached[dev] = n;
-    }
-    return cached[dev];
 }
 
 // split_rows 0, the grid rule: S = floor(W / (B n_kv)) splits a token (at

@@ -371,3 +371,17 @@ def test_prefill_without_room_for_the_staging_copy(fl, dev, monkeypatch, T, pos0
     fl.ops.attention_prefill_q8(q, k8, v8, pos0=pos0, max_pos=L, z=z)
     torch.cuda.synchronize()
     assert torch.isfinite(want.float()).all() and torch.equal(z, want)
+
+
+# grids of more than two and at most three workgroups a CU: each wave's own scale
+# loads, 1 .. 3, 5 .. 8 and 8 .. 17 tiles a split, the last one ragged or whole
+@pytest.mark.parametrize("T", [1, 3])
+@pytest.mark.parametrize("lens,splits", [([31, 64, 95, 127, 128, 700, 1300, 1500], 23),
+                                         ([9729, 5120, 6150, 97, 4], 38), ([33000, 12000, 33], 64)])
+def test_decode_q8_own_scales_batched_equals_single(fl, dev, T, lens, splits):
+    """As above for those grids: the same bits as the staged tiles of one sequence."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    assert 2 * cus < splits * 4 * len(lens) <= 3 * cus
+    n = max(lens)
+    assert splits == min(64, max(n // fl.geometry.SPLIT_ROWS, min(n // 64, 32)))
+    test_decode_q8_tiles_a_split_batched_equals_single(fl, dev, T, lens)
