@@ -42,6 +42,7 @@
 #include <cstdlib>
 #include <functional>
 #include <mutex>
+#include <new>
 #include <queue>
 #include <vector>
 
@@ -967,7 +968,7 @@ int prefill_device_setup(int& n_cu) {
 // entries used (bins + 1 + row tiles), 0 where the grid of row tiles x kv
 // heads is launched instead: a kv-head count that does not divide the 8 XCDs,
 // no more row tiles than bins, or a plan over R64_PLAN_MAX entries.
-int r64_build_plan(int T, int pos0, int G, int n_kv, int n_cu, R64Plan& plan) {
+int r64_cut_plan(int T, int pos0, int G, int n_kv, int n_cu, R64Plan& plan) {
     if (T < 1 || pos0 < 0 || G < 1 || n_kv < 1 || 8 % n_kv != 0 || n_cu < 8 || n_cu % 8 != 0)
         return 0;
     const int RT = T * G;
@@ -1068,6 +1069,16 @@ int r64_build_plan(int T, int pos0, int G, int n_kv, int n_cu, R64Plan& plan) {
     return k;
 }
 
+// The plans are made in host vectors and C entry points call for them: without
+// memory for one there is none, and the call runs the way it does without.
+int r64_build_plan(int T, int pos0, int G, int n_kv, int n_cu, R64Plan& plan) {
+    try {
+        return r64_cut_plan(T, pos0, G, n_kv, n_cu, plan);
+    } catch (const std::bad_alloc&) {
+        return 0;
+    }
+}
+
 // r64_build_plan, kept for the last few shapes (a serving loop repeats its
 // chunk shapes); copied out under the lock.
 struct R64PlanEntry {
@@ -1116,7 +1127,7 @@ struct StreamPlan {
     int bins, slots, cost;
 };
 
-int r64_stream_plan(int T, int pos0, int G, int n_kv, int n_cu, StreamPlan& sp) {
+int r64_cut_stream(int T, int pos0, int G, int n_kv, int n_cu, StreamPlan& sp) {
     if (T < 1 || pos0 < 0 || G < 1 || n_kv < 1 || 8 % n_kv != 0 || n_cu < 8 || n_cu % 8 != 0)
         return 0;
     const long long RT = (long long)T * G;
@@ -1215,6 +1226,14 @@ int r64_stream_plan(int T, int pos0, int G, int n_kv, int n_cu, StreamPlan& sp) 
     sp.slots = slot0[N];
     sp.cost = (int)longest + R64_MERGE_COST + sp.slots * n_kv / R64_SLOTS_PER_TILE;
     return 3 * bins + 2 + (int)N + 1;
+}
+
+int r64_stream_plan(int T, int pos0, int G, int n_kv, int n_cu, StreamPlan& sp) {
+    try {
+        return r64_cut_stream(T, pos0, G, n_kv, n_cu, sp);
+    } catch (const std::bad_alloc&) {
+        return 0;
+    }
 }
 
 size_t stream_work_bytes(const StreamPlan& sp, int n_kv) {
@@ -1419,7 +1438,12 @@ void auto_choice(int T, int pos0, int n_q_heads, int n_kv_heads, int n_cu, bool 
             }
         }
     }
-    choose(T, pos0, n_q_heads, n_kv_heads, n_cu, q8, c);
+    try {
+        choose(T, pos0, n_q_heads, n_kv_heads, n_cu, q8, c);
+    } catch (const std::bad_alloc&) {   // (not kept)
+        c.stage = c.stream = false;
+        return;
+    }
     std::lock_guard<std::mutex> lock(g_auto_mu);
     g_auto_cache[g_auto_next] = {T, pos0, n_q_heads, n_kv_heads, n_cu, q8, c};
     g_auto_next = (g_auto_next + 1) % AUTO_CACHE;

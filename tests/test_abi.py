@@ -241,6 +241,47 @@ def test_prefill_q8_staging_is_bounded(fl, monkeypatch):
         fl.ops._prefill_split(1024, 98000, *args, q8=False)
 
 
+def test_plans_survive_a_failed_allocation(tmp_path):
+    """The prefill's host plans without memory for them (operator new made to
+    throw): the entry points return what they do without a plan and nothing
+    leaves them, in a fresh process."""
+    import subprocess
+    import sys
+    from __graft_entry__ import PKG_DIR
+    (tmp_path / "full.cpp").write_text(
+        "#include <cstdlib>\n#include <new>\nstatic bool full;\n"
+        "extern \"C\" void set_full(int f) { full = f != 0; }\n"
+        "void* operator new(std::size_t n) {\n"
+        "    void* p = full ? nullptr : std::malloc(n ? n : 1);\n"
+        "    if (!p) throw std::bad_alloc();\n    return p;\n}\n"
+        "void operator delete(void* p) noexcept { std::free(p); }\n"
+        "void operator delete(void* p, std::size_t) noexcept { std::free(p); }\n")
+    subprocess.run(["g++", "-shared", "-fPIC", "-o", str(tmp_path / "full.so"),
+                    str(tmp_path / "full.cpp")], check=True)
+    code = (
+        "import ctypes\n"
+        f"full = ctypes.CDLL({str(tmp_path / 'full.so')!r}, ctypes.RTLD_GLOBAL)\n"
+        f"lib = ctypes.CDLL({str(PKG_DIR / 'libfl355.so')!r})\n"
+        "size = lib.fl_attention_prefill_auto_work_bytes\n"
+        "size.restype = ctypes.c_size_t\n"
+        "buf = (ctypes.c_ushort * 1024)()\n"
+        "plan = lambda: lib.fl_attention_prefill_plan(8192, 0, 24, 4, 256, buf, 1024)\n"
+        "pieces = lambda: lib.fl_attention_prefill_pieces(777, 3001, 24, 4, 256, buf, 1024, None, None)\n"
+        "size(5, 0, 24, 4, 256, 0)   # the HIP runtime is up\n"
+        "assert plan() > 0 and pieces() > 0\n"
+        "full.set_full(1)\n"
+        "got = [plan(), pieces()] + [size(T, 3001, 24, 4, 256, q8) for T in (683, 777) for q8 in (0, 1)]\n"
+        "full.set_full(0)\n"
+        "split = lib.fl_attention_prefill_split_count   # and int8: the staged rows\n"
+        "want = [0, 0] + [24 * T * 1032 * split(T, 3001, 24, 4) + q8 * (3001 + T) * 4096\n"
+        "                 for T in (683, 777) for q8 in (0, 1)]\n"
+        "assert got == want, (got, want)\n"
+        "assert plan() > 0 and pieces() > 0 and size(683, 3001, 24, 4, 256, 0) != want[2]\n"
+        "print('survived')\n")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and "survived" in r.stdout, (r.returncode, r.stdout + r.stderr)
+
+
 
 def _plan_weights(T, pos0, G):
     RT = T * G
