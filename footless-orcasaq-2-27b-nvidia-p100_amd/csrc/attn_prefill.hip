@@ -1069,17 +1069,7 @@ int r64_cut_plan(int T, int pos0, int G, int n_kv, int n_cu, R64Plan& plan) {
     return k;
 }
 
-// The plans are made in host vectors and C entry points call for them: without
-// memory for one there is none, and the call runs the way it does without.
-int r64_build_plan(int T, int pos0, int G, int n_kv, int n_cu, R64Plan& plan) {
-    try {
-        return r64_cut_plan(T, pos0, G, n_kv, n_cu, plan);
-    } catch (const std::bad_alloc&) {
-        return 0;
-    }
-}
-
-// r64_build_plan, kept for the last few shapes (a serving loop repeats its
+// r64_cut_plan, kept for the last few shapes (a serving loop repeats its
 // chunk shapes); copied out under the lock.
 struct R64PlanEntry {
     int T, pos0, G, n_kv, n_cu, used;
@@ -1101,7 +1091,15 @@ int r64_plan(int T, int pos0, int G, int n_kv, int n_cu, R64Plan& plan) {
             }
         }
     }
-    const int used = r64_build_plan(T, pos0, G, n_kv, n_cu, plan);
+    // (made in host vectors, like the piece list below, and C entry points call for
+    // both: without memory for one there is none, the call runs as it does without,
+    // and nothing is kept)
+    int used = 0;
+    try {
+        used = r64_cut_plan(T, pos0, G, n_kv, n_cu, plan);
+    } catch (const std::bad_alloc&) {
+        return 0;
+    }
     std::lock_guard<std::mutex> lock(g_plan_mu);
     R64PlanEntry& e = g_plan_cache[g_plan_next];
     e = {T, pos0, G, n_kv, n_cu, used, plan};
@@ -1226,14 +1224,6 @@ int r64_cut_stream(int T, int pos0, int G, int n_kv, int n_cu, StreamPlan& sp) {
     sp.slots = slot0[N];
     sp.cost = (int)longest + R64_MERGE_COST + sp.slots * n_kv / R64_SLOTS_PER_TILE;
     return 3 * bins + 2 + (int)N + 1;
-}
-
-int r64_stream_plan(int T, int pos0, int G, int n_kv, int n_cu, StreamPlan& sp) {
-    try {
-        return r64_cut_stream(T, pos0, G, n_kv, n_cu, sp);
-    } catch (const std::bad_alloc&) {
-        return 0;
-    }
 }
 
 size_t stream_work_bytes(const StreamPlan& sp, int n_kv) {
@@ -1401,7 +1391,7 @@ void choose(int T, int pos0, int n_q_heads, int n_kv_heads, int n_cu, bool q8, A
                           use_r64_split(T, pos0, n_q_heads, n_kv_heads) &&
                           (pos0 + (long long)T) * n_kv_heads > R64_LLC_ROWS * 4;
     c.stage = false;
-    c.stream = !together && r64_stream_plan(T, pos0, G, n_kv_heads, n_cu, c.sp) > 0 &&
+    c.stream = !together && r64_cut_stream(T, pos0, G, n_kv_heads, n_cu, c.sp) > 0 &&
                10 * (long long)c.sp.cost < cost;
     if (!q8) return;
     if (c.stream) cost = 10 * (long long)c.sp.cost;
@@ -1440,7 +1430,7 @@ void auto_choice(int T, int pos0, int n_q_heads, int n_kv_heads, int n_cu, bool 
     }
     try {
         choose(T, pos0, n_q_heads, n_kv_heads, n_cu, q8, c);
-    } catch (const std::bad_alloc&) {   // (not kept)
+    } catch (const std::bad_alloc&) {   // the plain path this time (not kept)
         c.stage = c.stream = false;
         return;
     }
@@ -1686,7 +1676,12 @@ extern "C" int fl_attention_prefill_plan(int T, int pos0, int n_q_heads, int n_k
         !use_r64(T, n_q_heads, n_kv_heads))
         return 0;
     R64Plan plan;
-    const int used = r64_build_plan(T, pos0, n_q_heads / n_kv_heads, n_kv_heads, n_cu, plan);
+    int used = 0;
+    try {
+        used = r64_cut_plan(T, pos0, n_q_heads / n_kv_heads, n_kv_heads, n_cu, plan);
+    } catch (const std::bad_alloc&) {
+        return 0;
+    }
     if (out != nullptr)
         for (int i = 0; i < used && i < cap; ++i) out[i] = plan.v[i];
     return used;
@@ -1696,7 +1691,12 @@ extern "C" int fl_attention_prefill_pieces(int T, int pos0, int n_q_heads, int n
                                            unsigned short* out, int cap, int* bins, int* slots) {
     if (n_kv_heads < 1 || n_q_heads < 1 || n_q_heads % n_kv_heads != 0) return 0;
     StreamPlan sp;
-    const int used = r64_stream_plan(T, pos0, n_q_heads / n_kv_heads, n_kv_heads, n_cu, sp);
+    int used = 0;
+    try {
+        used = r64_cut_stream(T, pos0, n_q_heads / n_kv_heads, n_kv_heads, n_cu, sp);
+    } catch (const std::bad_alloc&) {
+        return 0;
+    }
     if (used == 0) return 0;
     if (bins != nullptr) *bins = sp.bins;
     if (slots != nullptr) *slots = sp.slots;

@@ -266,17 +266,20 @@ def test_plans_survive_a_failed_allocation(tmp_path):
         "size.restype = ctypes.c_size_t\n"
         "buf = (ctypes.c_ushort * 1024)()\n"
         "plan = lambda: lib.fl_attention_prefill_plan(8192, 0, 24, 4, 256, buf, 1024)\n"
-        "pieces = lambda: lib.fl_attention_prefill_pieces(777, 3001, 24, 4, 256, buf, 1024, None, None)\n"
+        "args = 777, 3001, 24, 4, 256, buf, 1024, None, None\n"
+        "pieces = lambda: lib.fl_attention_prefill_pieces(*args)\n"
+        "calls = [(683, 0), (683, 1), (777, 0), (777, 1)]\n"
         "size(5, 0, 24, 4, 256, 0)   # the HIP runtime is up\n"
         "assert plan() > 0 and pieces() > 0\n"
         "full.set_full(1)\n"
-        "got = [plan(), pieces()] + [size(T, 3001, 24, 4, 256, q8) for T in (683, 777) for q8 in (0, 1)]\n"
+        "got = [plan(), pieces()] + [size(T, 3001, 24, 4, 256, q8) for T, q8 in calls]\n"
         "full.set_full(0)\n"
-        "split = lib.fl_attention_prefill_split_count   # and int8: the staged rows\n"
-        "want = [0, 0] + [24 * T * 1032 * split(T, 3001, 24, 4) + q8 * (3001 + T) * 4096\n"
-        "                 for T in (683, 777) for q8 in (0, 1)]\n"
+        "S = lib.fl_attention_prefill_split_count, lib.fl_attention_prefill_split_count_q8\n"
+        "want = [0, 0] + [24 * T * 1032 * S[q8](T, 3001, 24, 4) for T, q8 in calls]\n"
         "assert got == want, (got, want)\n"
-        "assert plan() > 0 and pieces() > 0 and size(683, 3001, 24, 4, 256, 0) != want[2]\n"
+        "assert plan() > 0 and pieces() > 0\n"
+        "again = [size(T, 3001, 24, 4, 256, q8) for T, q8 in calls]   # nothing was kept\n"
+        "assert all(a != w for a, w in zip(again, want[2:])), (again, want)\n"
         "print('survived')\n")
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and "survived" in r.stdout, (r.returncode, r.stdout + r.stderr)
