@@ -395,13 +395,29 @@ def test_prefill_kv_split_vs_oracle(fl, dev, orc, rng, T, pos0, split):
     assert ok, f"T={T} pos0={pos0} split={split}: max|err| {err}"
 
 
-# the long-prompt kernel whole (4096 tokens) and with its KV split (683 at 16000)
-@pytest.mark.parametrize("T,pos0", [(4096, 0), (683, 16000)])
+def prefill_route(fl, T, pos0, split, kv8=False):
+    """What a call runs: "whole" row tiles, a uniform KV "split", the equal runs'
+    "pieces", or over an int8 cache "staged" rows first (24 / 4 heads)."""
+    if split is not None:
+        return "split" if split > 1 else "whole"
+    lib = fl._lib.lib()
+    need = int(lib.fl_attention_prefill_auto_work_bytes(T, pos0, 24, 4, 256, int(kv8)))
+    count = (fl.ops.prefill_split_count_q8 if kv8 else fl.ops.prefill_split_count)(T, pos0)
+    if need == int(lib.fl_attention_prefill_work_bytes(T, 24, 256, count)):
+        return "split" if count > 1 else "whole"
+    return "staged" if kv8 else "pieces"
+
+
+# the three forms of the 64-rows-a-wave kernel: whole row tiles (4096 tokens), its
+# uniform KV split and its piece list (683 at 16000)
+@pytest.mark.parametrize("T,pos0,split,route", [(4096, 0, None, "whole"), (683, 16000, 5, "split"),
+                                                (683, 16000, None, "pieces")])
 @pytest.mark.parametrize("which", ["k", "v"])
-def test_prefill_cache_across_4gib_boundary(fl, dev, T, pos0, which):
+def test_prefill_cache_across_4gib_boundary(fl, dev, T, pos0, split, route, which):
     """A K or V cache whose rows cross a 4 GiB boundary of the address space: the
     row addresses of the tile copies carry into their upper half there. The
     same bits as over a copy of it elsewhere."""
+    assert prefill_route(fl, T, pos0, split) == route
     L = pos0 + T
     n = L * 4 * 256 * 2
     g = torch.Generator(device=dev).manual_seed(L)
@@ -413,9 +429,9 @@ def test_prefill_cache_across_4gib_boundary(fl, dev, T, pos0, which):
     assert base <= at and at + n <= base + room.numel() and at >> 32 != (at + n - 1) >> 32
     across = room[at - base:at - base + n].view(torch.float16).view(L, 4, 256)
     across.copy_(cache[which])
-    want = fl.ops.attention_prefill(q, cache["k"], cache["v"], pos0=pos0, scale=1.0)
+    want = fl.ops.attention_prefill(q, cache["k"], cache["v"], pos0=pos0, scale=1.0, split=split)
     got = fl.ops.attention_prefill(q, *(across if c == which else cache[c] for c in "kv"),
-                                   pos0=pos0, scale=1.0)
+                                   pos0=pos0, scale=1.0, split=split)
     torch.cuda.synchronize()
     assert torch.isfinite(want.float()).all() and torch.equal(got, want)
 
@@ -466,7 +482,7 @@ def test_prefill_left_to_the_library_vs_fp32(fl, dev, kv8, T, pos0):
     kd = torch.randn((L, 4, 256), generator=g, device=dev).half()
     vd = torch.randn((L, 4, 256), generator=g, device=dev).half()
     need = int(fl._lib.lib().fl_attention_prefill_auto_work_bytes(T, pos0, 24, 4, 256, int(kv8)))
-    assert need > 0
+    assert need > 0 and prefill_route(fl, T, pos0, None, kv8) == ("staged" if kv8 else "pieces")
     if kv8:
         k8, v8 = fl.ops.kv8_cache(L), fl.ops.kv8_cache(L)
         fl.ops.kv_store_q8(kd, vd, k8, v8, pos0=0, max_pos=L)
@@ -507,6 +523,7 @@ def test_prefill_kv_split_chunk_deep_in_prompt(fl, dev):
 
     T, pos0 = 1024, 98000
     assert fl.ops.prefill_split_count(T, pos0) == 8
+    assert prefill_route(fl, T, pos0, None) == "split"
     L = pos0 + T
     g = torch.Generator(device=dev).manual_seed(98)
     q = (torch.randn((T, 24, 256), generator=g, device=dev) / 16).half()
@@ -611,23 +628,24 @@ def test_merge_layouts_vs_oracle(fl, dev, orc, rng, head_dim, z_pitch, split, T)
     assert not got[..., head_dim:].any(), "wrote past head_dim"
 
 
-# the KV-split prefills' merge carries the gate; the unsplit ones run the gate
-# after them: split 3 of the 128-row kernel, the 64-rows-a-wave kernel's own
-# split (683 tokens at 16000), the unsplit 128-row and long-prompt kernels,
-# and over an int8 cache its split, an unsplit call and a staged long prompt
-@pytest.mark.parametrize("kv8,T,pos0,split,splits", [
-    (False, 300, 500, 3, True), (False, 683, 16000, None, True), (False, 300, 500, 1, False),
-    (False, 4096, 0, None, False), (True, 300, 500, 3, True), (True, 1024, 8000, None, True),
-    (True, 300, 500, 1, False), (True, 4096, 512, None, False)])
-def test_prefill_gated_equals_prefill_then_gate(fl, dev, kv8, T, pos0, split, splits):
+# the split prefills' merges and the piece list's carry the gate; the unsplit calls
+# run the gate after them: split 3 of the 128-row kernel, the 64-rows-a-wave
+# kernel's split and its pieces (683 tokens at 16000), the unsplit 128-row and
+# long-prompt kernels, and over an int8 cache its kernel's split (300 and 1024
+# tokens), an unsplit call, and the staged rows' pieces and long prompt
+@pytest.mark.parametrize("kv8,T,pos0,split,route", [
+    (False, 300, 500, 3, "split"), (False, 683, 16000, 5, "split"),
+    (False, 683, 16000, None, "pieces"), (False, 300, 500, 1, "whole"),
+    (False, 4096, 0, None, "whole"), (True, 300, 500, 3, "split"), (True, 1024, 8000, 3, "split"),
+    (True, 1024, 8000, None, "staged"), (True, 300, 500, 1, "whole"),
+    (True, 4096, 512, None, "staged")])
+def test_prefill_gated_equals_prefill_then_gate(fl, dev, kv8, T, pos0, split, route):
     """fl_attention_prefill_gated (the layer's attention output: the gate half
-    of each head's q | gate row applied in the KV-split merge, or by
+    of each head's q | gate row applied in the split's or the pieces' merge, or by
     attn_gate after an unsplit prefill) against the prefill then attn_gate,
     bit for bit."""
+    assert prefill_route(fl, T, pos0, split, kv8) == route
     L = pos0 + T
-    if split is None:
-        count = (fl.ops.prefill_split_count_q8 if kv8 else fl.ops.prefill_split_count)(T, pos0)
-        assert (count > 1) == splits, count
     g = torch.Generator(device=dev).manual_seed(T + pos0)
     qg = torch.randn((T, 24, 512), generator=g, device=dev)
     qg[..., :256] /= 16
