@@ -1320,7 +1320,13 @@ int grid_makespan(int wgs, int cus, int heavy, int light) {
 // from 0 56 / 56 us, 1024 79 / 102, 3072 135 / 151, 8000 251 / 278, 30000 767 /
 // 795, 98000 2458 / 2366; T = 777 at 3072 104 / 134, 683 at 8000 185 / 235, 512 at
 // 98000 1284 / 1437, 2048 at 8000 487 / 603, 3000 at 30000 2328 / 3324, 16 at
-// 98000 132 / 236, 4096 from 0 286 / 273.
+// 98000 132 / 236, 4096 from 0 286 / 273. Around the line, the list forced on both
+// sides of it, T = 1024 / 1300: at 56000 1402 / 1460 and 1850 / 1864, 64000 1616 /
+// 1622 and 2101 / 2100, 70000 1791 / 1770 and 2369 / 2335, 80000 2053 / 2044 and
+// 2784 / 2692; 16 / 2 heads, T = 1500, at 100000 2460 / 2454, 135000 (past it)
+// 3319 / 3296. It stands for the even rounds of those grids: where the uniform
+// split's are uneven (32 / 8 heads, T = 1024 at 40000: 1304 / 1675) the list would
+// still pay past it, which the rule leaves.
 constexpr long long R64_LLC_ROWS = 65536;   // x 4 kv heads x 1 KiB: 256 MiB
 constexpr int PF_UNIT_TENTHS = 11;
 constexpr int PF_UNIT_Q8_TENTHS = 15;   // the int8 128-row kernel

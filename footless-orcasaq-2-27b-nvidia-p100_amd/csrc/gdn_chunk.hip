@@ -506,7 +506,7 @@ chunk_prep_kernel(const f16* __restrict__ q, const f16* __restrict__ k, const Pr
 // 16 chunks x 16 k heads are one workgroup a CU and 23 us (kernel traces).
 // Bound by the conv's vector instructions (of 43 k clocks ~18 k, most of them
 // the silu), then the chain from A to T's operands (~13 k) that one workgroup
-// a CU leaves exposed. 139 KiB of LDS.
+// a CU leaves exposed. 138 KiB of LDS.
 //
 // Conv: a 16-lane group takes one head's 128 channels (8 a lane) of 4
 // consecutive tokens, all 7 rows requested at once; the chunk's 5 heads x 16

@@ -37,3 +37,17 @@ def test_asm_that_writes_scc_says_so(src):
     for line, stmt in asm_statements(text):
         if WRITES_SCC.search(stmt):
             assert '"scc"' in stmt, f"{src}:{line}: writes SCC without the clobber"
+
+
+def test_files_compiled_without_nans_keep_none():
+    """A source whose flags assume that there are no NaNs must not use the helpers
+    that promise to keep one (f16_sat, the gate's sigmoid and silu): compiled so
+    they turn it into a number."""
+    import __graft_entry__ as ge
+    flags = ge._load_builder().FILE_FLAGS
+    without = [name for name, f in flags.items() if "-fno-honor-nans" in f]
+    assert without == ["attn_prefill"]
+    for name in without:
+        text = re.sub(r"//[^\n]*", "", (CSRC / f"{name}.hip").read_text())
+        used = re.findall(r"\b(f16_sat8?|sigmoid_f|silu_f|div_big)\s*\(", text)
+        assert not used, f"{name}.hip: {sorted(set(used))}"
