@@ -295,18 +295,20 @@ def _prefill_gated(args, q8: int, split: int, zargs, work):
 
 def prefill_split_count(T: int, pos0: int, n_q_heads: int = N_HEADS,
                         n_kv_heads: int = N_KV) -> int:
-    """The KV split the prefill takes for T queries at pos0 (runtime.py:
-    2932-2941's role): 1 unless the 128-row workgroups are too few for the
-    CUs (the 64-rows-a-wave kernel's split from 64 workgroups of 256 rows
-    and 16384 cache rows, the 128-row kernel's otherwise). The int8 prefill
-    takes prefill_split_count_q8's."""
+    """The best uniform KV split for T queries at pos0 (runtime.py:2932-2941's
+    role): 1 unless the 128-row workgroups are too few for the CUs (the
+    64-rows-a-wave kernel's split from 64 workgroups of 256 rows and 16384
+    cache rows, the 128-row kernel's otherwise). A call left to the library
+    takes it where its equal runs are no cheaper. Over an int8 cache:
+    prefill_split_count_q8."""
     return int(_lib.lib().fl_attention_prefill_split_count(T, pos0, n_q_heads, n_kv_heads))
 
 
 def prefill_split_count_q8(T: int, pos0: int, n_q_heads: int = N_HEADS,
                            n_kv_heads: int = N_KV) -> int:
     """prefill_split_count for an int8 cache: the 128-row int8 kernel's split
-    (what fl_attention_prefill_kv_q8 takes for split 0)."""
+    (what fl_attention_prefill_kv_q8 takes for split 0 where it does not stage
+    the cache rows)."""
     return int(_lib.lib().fl_attention_prefill_split_count_q8(T, pos0, n_q_heads, n_kv_heads))
 
 
@@ -492,10 +494,11 @@ def attention_prefill_q8(q, kcache, vcache, *, pos0: int, max_pos: int, T: int |
                          scale: float = ATTN_SCALE, split: int | None = None, work=None,
                          gated: bool = False):
     """attention_prefill_fh_q8 (kernels.cu:2778-2786) over an int8 cache, with
-    kv_store_q8 of k_new / v_new fused in front when given. Long prompts run
-    the fp16 long-prompt kernel on an fp16 copy of the cache rows made first
-    (in `work`, allocated here when not given or too small). gated: as
-    attention_prefill's."""
+    kv_store_q8 of k_new / v_new fused in front when given. Long prompts, and
+    shorter calls left to the library where that costs less, run the fp16
+    kernels on an fp16 copy of the cache rows made first (in `work`, allocated
+    here when not given or too small for a long prompt; without room for the
+    copy the int8 kernel reads the cache). gated: as attention_prefill's."""
     T = q.shape[0] if T is None else T
     q_pitch = q.shape[-1] if q_pitch is None else q_pitch
     row = n_kv_heads * HEAD_DIM

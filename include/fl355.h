@@ -283,8 +283,9 @@ size_t fl_attn_decode_noalloc_max_bytes(void);
  * fl_attention_prefill (no work needed). */
 int fl_attention_prefill_split_count(int T, int pos0, int n_q_heads, int n_kv_heads);
 /* The same choice for an int8 cache (_fh_split's role for
- * attention_prefill_fh_q8, runtime.py:2932-2941): always the 128-row int8
- * kernel's split, what fl_attention_prefill_kv_q8 takes for split 0. */
+ * attention_prefill_fh_q8, runtime.py:2932-2941): the 128-row int8 kernel's
+ * split, what fl_attention_prefill_kv_q8 takes for split 0 where it does not
+ * stage the rows. */
 int fl_attention_prefill_split_count_q8(int T, int pos0, int n_q_heads, int n_kv_heads);
 size_t fl_attention_prefill_work_bytes(int T, int n_q_heads, int head_dim, int split);
 /* The `work` bytes of a call that leaves its split to the library (split 0):
@@ -325,12 +326,11 @@ int fl_attention_prefill_kv_q8(const void* q, int q_pitch, const void* k_new, co
                                int T, int split, void* z, int z_pitch, void* work,
                                size_t work_bytes, fl_stream_t stream);
 /* A prefill chunk's attention output as the layer uses it: the prefill
- * (fl_attention_prefill_kv, or fl_attention_prefill_kv_q8 when q8 != 0; split
- * 0 takes that cache's split count) followed by attn_gate, z = f16_sat(z *
- * sigmoid(gate)), the gate being the second half of each head's q row (q |
- * gate rows of q_pitch >= 2*head_dim halves, the reference's qg buffer).
- * When the KV is split the gate rides in the merge (one launch fewer); the
- * values are the pair's bit for bit. Replaces the sequence _attn_fh then
+ * (fl_attention_prefill_kv, or fl_attention_prefill_kv_q8 when q8 != 0, split and
+ * work as theirs) followed by attn_gate, z = f16_sat(z * sigmoid(gate)), the gate
+ * being the second half of each head's q row (q | gate rows of q_pitch >=
+ * 2*head_dim halves, the reference's qg buffer). Where there is a merge the gate
+ * rides in it (one launch fewer); the values are the pair's bit for bit. Replaces the sequence _attn_fh then
  * attn_gate, runtime.py:2943-2959 then 2860-2862 (kernels.cu:2461-2807,
  * 1585-1600). */
 int fl_attention_prefill_gated(const void* q, int q_pitch, const void* k_new, const void* v_new,
@@ -513,9 +513,8 @@ int fl_gdn_prefill_chunked_logits(const void* q, const void* k, const void* v, c
  * sequence runtime.py:3035-3111 launches, the same values as the separate
  * calls; the conv, the norm and the scan's prep are one launch where a k head
  * has three v heads and there are 96 chunks x k heads or more. x [T][x_stride]
- * f16 the raw q|k|v rows; conv_w [dim][4],
- * st_in / st_out [dim][3] f16 as fl_conv1d_causal's (distinct); a, b
- * [T][ab_stride] f32; S as fl_gdn_prefill_chunked; z, y [T][n_vheads][V] f16,
+ * f16 the raw q|k|v rows; conv_w [dim][4], st_in / st_out [dim][3] f16 as
+ * fl_conv1d_causal's (distinct); a, b [T][ab_stride] f32; S as fl_gdn_prefill_chunked; z, y [T][n_vheads][V] f16,
  * norm_w [V] f32. work: fl_gdn_prefill_layer_work_bytes(...) bytes, 16-byte
  * aligned. K == V == 128, x_stride a multiple of 8. */
 size_t fl_gdn_prefill_layer_work_bytes(int T, int x_stride, int n_vheads, int K, int V);
