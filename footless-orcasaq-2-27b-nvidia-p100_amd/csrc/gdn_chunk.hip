@@ -518,14 +518,16 @@ chunk_prep_kernel(const f16* __restrict__ q, const f16* __restrict__ k, const Pr
 constexpr int FG = 3;                        // v heads a k head
 constexpr int FR_THREADS = 256 * FG;
 constexpr int FR_TB = 4;                     // tokens a conv task
-// The front kernel from this many workgroups up. One takes its ~20 us however
-// few there are (a workgroup's own chain), while the three launches that it
-// replaces spread a short call over more of the chip. Same box, both sides, four
-// layers of 16 k heads, us, front / separate: 1 chunk 108 / 82, 2 (32
-// workgroups) 128 / 114, 5 (80) 166 / 163, 6 (96) 173 / 177, 8 (128) 186 / 201, 16
-// (256) 259 / 306; a layer of 8 k heads at 80 workgroups 50.5 / 49.5, 96 53.5 /
-// 54.5; of 32 at 64 43.5 / 42.3, 96 47.5 / 51.3.
-constexpr int FR_MIN_WGS = 96;
+// The front kernel from this many workgroups up: two chunks at 16 k heads. One
+// takes its ~20 us however few there are (a workgroup's own chain), while the three
+// launches that it replaces spread a short call over more of the chip. Same box,
+// GPU time of four layers of 16 k heads, us, front / separate: 1 chunk 108 / 82, 2
+// (32 workgroups) 128 / 114, 3 142 / 131, 5 (80) 166 / 163, 6 (96) 173 / 177, 8 186 /
+// 201, 16 259 / 306; the line lies at 96 workgroups for 4, 8 and 32 k heads too. But
+// two launches more a layer cost an eager caller ~5 us of host time a layer (a
+// 65-token prompt through three of them and an attention layer, nothing else
+// running: 120 / 132), which only one chunk saves on the GPU.
+constexpr int FR_MIN_WGS = 32;
 constexpr int FR_TILE = CK_C * PK_P * 2;     // staged K or Q rows; A or M o QK^T of a team
 constexpr int FR_LDS = 2 * FR_TILE + FG * 2 * FR_TILE + FG * (2 * CK_C + 8) * 4;
 static_assert(FR_LDS <= 160 * 1024, "the front kernel's LDS fits 160 KiB");

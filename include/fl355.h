@@ -512,7 +512,7 @@ int fl_gdn_prefill_chunked_logits(const void* q, const void* k, const void* v, c
  * and the chunked scan (fl_gdn_prefill_chunked_logits), rmsnorm_gated -- the
  * sequence runtime.py:3035-3111 launches, the same values as the separate
  * calls; the conv, the norm and the scan's prep are one launch where a k head
- * has three v heads and there are 96 chunks x k heads or more. x [T][x_stride]
+ * has three v heads and there are 32 chunks x k heads or more. x [T][x_stride]
  * f16 the raw q|k|v rows; conv_w [dim][4], st_in / st_out [dim][3] f16 as
  * fl_conv1d_causal's (distinct); a, b [T][ab_stride] f32; S as fl_gdn_prefill_chunked; z, y [T][n_vheads][V] f16,
  * norm_w [V] f32. work: fl_gdn_prefill_layer_work_bytes(...) bytes, 16-byte

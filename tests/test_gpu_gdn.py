@@ -808,14 +808,15 @@ def test_gate_logits_of_a_fused_projection(fl, dev, rng, entry, T):
             run(la, lb)
 
 
-# the one-launch front (three v heads a k head, 96 chunks x k heads or more): one
-# chunk of 96 k heads around the conv's 4-token tasks and the frames of history, the
-# model's heads on both sides of the rule and with ragged last chunks; one, two and
-# four v heads a k head (the separate kernels inside the call)
+# the one-launch front (three v heads a k head, 32 chunks x k heads or more): one
+# chunk of 32 k heads around the conv's 4-token tasks and the frames of history, the
+# model's heads on both sides of the rule and with ragged last chunks, 8 k heads
+# below and above it; one, two and four v heads a k head (the separate kernels)
 @pytest.mark.parametrize("nk,nv,T,pos0", [
-    (96, 288, 1, 0), (96, 288, 2, 7), (96, 288, 3, 0), (96, 288, 5, 9), (96, 288, 63, 0),
-    (96, 288, 64, 5), (48, 144, 65, 3), (16, 48, 320, 7), (16, 48, 321, 0), (16, 48, 323, 64),
-    (16, 48, 1000, 5), (4, 4, 70, 3), (4, 8, 70, 0), (4, 16, 200, 9)])
+    (32, 96, 1, 0), (32, 96, 2, 7), (32, 96, 3, 0), (32, 96, 5, 9), (32, 96, 63, 0),
+    (32, 96, 64, 5), (16, 48, 64, 7), (16, 48, 65, 3), (16, 48, 128, 0), (16, 48, 323, 64),
+    (16, 48, 1000, 5), (8, 24, 192, 5), (8, 24, 193, 0), (4, 4, 70, 3), (4, 8, 70, 0),
+    (4, 16, 200, 9)])
 def test_prefill_layer_head_counts_equal_separate_calls(fl, dev, rng, nk, nv, T, pos0):
     """The GDN layer's prefill in one call at other head counts against the
     separate calls: the normed rows, the state and the conv frames bit for bit."""
