@@ -51,6 +51,15 @@ def _ptr(t: torch.Tensor | None, dtype, name: str, span: int = 0):
     return _ptr_any(t, dtype, name, span)
 
 
+def _dense_ptr(t: torch.Tensor, dtype, name: str, span: int = 0):
+    """_ptr of a tensor that has to be contiguous (no further check of a dense one)."""
+    if (isinstance(t, torch.Tensor) and t.dtype is dtype and t.is_cuda and t.numel() >= span
+            and t.is_contiguous()):
+        return t.data_ptr()
+    _contig(t, name)
+    return _ptr_any(t, dtype, name, span)
+
+
 def _ptr_any(t, dtype, name, span):
     if t is None:
         return None

@@ -462,11 +462,9 @@ class HybridRuntime:
                 qg, k, v = proj.full_attn_in(i, B)
                 lcaps = [st.lcap[li] for st in states]
                 spans = [kv8_nbytes(n) if kv8 else n * N_KV * HEAD_DIM for n in lcaps]
-                for st in states:
-                    ops._contig(st.kk[li], "kcache"), ops._contig(st.kv[li], "vcache")
-                kps = _lib.ptr_array([ops._ptr(st.kk[li], kv_type, "kcache", n)
+                kps = _lib.ptr_array([ops._dense_ptr(st.kk[li], kv_type, "kcache", n)
                                       for st, n in zip(states, spans)])
-                vps = _lib.ptr_array([ops._ptr(st.kv[li], kv_type, "vcache", n)
+                vps = _lib.ptr_array([ops._dense_ptr(st.kv[li], kv_type, "vcache", n)
                                       for st, n in zip(states, spans)])
                 out = ops.attn_step(qg, k, v, wt.q_norm, wt.k_norm, kps, vps, pos,
                                     _lib.int_array(lcaps), B=B, kv8=kv8,
