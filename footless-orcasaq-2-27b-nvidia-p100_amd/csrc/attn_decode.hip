@@ -34,8 +34,9 @@
 //     8 lanes and transposed into a per-wave LDS slice. The next tile's loads
 //     are issued before the current tile's math.
 //   * Over the int8 cache the same kernel runs on dequantized tiles: a lane
-//     loads its K / V bytes (half the fp16 bytes) and one dword of scales,
-//     and each value becomes fp16(byte * scale) in registers -- the
+//     loads its K / V bytes (half the fp16 bytes), the scales come through
+//     LDS or a dword a lane, and each value becomes fp16(byte * scale) in
+//     registers -- the
 //     reference's prefill dequantizes V the same way (kernels.cu:2500-2509);
 //     its decode keeps byte * scale in fp32, so scores and outputs differ
 //     from it by fp16 rounding, far below the int8 format's own error. An
